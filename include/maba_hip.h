@@ -122,6 +122,14 @@ int maba_hip_abi_version(void);
 size_t maba_hip_dgda_prefill_workspace_size(const maba_tensor* q, const maba_tensor* v,
                                             const maba_tensor* log_alpha_or_alpha,
                                             const maba_tensor* b);
+/*
+ * The workspace with which the call is cut into as many segments as pay: never less than
+ * maba_hip_dgda_prefill_workspace_size, which is enough for a right result at any size (the
+ * cut, and with it the last bits of the result, follows workspace_bytes).
+ */
+size_t maba_hip_dgda_prefill_workspace_preferred(const maba_tensor* q, const maba_tensor* v,
+                                                 const maba_tensor* log_alpha_or_alpha,
+                                                 const maba_tensor* b);
 int maba_hip_dgda_prefill(const maba_tensor* q, const maba_tensor* k, const maba_tensor* v,
                           const maba_tensor* alpha, const maba_tensor* log_alpha,
                           const maba_tensor* b, const maba_tensor* w,

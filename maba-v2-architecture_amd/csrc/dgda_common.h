@@ -200,9 +200,4 @@ __device__ __forceinline__ float pro_log_decay(float x) {
 // 1 / (||k|| + eps) from the sum of squares
 __device__ __forceinline__ float pro_knorm_inv(float ss, float eps) { return fast_rcp(fast_sqrt(ss) + eps); }
 
-// The conv history a fused layer prefill leaves (the inputs of its last three tokens per
-// stream and channel); defined with the prologue kernels.
-int launch_dgda_new_history(const maba_tensor* const* xs, const maba_tensor* const* hist,
-                            maba_tensor* const* new_hist, hipStream_t stream);
-
 }  // namespace maba

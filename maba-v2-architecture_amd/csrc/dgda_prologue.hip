@@ -224,51 +224,6 @@ static void pro_launch_g(const ProArgs& a, int gdt, dim3 grid, dim3 block, hipSt
   }
 }
 
-// New conv history of a prefill whose conv runs inside the DGDA kernels (the fused layer
-// prefill): the conv inputs of tokens L-3 .. L-1 per stream and channel, from the
-// projections or, for L < 3, the old history.  One thread per channel reads its three
-// inputs before writing, so the new history may overwrite the old one in place.
-template <class XT>
-__global__ __launch_bounds__(256) void dgda_history_kernel(ProArgs a, int C) {
-  const int c = blockIdx.x * 256 + threadIdx.x;
-  const int64_t b = blockIdx.y;
-  if (c >= C) return;
-  float v[3][PRO_KH];
-#pragma unroll
-  for (int s = 0; s < 3; ++s)
-#pragma unroll
-    for (int j = 0; j < PRO_KH; ++j) v[s][j] = pro_input<XT>(a, s, b, c, a.L - PRO_KH + j);
-#pragma unroll
-  for (int s = 0; s < 3; ++s)
-#pragma unroll
-    for (int j = 0; j < PRO_KH; ++j)
-      store_elem(a.nh[s], a.nhdt, b * a.nhsb[s] + c * a.nhsc[s] + j * a.nhst[s], v[s][j]);
-}
-
-// Host side of the above for the fused layer prefill, whose entry point has validated the
-// shapes ([B,L,C] projections with unit channel stride, [B,C,3] histories).
-int launch_dgda_new_history(const maba_tensor* const* xs, const maba_tensor* const* hist,
-                            maba_tensor* const* new_hist, hipStream_t stream) {
-  const int64_t B = xs[0]->shape[0], L = xs[0]->shape[1], C = xs[0]->shape[2];
-  if (B == 0) return MABA_OK;
-  ProArgs a = {};
-  for (int s = 0; s < 3; ++s) {
-    a.x[s] = xs[s]->data; a.xsb[s] = xs[s]->stride[0]; a.xsl[s] = xs[s]->stride[1];
-    a.hist[s] = hist ? hist[s]->data : nullptr;
-    a.hsb[s] = hist ? hist[s]->stride[0] : 0; a.hsc[s] = hist ? hist[s]->stride[1] : 0;
-    a.hst[s] = hist ? hist[s]->stride[2] : 0;
-    a.nh[s] = new_hist[s]->data; a.nhsb[s] = new_hist[s]->stride[0]; a.nhsc[s] = new_hist[s]->stride[1];
-    a.nhst[s] = new_hist[s]->stride[2];
-  }
-  a.hdt = hist ? hist[0]->dtype : MABA_F32;
-  a.nhdt = new_hist[0]->dtype;
-  a.L = L;
-  const dim3 grid((unsigned)ceil_div(C, 256), (unsigned)B);
-  if (xs[0]->dtype == MABA_F32) hipLaunchKernelGGL(dgda_history_kernel<float>, grid, dim3(256), 0, stream, a, (int)C);
-  else hipLaunchKernelGGL(dgda_history_kernel<uint16_t>, grid, dim3(256), 0, stream, a, (int)C);
-  return check_launch("dgda_layer_prefill/history");
-}
-
 }  // namespace maba
 
 using namespace maba;

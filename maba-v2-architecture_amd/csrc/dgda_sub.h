@@ -1,768 +1,1026 @@
 // DGDA prefill for per-channel gates (decay, erase and write gates [B,H,L,d] with
 // unit or zero channel stride): the layer's gate layout, and every head size the
 // reference's GPU prefill takes (d_k, d_v in {32, 64, 128}, triton_dgda.py:389-396):
-// the kernels are instantiated for d_k in {32, 64, 128} and d_v in {32, 64}; d_v = 128
-// runs as two d_v = 64 calls over the two halves of the value columns (the recurrence
-// is separable over value columns: every operation on them is column by column given
-// the key-side quantities).  q, k, v in bf16, fp16 or fp32.
+// the kernels are instantiated for d_k in {32, 64, 128} and 32 or 64 value columns;
+// d_v = 128 runs as two groups of 64 columns in the same launches (the recurrence is
+// separable over value columns).  q, k, v in bf16, fp16 or fp32.
 //
 // Sub-chunks of SC = 16 tokens.  With Lam_i the inclusive cumulative log-decay of
 // token i within the sub-chunk (a d_k-vector over key channels) and S the state at the
 // sub-chunk start (reference math: cpu_dgda.py:101-146, common.py:229-268):
 //   L_ij = sum_c (b*k)_ic k_jc e^{Lam_ic - Lam_jc}      i > j
 //   A_ij = sum_c  q_ic    k_jc e^{Lam_ic - Lam_jc}      i >= j
-//   u    = (I + L)^-1 (w*v - (b*k*e^Lam) S)
+//   (I + L) u = w*v - (b*k*e^Lam) S
 //   o    = (q*e^Lam) S + A u
-//   S'   = diag(e^{Lam_15}) S + (k*e^{Lam_15 - Lam})^T u
-// With decay gates a <= 1 every factor above is e^{<= 0}; gates above 1 (growth) are
-// taken as the token recurrence takes them.  L and A are computed as
-// (b*k*e^Lam)(k*e^{-Lam})^T and (q*e^Lam)(k*e^{-Lam})^T on MFMA when |Lam| <= 64 at every
-// token and channel of the sub-chunk (so e^{+-Lam} stay far inside fp32), and pair by
-// pair with exact exponentials on the VALU otherwise.  Products
-// with fp32 operands split them into bf16 hi + lo (three MFMAs), so they carry ~16
-// mantissa bits; the state stays in fp32 registers.
+//   S'   = diag(e^{Lam_15}) (S + (k*e^-Lam)^T u)
+// L and A are formed as (b*k*e^Lam)(k*e^-Lam)^T and (q*e^Lam)(k*e^-Lam)^T.  All of this
+// holds while |Lam| <= 64 at every token and channel of the sub-chunk (e^{+-Lam} stay
+// far inside fp32); in a sub-chunk with a wider range L and A are summed pair by pair on
+// the VALU with exact exponentials and the update takes k*e^{Lam_15 - Lam}.  Decays above
+// one are taken as the recurrence takes them.
+// Products with fp32 operands split them into bf16 hi + lo (three or four MFMA products),
+// so they carry ~16 mantissa bits; the triangular solve and the state are fp32.
 //
-// MFMA layouts (16x16 tiles, lane (c16, g)): a result lane holds rows 4g..4g+3 of
-// column c16.  The per-token vectors v_e, u and o of a wave's 16 state columns are in
-// that layout (tokens 4g + i, column c16), which is the B-operand layout of the K = 16
-// products T u, A u and (K_C^T) u, so they chain without data movement; the state slab
-// Sr[kt] holds rows 16 kt + 4g + i of column c16 (the layout the segment map uses).
+// One wave runs one segment of one (b, h) sequence on its own: no workgroup barriers, no
+// operand staged twice.  What bounded the four-wave form it replaced was latency: three
+// barriers and a 16-step inverse on one of its waves per sub-chunk, every shared operand
+// read from LDS by all four.  Here the waves of a SIMD hide each other's latencies, and
+// the operand layouts below keep the value side out of LDS altogether.  What bounds a wave now
+// is VALU issue: per sub-chunk at d_k = d_v = 64 about 1,100 VALU instructions (fused layer
+// 1,700, 200 of them transcendental) beside 100 MFMAs, so that one wave per SIMD takes 3.5 us
+// (6.5 us) and two take hardly less time each.  Before and after, whole calls: B=4 H=10
+// T=8192 d=128 fp16 1,377 -> 525 us; B=1 H=10 T=2048 fp32 212 -> 51 us; the fused layer's
+// launches at B=4 T=32768 1,150 -> 680 us, at B=1 T=1000 310 -> 100 us.
 //
-// Sequence parallelism, passes and modes: as the chunked path in dgda_chunk.hip (slots
-// of U sub-chunks, aggregate [N | M] pass, zero-start and fix-up output passes).
+// Layouts.  NKT = d_k / 16, NCT = columns / 16.  Lane (c = lane & 15, g = lane >> 4):
+//  * staging: tokens 4g .. 4g+3, key channels NKT c .. NKT c + NKT-1, value channels
+//    NCT c .. NCT c + NCT-1: every row load is 16 lanes on consecutive bytes;
+//  * state: rows (key channels) (d_k/4) g .. (d_k/4) g + d_k/4 - 1, columns NCT c ..: the
+//    accumulator tile (kt, t) has rows NKT m + kt (m = 0..15) and columns NCT n + t, so
+//    element i of lane (c, g) is row (d_k/4) g + NKT i + kt, column NCT c + t;
+//  * with that choice the staged k*e^-Lam are the A operand of the state update and the
+//    staged w*v and the stored outputs are accumulator fragments, all without moving
+//    between lanes; only the row operands b*k*e^Lam, q*e^Lam and k*e^-Lam (rows = tokens)
+//    pass through LDS, written 8 and read 16 bytes at a time in the natural order;
+//  * the solve wants one column per lane: a 4 x 4 transpose between registers and lane
+//    groups with permlane swaps, then 120 FMAs against rows of L broadcast from LDS.
+//
+// Sequence parallelism.  A sequence is cut into nseg segments of equal length (see
+// sub_nseg).  One launch runs every segment from a zero state (the first from the initial
+// state) and, as further waves, every later segment's transition M (S <- M S + N) from
+// the identity, until M is exactly zero.  scan (three segments or more): start states of
+// segments whose predecessor's M survived.  fix: every later segment from its true start
+// state, over the sub-chunks until its M vanished, or in full.
 //
 // Fused layer prologue (PRO, d_k = d_v = 64; maba_hip_dgda_layer_prefill; reference layers/dgda.py:103-121,
 // 186-207): the kernels read the layer's six bf16 projections instead of q, k, v and the
 // gates, and form the op inputs in the staging step: the causal depthwise conv (kernel 4)
 // + SiLU of q, k, v over [history, projections], the per-head L2 norm of k, the decay
 // max(-softplus, -14) and the sigmoid erase and write gates, all in fp32 and never
-// written back.  A stager lane loads the four conv taps of its token (tokens t-3 .. t,
-// the earlier three mostly L1 hits from its neighbours' loads).  The key norm sums the
-// 64 channels of a token over four waves: each stager wave leaves its partial sums in LDS
-// before the loop-top barrier and the staging after it adds them.
+// written back.  The decays e^max(-softplus(x), -14) = max(sigmoid(-x), e^-14) enter as they
+// are and e^Lam as their running product, which saves a logarithm and an exponential per
+// element.  A lane loads the seven rows its four tokens' taps cover.
 #pragma once
 #include "dgda_common.h"
 
 namespace maba {
 
-constexpr int SC = 16;             // tokens per sub-chunk
-constexpr int SUB_MIN_U = 64;      // sub-chunks per slot at least (1,024 tokens)
-constexpr int SUB_ZERO = 1, SUB_FIX = 2;
-constexpr int TP = 20;             // bf16 row pitch of 16-column tiles
-constexpr float SUB_MFMA_RANGE = 64.f;   // largest |Lam| within a sub-chunk on the MFMA path
+constexpr int SC = 16;                   // tokens per sub-chunk
+constexpr int SUB_MAX_SEG = 2048;         // segments per sequence at most
+constexpr float LOG2E = 1.4426950408889634f;
+constexpr float SUB_MFMA_RANGE = 64.f * LOG2E;   // largest |Lam| within a sub-chunk on the MFMA path, in log2 units
+constexpr float SUB_MFMA_MIN = 1.6038108e-28f;   // e^-64, the same limit for the prologue's decay products
+constexpr float DECAY_MIN = 8.3152872e-7f;       // e^-14
+enum { SUB_MAIN = 0, SUB_FIX = 1 };
 
 struct SubArgs {
   const void* q; int qs0, qs1, qs2;         // [B,H,L,dk], channel stride 1 (16-bit or fp32, see F32IN)
   const void* k; int ks0, ks1, ks2;
   const void* vp; int vs0, vs1, vs2;
-  // gates: fp32, or 16-bit in q's format (see G16); channel stride 0 or 1
+  // gates: fp32, or 16-bit in q's format (see G16); channel stride 0 or 1 (all 1: GCH)
   const void* gp; int gs0, gs1, gs2, gs3;   // log_alpha (use_log) or alpha
   const void* bp; int bs0, bs1, bs2, bs3;   // erase gate b
   const void* wp; int ws0, ws1, ws2, ws3;   // write gate w
   View4 s0;
-  void* op; int os0, os1, os2;              // output [B,H,L,dv], channel stride 1 (bf16 or fp32, see OBF)
+  void* op; int odt; int os0, os1, os2;     // output [B,H,L,dv], channel stride 1
+  int ovec;        // output rows allow one vector store per lane and token
   MView4 sf;
-  float* agg;      // [BH, nseg_max, dk, dv + dk]: [N | M] of segments whose M never vanished, N_k of the others
-  int* zc;         // [BH, nseg_max]: sub-chunks after which the segment's M is exactly zero, -1 if never
-  int64_t U;       // sub-chunks per slot
-  int H, L, BH, nseg_max, nchunks, use_log, has_s0;
-  int mode;        // output kernel: SUB_ZERO or SUB_FIX
+  // [BH, nseg, dk (dv + dk)]: a slot per segment.  First N as the waves hold it, [column group]
+  // [tile t][lane][tile kt][4]; then M, rows of dk bf16 hi and dk lo parts.  The scan turns N
+  // into start states.
+  float* agg;
+  int* zc;         // [BH, nseg, 2]: sub-chunks after which the segment's M (64 columns each) is zero, -1 if never
+  int H, L, BH, nseg, seglen, nchunks, nvh, dvt, use_log, has_s0;
+  int mode;        // SUB_MAIN or SUB_FIX
   // fused prologue (PRO): the six bf16 projections [B, L, C] (q, k, v, decay, erase, write;
   // unit channel stride, head h at channels 64h ..), conv taps [C, 1, 4] (f32/bf16), the
-  // bf16 conv history [B, C, 3] (null: zeros) and the key-norm eps
+  // bf16 conv history [B, C, 3] (null: zeros), the new history and the key-norm eps
   const uint16_t* px[6]; int pxs0[6], pxs1[6];
   const void* cw[3]; int cwdt; int cwsc[3], cwst[3];
   const uint16_t* ph[3]; int phs0[3], phs1[3], phs2[3];
+  void* nh[3]; int nhdt[3]; int64_t nhs0[3], nhs1[3], nhs2[3];
   float eps;
   int f16;         // 16-bit q, k, v are fp16 (else bf16)
-  int of16;        // 16-bit output is fp16 (else bf16)
-};
-typedef const __attribute__((address_space(4))) SubArgs KSubArgs;
-
-#define SM_ALIGN_SUB __attribute__((aligned(16)))
-// fp32 rows of DK (or DV) channels are padded by 4 floats, bf16 rows of DK channels by 8
-// (16-byte aligned rows that shift banks).
-template <bool AGG, bool PRO, int DK, int DV>
-struct SubSmem {
-  static constexpr int FK = DK + 4, FV = DV + 4, PK = DK + 8;
-  SM_ALIGN_SUB float Q[AGG ? 1 : SC][FK];
-  SM_ALIGN_SUB float K[SC][FK];
-  SM_ALIGN_SUB float BK[SC][FK];            // b * k
-  SM_ALIGN_SUB float WV[SC][FV];            // w * v
-  SM_ALIGN_SUB float LA[SC][FK];            // log decay, then the inclusive prefix Lam
-  SM_ALIGN_SUB short QEh[AGG ? 8 : SC * PK], QEl[AGG ? 8 : SC * PK];   // q e^Lam
-  SM_ALIGN_SUB short BKEh[SC * PK], BKEl[SC * PK];                     // b k e^Lam
-  SM_ALIGN_SUB short KIh[SC * PK], KIl[SC * PK];                       // k e^-Lam
-  SM_ALIGN_SUB short KCh[DK * TP], KCl[DK * TP];                       // (k e^{Lam_15 - Lam})^T
-  SM_ALIGN_SUB short Th[SC * TP], Tl[SC * TP];                               // (I + L)^-1
-  SM_ALIGN_SUB short Ah[AGG ? 8 : SC * TP], Al[AGG ? 8 : SC * TP];           // A (lower, with diagonal)
-  SM_ALIGN_SUB float Lq[SC][4][4];                                            // L[i][p + 4 r] at [i][p][r]
-  SM_ALIGN_SUB float elast[DK];                                               // e^{Lam_15}
-  SM_ALIGN_SUB float nrm[PRO ? 2 : 1][4][16];   // fused prologue: |k|^2 partials [sub-chunk parity][stager wave][token]
-  SM_ALIGN_SUB float cw[PRO ? 3 : 1][4][64];    // fused prologue: the head's conv taps [stream][tap][channel]
-  int big[2];                               // some |Lam| exceeds SUB_MFMA_RANGE (by sub-chunk parity)
 };
 
-// Raw registers of four consecutive row elements (bf16 bits or fp32).  Prefetched rows
-// stay raw until they are staged, so that no conversion waits for the loads.
-template <bool F32IN>
-using Raw4 = std::conditional_t<F32IN, f32x4, i16x4>;
+template <int N> using fvec = float __attribute__((ext_vector_type(N)));
 
-template <bool F32IN>
-__device__ __forceinline__ Raw4<F32IN> load_raw4(const void* base, int64_t off) {
-  if constexpr (F32IN) return *(const f32x4*)((const float*)base + off);
-  else return *(const i16x4*)((const uint16_t*)base + off);
+// N consecutive row elements as loaded (16-bit pairs or fp32 words).  Prefetched rows stay
+// raw until they are staged, so that no conversion waits for the loads.
+template <bool F32, int N>
+struct Row { uint32_t w[F32 ? N : N / 2]; };
+
+// Rows start at a multiple of four elements (checked on the host).
+template <bool F32, int N>
+__device__ __forceinline__ Row<F32, N> load_row(const char* p) {
+  constexpr int NW = F32 ? N : N / 2;
+  Row<F32, N> r;
+  if constexpr (NW == 1) {
+    r.w[0] = *(const uint32_t*)p;
+  } else if constexpr (NW == 2) {
+    typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+    const u2 v = *(const u2*)p;
+    r.w[0] = v[0]; r.w[1] = v[1];
+  } else {
+    typedef uint32_t u4 __attribute__((ext_vector_type(4), aligned(8)));
+#pragma unroll
+    for (int i = 0; i < NW / 4; ++i) {
+      const u4 v = ((const u4*)p)[i];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) r.w[4 * i + j] = v[j];
+    }
+  }
+  return r;
 }
-template <bool F32IN>
-__device__ __forceinline__ f32x4 raw_f32(Raw4<F32IN> r, bool f16) {
-  if constexpr (F32IN) {
+template <bool F32, int N>
+__device__ __forceinline__ float row_at(const Row<F32, N>& r, int j, bool f16) {
+  if constexpr (F32) return __uint_as_float(r.w[j]);
+  else {
+    const uint32_t h = (j & 1) ? r.w[j / 2] >> 16 : r.w[j / 2] & 0xffffu;
+    if (f16) return __half2float(__ushort_as_half((unsigned short)h));
+    return __uint_as_float((j & 1) ? r.w[j / 2] & 0xffff0000u : r.w[j / 2] << 16);
+  }
+}
+// N gate values of one token at channel stride cs (0 or 1), p at the first, as raw elements.
+template <bool G16, bool GCH, int N>
+__device__ __forceinline__ Row<!G16, N> load_gate(const char* p, int cs) {
+  if constexpr (GCH) {
+    return load_row<!G16, N>(p);
+  } else {
+    Row<!G16, N> r;
+    if constexpr (G16) {
+#pragma unroll
+      for (int j = 0; j < N / 2; ++j)
+        r.w[j] = (uint32_t)((const uint16_t*)p)[2 * j * cs] | ((uint32_t)((const uint16_t*)p)[(2 * j + 1) * cs] << 16);
+    } else {
+#pragma unroll
+      for (int j = 0; j < N; ++j) r.w[j] = ((const uint32_t*)p)[j * cs];
+    }
     return r;
-  } else {
-    if (f16) {
-      auto h = [](short x) { return __half2float(__ushort_as_half((unsigned short)x)); };
-      return f32x4{h(r[0]), h(r[1]), h(r[2]), h(r[3])};
-    }
-    return f32x4{bf16_val(r[0]), bf16_val(r[1]), bf16_val(r[2]), bf16_val(r[3])};
   }
 }
 
-// S <- M S + N for a segment map X = [N | M] (DK x (DV + DK) fp32, row-major: N in columns
-// [0, DV), M in [DV, DV + DK)) on the slab Sr[kt][i] = S[16kt + 4g + i][col0 + c16] of one
-// wave, with fp32 accuracy (M and S both split into bf16 hi/lo, three products).
-template <int DK, int DV>
-__device__ __forceinline__ void apply_map(const float* X, f32x4 (&Sr)[DK / 16], int col0, int c16, int g) {
-  constexpr int NKT = DK / 16, AW = DV + DK;
-  i16x4 Sh[NKT], Sl[NKT];
-#pragma unroll
-  for (int kt = 0; kt < NKT; ++kt) split4(Sr[kt], Sh[kt], Sl[kt]);
-#pragma unroll
-  for (int mt = 0; mt < NKT; ++mt) {
-    f32x4 acc;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) acc[i] = X[(16 * mt + 4 * g + i) * AW + col0 + c16];  // N
-    const int row = 16 * mt + c16;
-#pragma unroll
-    for (int p = 0; p < DK / 32; ++p) {
-      // A operand: M[row][32p + 4g..+3] and [32p + 16 + 4g..+3]
-      const f32x4 m0 = *(const f32x4*)(X + row * AW + DV + 32 * p + 4 * g);
-      const f32x4 m1 = *(const f32x4*)(X + row * AW + DV + 32 * p + 16 + 4 * g);
-      i16x4 h0, l0, h1, l1;
-      split4(m0, h0, l0);
-      split4(m1, h1, l1);
-      const i16x8 ah = cat8(h0, h1), al = cat8(l0, l1);
-      const i16x8 bh8 = cat8(Sh[2 * p], Sh[2 * p + 1]), bl8 = cat8(Sl[2 * p], Sl[2 * p + 1]);
-      acc = mma32(acc, ah, bh8);
-      acc = mma32(acc, ah, bl8);
-      acc = mma32(acc, al, bh8);
-    }
-    Sr[mt] = acc;
-  }
-}
-// Four gate values of one token, channels c0 .. c0+3 at channel stride cs (0 or 1):
-// four element loads, the same code for both strides (no branch, so the prefetched
-// registers are not merged across paths, which would wait for the loads).  Raw fp32, or
-// raw 16-bit (G16).
-template <bool G16>
-__device__ __forceinline__ Raw4<!G16> load_gate4(const void* base, int64_t off, int cs, int c0) {
-  if constexpr (G16) {
-    const uint16_t* row = (const uint16_t*)base + off;
-    return i16x4{(short)row[c0 * cs], (short)row[(c0 + 1) * cs], (short)row[(c0 + 2) * cs], (short)row[(c0 + 3) * cs]};
-  } else {
-    const float* row = (const float*)base + off;
-    return f32x4{row[c0 * cs], row[(c0 + 1) * cs], row[(c0 + 2) * cs], row[(c0 + 3) * cs]};
-  }
-}
+// ------------------------------------------------------------------ lane-group moves
 
-// Inclusive prefix sum over each 16-lane DPP row (row_shr 1, 2, 4, 8; lanes shifted in
-// from outside the row read zero).
-__device__ __forceinline__ float row16_incl_scan(float x) {
-  auto dpp = [](float v, auto ctrl_c) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(ctrl_c)::value, 0xf, 0xf, true));
+// Exchanges a's upper 32 lanes with b's lower 32 (swap32), a's odd 16-lane rows with b's
+// even ones (swap16).
+__device__ __forceinline__ void swap32(uint32_t& a, uint32_t& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  a = r[0]; b = r[1];
+}
+__device__ __forceinline__ void swap16(uint32_t& a, uint32_t& b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+  a = r[0]; b = r[1];
+}
+// x[t] of lane group g  <->  x[g] of lane group t (4 x 4 transpose; its own inverse).
+__device__ __forceinline__ void transpose4(uint32_t (&x)[4]) {
+  swap32(x[0], x[2]);
+  swap32(x[1], x[3]);
+  swap16(x[0], x[1]);
+  swap16(x[2], x[3]);
+}
+// Exclusive prefix over the lane groups (g = 0: the neutral element) and the total, of sums or
+// (MUL) products.
+template <bool MUL>
+__device__ __forceinline__ void group_prefix(float x, int g, float& excl, float& tot) {
+  auto op = [](float p, float q) { return MUL ? p * q : p + q; };
+  const float one = MUL ? 1.f : 0.f;
+  uint32_t a = __float_as_uint(x), b = a;
+  swap16(a, b);                                    // a: x0 x0 x2 x2, b: x1 x1 x3 x3
+  uint32_t lo = __float_as_uint(op(__uint_as_float(a), __uint_as_float(b))), hi = lo;
+  swap32(lo, hi);                                  // lo: x0, x1 and hi: x2, x3 together, in every lane
+  excl = op((g & 1) ? __uint_as_float(a) : one, (g & 2) ? __uint_as_float(lo) : one);
+  tot = op(__uint_as_float(lo), __uint_as_float(hi));
+}
+// Sum over the 16 lanes of a row, in every lane (row_ror 8, 4, 2, 1).
+__device__ __forceinline__ float row16_sum(float x) {
+  auto ror = [](float v, auto ctrl_c) {
+    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(ctrl_c)::value, 0xf, 0xf, true));
   };
   using std::integral_constant;
-  x += dpp(x, integral_constant<int, 0x111>{});
-  x += dpp(x, integral_constant<int, 0x112>{});
-  x += dpp(x, integral_constant<int, 0x114>{});
-  x += dpp(x, integral_constant<int, 0x118>{});
-  return x;
+  x = ror(x, integral_constant<int, 0x128>{});
+  x = ror(x, integral_constant<int, 0x124>{});
+  x = ror(x, integral_constant<int, 0x122>{});
+  return ror(x, integral_constant<int, 0x121>{});
+}
+// LDS traffic of the wave so far is ordered before what follows (a wave's LDS operations
+// execute in order; this keeps the compiler from moving them across).
+__device__ __forceinline__ void wave_fence() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
 }
 
-// One segment: sub-chunks [c_begin, c_end) of sequence bh, segment k of n.
-template <bool AGG, bool F32IN, bool G16, bool OBF, bool PRO, int DK, int DV>
-__device__ __forceinline__ void sub_segment(KSubArgs& a, SubSmem<AGG, PRO, DK, DV>& sm, int* s_mzero, int tid,
-                                            int bh, int k, int n, int c_begin, int c_end) {
+// bf16 hi and lo parts of a pair, packed (x ~= hi + lo).
+__device__ __forceinline__ void split2(float x0, float x1, uint32_t& h, uint32_t& l) {
+  h = cvt_pk_bf16(x0, x1);
+  l = cvt_pk_bf16(bf16_rem<0>(h, x0), bf16_rem<1>(h, x1));
+}
+__device__ __forceinline__ i16x8 pack8(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+  typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+  const u4 v = {a, b, c, d};
+  return __builtin_bit_cast(i16x8, v);
+}
+
+// ------------------------------------------------------------------ the wave's LDS
+
+template <bool PRO, int DK>
+struct SubSmem {
+  static constexpr int PK = DK + 8;   // row pitch of the bf16 row operands (16-byte aligned rows that shift banks)
+  union {
+    struct {   // rows = tokens
+      __attribute__((aligned(16))) short BKh[SC * PK], BKl[SC * PK];   // -(b k e^Lam)
+      __attribute__((aligned(16))) short QEh[SC * PK], QEl[SC * PK];   // q e^Lam
+      __attribute__((aligned(16))) short KIh[SC * PK], KIl[SC * PK];   // k e^-Lam
+      __attribute__((aligned(16))) float Lm[SC][SC];         // -L, rows i, zero for j >= i
+      __attribute__((aligned(16))) float elast[DK];          // e^{Lam_15}
+    } r;
+    struct {   // pair-by-pair sums, fp32
+      __attribute__((aligned(16))) float k[SC][DK], bk[SC][DK], q[SC][DK], lam[SC][DK];
+    } f;
+  };
+  __attribute__((aligned(16))) float cw[PRO ? 3 : 1][4][PRO ? 64 : 1];   // the head's conv taps [stream][tap][channel]
+};
+
+// ------------------------------------------------------------------ one segment
+
+// Sub-chunks [c_begin, c_end) of sequence bh.  ROLE OUT: from the state in Sr, outputs
+// stored, state left in Sr.  ROLE MAP: the transition, v = 0 and no outputs; returns the
+// sub-chunks after which Sr is exactly zero (-1: never).  col: the lane's first value
+// column (of dvt); key-side work is the same for every column group.
+template <bool MAP, bool F32IN, bool G16, bool GCH, bool PRO, int DK, int DV>
+__device__ __forceinline__ int sub_run(const SubArgs& a, SubSmem<PRO, DK>& sm, int lane, int bh, int col,
+                                       int c_begin, int c_end, f32x4 (&Sr)[DK / 16][MAP ? (DK < 64 ? DK : 64) / 16 : DV / 16]) {
+  constexpr int NKT = DK / 16, NCT = MAP ? (DK < 64 ? DK : 64) / 16 : DV / 16, NVT = DV / 16;
+  constexpr int NP = DK / 32;              // K = 32 steps over the key channels
+  constexpr int PK = SubSmem<PRO, DK>::PK;
+  constexpr int NL = DK / 4;               // state rows of a lane: channel NL g + l, l = NKT i + kt
+  constexpr int ES = F32IN ? 4 : 2, EG = G16 ? 2 : 4;
+  const int g = lane >> 4, c = lane & 15;
+  const int bi = bh / a.H, hi = bh % a.H;
+  const int kch = NKT * c;                 // the lane's first key channel
+
+  // ---- row sources: a uniform base per sub-chunk plus a 32-bit lane offset
+  auto base = [&](const void* p, int s0, int s1, int s2, int es, int t0) {
+    return (const char*)p + ((int64_t)bi * s0 + (int64_t)hi * s1 + (int64_t)t0 * s2) * es;
+  };
+  Row<F32IN, NKT> pq[4], pk[4];
+  Row<F32IN, NVT> pv[4];
+  Row<!G16, NKT> pg[4], pb[4];
+  Row<!G16, NVT> pw[4];
+  Row<false, 4> tq[7], tk[7], tv[7], xg[3][4];   // fused prologue: rows 4g-3 .. 4g+3, and the gate rows
+  // rows past the end re-read the last one, rows before the first (replaced by the history) the first
+  auto prefetch = [&](int cc) {
+    const int t0 = cc * SC;
+    if constexpr (PRO) {
+      const int d = min(t0, 3), last = a.L - 1 - (t0 - d);   // rows are counted from token t0 - d
+      auto rows = [&](int s, auto& x, int m0, auto n_c) {
+        const char* p = base(a.px[s], a.pxs0[s], 0, a.pxs1[s], 2, t0 - d);
+        const int S = 2 * a.pxs1[s], chb = 2 * (hi * 64 + kch);
+        const int lane0 = 4 * g * S + chb, end = last * S + chb;
+#pragma unroll
+        for (int m = 0; m < decltype(n_c)::value; ++m)
+          x[m] = load_row<false, 4>(p + (uint32_t)max(min(lane0 + (m + m0 + d) * S, end), chb));
+      };
+      using std::integral_constant;
+      if (!MAP) rows(0, tq, -3, integral_constant<int, 7>{});
+      rows(1, tk, -3, integral_constant<int, 7>{});
+      if (!MAP) rows(2, tv, -3, integral_constant<int, 7>{});
+      rows(3, xg[0], 0, integral_constant<int, 4>{});
+      rows(4, xg[1], 0, integral_constant<int, 4>{});
+      if (!MAP) rows(5, xg[2], 0, integral_constant<int, 4>{});
+    } else {
+      const int last = a.L - 1 - t0;
+      const char* bk = base(a.k, a.ks0, a.ks1, a.ks2, ES, t0);
+      const char* bv = base(a.vp, a.vs0, a.vs1, a.vs2, ES, t0);
+      const char* bg = base(a.gp, a.gs0, a.gs1, a.gs2, EG, t0);
+      const char* bb = base(a.bp, a.bs0, a.bs1, a.bs2, EG, t0);
+      const char* bw = base(a.wp, a.ws0, a.ws1, a.ws2, EG, t0);
+      auto rows = [&](const char* p, int S, int chb, auto& x, auto load) {
+        const int lane0 = 4 * g * S + chb, end = last * S + chb;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] = load(p + (uint32_t)min(lane0 + i * S, end));
+      };
+      auto lk = [](const char* p) { return load_row<F32IN, NKT>(p); };
+      auto lv = [](const char* p) { return load_row<F32IN, NVT>(p); };
+      // a gate's rows at channel stride 1, or its element at stride 0 (then chb is zero)
+      const int ck = kch * EG, cv = col * EG;
+      rows(bk, a.ks2 * ES, kch * ES, pk, lk);
+      rows(bg, a.gs2 * EG, GCH ? ck : ck * a.gs3, pg, [&](const char* p) { return load_gate<G16, GCH, NKT>(p, a.gs3); });
+      rows(bb, a.bs2 * EG, GCH ? ck : ck * a.bs3, pb, [&](const char* p) { return load_gate<G16, GCH, NKT>(p, a.bs3); });
+      if (!MAP) {
+        rows(base(a.q, a.qs0, a.qs1, a.qs2, ES, t0), a.qs2 * ES, kch * ES, pq, lk);
+        rows(bv, a.vs2 * ES, col * ES, pv, lv);
+        rows(bw, a.ws2 * EG, GCH ? cv : cv * a.ws3, pw, [&](const char* p) { return load_gate<G16, GCH, NVT>(p, a.ws3); });
+      }
+    }
+  };
+  // fused prologue: taps before token 0 come from the history, or are zero
+  auto hist_rows = [&](int s, Row<false, 4> (&t)[7]) {
+    if (g != 0) return;
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+      uint32_t h[4] = {0, 0, 0, 0};
+      if (a.ph[s]) {
+        const uint16_t* hp = a.ph[s] + (int64_t)bi * a.phs0[s] + (int64_t)(hi * 64 + kch) * a.phs1[s] + (int64_t)m * a.phs2[s];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) h[e] = hp[(int64_t)e * a.phs1[s]];
+      }
+      t[m].w[0] = h[0] | (h[1] << 16);
+      t[m].w[1] = h[2] | (h[3] << 16);
+    }
+  };
+  // fused prologue: SiLU(depthwise conv) of the lane's four tokens and channels
+  auto conv = [&](int s, const Row<false, 4> (&t)[7], float (&y)[4][4]) {
+    f32x4 w[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w[j] = *(const f32x4*)&sm.cw[s][j][PRO ? kch : 0];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float x[7];
+#pragma unroll
+      for (int m = 0; m < 7; ++m) x[m] = row_at<false, 4>(t[m], e, false);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float acc = w[3][e] * x[i + 3];
+        acc = fmaf(w[2][e], x[i + 2], acc);
+        acc = fmaf(w[1][e], x[i + 1], acc);
+        acc = fmaf(w[0][e], x[i], acc);
+        y[i][e] = pro_silu(acc);
+      }
+    }
+  };
+
+  // ---- outputs of a sub-chunk are stored during the next one's staging, before its
+  // prefetch: the wait for the prefetched rows then does not cover the stores
+  f32x4 ob[NVT];
+  int ot0 = -1;
+  auto flush = [&]() {
+    if (MAP || ot0 < 0) return;
+    const int nt = a.L - ot0;
+    const int64_t ub = (int64_t)bi * a.os0 + (int64_t)hi * a.os1 + (int64_t)ot0 * a.os2;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int t = 4 * g + i;
+      if (t >= nt) continue;
+      const int64_t off = ub + (int64_t)t * a.os2 + col;
+      if (a.ovec && a.odt == MABA_BF16) {
+        uint32_t* p = (uint32_t*)((uint16_t*)a.op + off);
+        if constexpr (NVT == 4) *(uint2*)p = make_uint2(cvt_pk_bf16(ob[0][i], ob[1][i]), cvt_pk_bf16(ob[2][i], ob[3][i]));
+        else p[0] = cvt_pk_bf16(ob[0][i], ob[1][i]);
+      } else if (a.ovec && a.odt == MABA_F16) {
+        auto pk = [](float x, float y) {
+          return (uint32_t)__half_as_ushort(__float2half(x)) | ((uint32_t)__half_as_ushort(__float2half(y)) << 16);
+        };
+        uint32_t* p = (uint32_t*)((uint16_t*)a.op + off);
+        if constexpr (NVT == 4) *(uint2*)p = make_uint2(pk(ob[0][i], ob[1][i]), pk(ob[2][i], ob[3][i]));
+        else p[0] = pk(ob[0][i], ob[1][i]);
+      } else if (a.ovec) {
+        float* p = (float*)a.op + off;
+        if constexpr (NVT == 4) *(f32x4*)p = f32x4{ob[0][i], ob[1][i], ob[2][i], ob[3][i]};
+        else *(float2*)p = make_float2(ob[0][i], ob[1][i]);
+      } else {
+#pragma unroll
+        for (int t2 = 0; t2 < NVT; ++t2) store_elem(a.op, a.odt, off + t2, ob[t2][i]);   // unaligned rows
+      }
+    }
+  };
+
+  if (c_begin < c_end) prefetch(c_begin);
+  for (int cc = c_begin; cc < c_end; ++cc) {
+    const int t0 = cc * SC, nt = a.L - t0;
+    // ---- staging: the op inputs of tokens 4g + i
+    float kk[4][NKT], la[4][NKT], be[4][NKT], qq[4][NKT];
+    f32x4 ve[NCT];                         // w*v, then the solve's right-hand side
+    if constexpr (PRO) {
+      if (cc == 0) {
+        if (!MAP) hist_rows(0, tq);
+        hist_rows(1, tk);
+        if (!MAP) hist_rows(2, tv);
+      }
+      conv(1, tk, kk);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float ss = row16_sum(kk[i][0] * kk[i][0] + kk[i][1] * kk[i][1] + kk[i][2] * kk[i][2] + kk[i][3] * kk[i][3]);
+        const float inv = pro_knorm_inv(ss, a.eps);
+#pragma unroll
+        for (int j = 0; j < NKT; ++j) {
+          kk[i][j] *= inv;
+          // the decay e^max(-softplus(x), -14) = max(1 / (1 + e^x), e^-14)
+          la[i][j] = fmaxf(fast_rcp(1.f + fast_exp(row_at<false, 4>(xg[0][i], j, false))), DECAY_MIN);
+          be[i][j] = pro_sigmoid(row_at<false, 4>(xg[1][i], j, false));
+        }
+      }
+      if (!MAP) {
+        float vv[4][4];
+        conv(2, tv, vv);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int j = 0; j < NVT; ++j) ve[j][i] = pro_sigmoid(row_at<false, 4>(xg[2][i], j, false)) * vv[i][j];
+        conv(0, tq, qq);
+      }
+    } else {
+      const bool f16 = a.f16 != 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+#pragma unroll
+        for (int j = 0; j < NKT; ++j) {
+          kk[i][j] = row_at(pk[i], j, f16);
+          be[i][j] = row_at(pb[i], j, f16);
+          const float x = row_at(pg[i], j, f16);
+          la[i][j] = a.use_log ? x * LOG2E : __builtin_amdgcn_logf(fmaxf(x, 1e-20f));
+          if (!MAP) qq[i][j] = row_at(pq[i], j, f16);
+        }
+        if (!MAP) {
+#pragma unroll
+          for (int j = 0; j < NVT; ++j) ve[j][i] = row_at(pw[i], j, f16) * row_at(pv[i], j, f16);
+        }
+      }
+    }
+    if (MAP) {
+#pragma unroll
+      for (int t = 0; t < NCT; ++t) ve[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    if (nt < SC) {   // tokens past the end: no decay, no key, no write
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const bool on = 4 * g + i < nt;
+#pragma unroll
+        for (int j = 0; j < NKT; ++j) {
+          kk[i][j] = on ? kk[i][j] : 0.f;
+          la[i][j] = on ? la[i][j] : PRO ? 1.f : 0.f;
+          be[i][j] = on ? be[i][j] : 0.f;
+          if (!MAP) qq[i][j] = on ? qq[i][j] : 0.f;
+        }
+#pragma unroll
+        for (int t = 0; t < NCT; ++t) ve[t][i] = on ? ve[t][i] : 0.f;
+      }
+    }
+    flush();
+    // ---- Lam (PRO: e^Lam): prefix over the lane's tokens, then over the lane groups
+    float lam[4][NKT], tot[NKT];
+    auto prefix = [&](auto mul_c) {
+      constexpr bool MUL = decltype(mul_c)::value;
+#pragma unroll
+      for (int j = 0; j < NKT; ++j) {
+        lam[0][j] = la[0][j];
+#pragma unroll
+        for (int i = 1; i < 4; ++i) lam[i][j] = MUL ? lam[i - 1][j] * la[i][j] : lam[i - 1][j] + la[i][j];
+        float ex;
+        group_prefix<MUL>(lam[3][j], g, ex, tot[j]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) lam[i][j] = MUL ? lam[i][j] * ex : lam[i][j] + ex;
+      }
+    };
+    prefix(std::integral_constant<bool, PRO>{});
+    float mx = PRO ? 1.f : 0.f;
+    bool over = false;
+#pragma unroll
+    for (int j = 0; j < NKT; ++j) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) mx = PRO ? fminf(mx, lam[i][j]) : fmaxf(mx, fabsf(lam[i][j]));
+      if (!PRO) over |= !(tot[j] == tot[j]);   // fmaxf drops NaN, which every prefix that meets one carries to the total
+    }
+    over |= PRO ? !(mx >= SUB_MFMA_MIN) : !(mx <= SUB_MFMA_RANGE);
+    const bool wide = __ballot(over) != 0ull;   // the same in every lane
+    wave_fence();   // the previous sub-chunk's LDS reads come first
+    // the row factors e^Lam and the keys scaled for the column side (wide: for the update only)
+    float e[4][NKT], kx[4][NKT];
+    f32x4 lt = {0.f, 0.f, 0.f, 0.f}, at = lt;    // -L and A: lane (c, g), element r: row i = c, column j = 4g + r
+    if (!wide) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < NKT; ++j) {
+          e[i][j] = PRO ? lam[i][j] : __builtin_amdgcn_exp2f(lam[i][j]);
+          kx[i][j] = kk[i][j] * (PRO ? fast_rcp(lam[i][j]) : __builtin_amdgcn_exp2f(-lam[i][j]));
+          if (!PRO && i == 0) tot[j] = __builtin_amdgcn_exp2f(tot[j]);
+        }
+    } else {
+      if constexpr (PRO) {   // in logarithms here: the products may have left fp32's range
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int j = 0; j < NKT; ++j) la[i][j] = __builtin_amdgcn_logf(la[i][j]);
+        prefix(std::false_type{});
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < NKT; ++j) {
+          sm.f.k[4 * g + i][kch + j] = kk[i][j];
+          sm.f.bk[4 * g + i][kch + j] = be[i][j] * kk[i][j];
+          if (!MAP) sm.f.q[4 * g + i][kch + j] = qq[i][j];
+          sm.f.lam[4 * g + i][kch + j] = lam[i][j];
+          e[i][j] = __builtin_amdgcn_exp2f(lam[i][j]);
+          kx[i][j] = kk[i][j] * __builtin_amdgcn_exp2f(tot[j] - lam[i][j]);
+        }
+#pragma unroll
+      for (int j = 0; j < NKT; ++j) tot[j] = __builtin_amdgcn_exp2f(tot[j]);
+      wave_fence();
+#pragma unroll 1
+      for (int ch = 0; ch < DK; ch += 4) {
+        const f32x4 li = *(const f32x4*)&sm.f.lam[c][ch], bi4 = *(const f32x4*)&sm.f.bk[c][ch];
+        const f32x4 qi = MAP ? li : *(const f32x4*)&sm.f.q[c][ch];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const f32x4 lj = *(const f32x4*)&sm.f.lam[4 * g + r][ch], kj = *(const f32x4*)&sm.f.k[4 * g + r][ch];
+#pragma unroll
+          for (int x = 0; x < 4; ++x) {
+            const float d = __builtin_amdgcn_exp2f(4 * g + r <= c ? li[x] - lj[x] : 0.f) * kj[x];   // later tokens' pairs are dropped below
+            lt[r] = fmaf(-bi4[x], d, lt[r]);
+            if (!MAP) at[r] = fmaf(qi[x], d, at[r]);
+          }
+        }
+      }
+      wave_fence();
+    }
+    {
+      // ---- row operands to LDS; the update's A operand kf stays in registers
+      i16x8 kf[NKT];
+      {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int tk_ = 4 * g + i;
+          uint32_t bh_[NKT / 2], bl_[NKT / 2], qh_[NKT / 2], ql_[NKT / 2], kh_[NKT / 2], kl_[NKT / 2];
+#pragma unroll
+          for (int j = 0; j < NKT; j += 2) {
+            split2(-(be[i][j] * kk[i][j]) * e[i][j], -(be[i][j + 1] * kk[i][j + 1]) * e[i][j + 1], bh_[j / 2], bl_[j / 2]);
+            split2(kx[i][j], kx[i][j + 1], kh_[j / 2], kl_[j / 2]);
+            if (!MAP) split2(qq[i][j] * e[i][j], qq[i][j + 1] * e[i][j + 1], qh_[j / 2], ql_[j / 2]);
+          }
+          auto put = [&](short* dst, const uint32_t (&v)[NKT / 2]) {
+            uint32_t* p = (uint32_t*)(dst + tk_ * PK + kch);
+            if constexpr (NKT == 2) p[0] = v[0];
+            else if constexpr (NKT == 4) *(uint2*)p = make_uint2(v[0], v[1]);
+            else *(uint4*)p = make_uint4(v[0], v[1], v[2], v[3]);
+          };
+          put(sm.r.BKh, bh_);
+          put(sm.r.BKl, bl_);
+          put(sm.r.KIh, kh_);
+          put(sm.r.KIl, kl_);
+          if (!MAP) {
+            put(sm.r.QEh, qh_);
+            put(sm.r.QEl, ql_);
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < NKT; ++j) {
+          uint32_t h0, h1, l0, l1;
+          split2(kx[0][j], kx[1][j], h0, l0);
+          split2(kx[2][j], kx[3][j], h1, l1);
+          kf[j] = pack8(h0, h1, l0, l1);   // [hi | lo] of tokens 4g .. 4g+3, channel kch + j
+        }
+        if (g == 3) {
+#pragma unroll
+          for (int j = 0; j < NKT; ++j) sm.r.elast[kch + j] = tot[j];
+        }
+      }
+      wave_fence();
+      // ---- -L and A as products, and the row operands for those with S
+      i16x8 bh8[NP], bl8[NP], qh8[NP], ql8[NP];
+      i16x8 af = {};
+      {
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+          const int off = c * PK + NL * g + 8 * p;
+          bh8[p] = *(const i16x8*)(sm.r.BKh + off);
+          bl8[p] = *(const i16x8*)(sm.r.BKl + off);
+          if (!MAP) {
+            qh8[p] = *(const i16x8*)(sm.r.QEh + off);
+            ql8[p] = *(const i16x8*)(sm.r.QEl + off);
+          }
+        }
+        if (!wide) {
+#pragma unroll
+          for (int p = 0; p < NP; ++p) {
+            const int off = c * PK + NL * g + 8 * p;
+            const i16x8 kh8 = *(const i16x8*)(sm.r.KIh + off), kl8 = *(const i16x8*)(sm.r.KIl + off);
+            lt = mma32(lt, kh8, bh8[p]);
+            lt = mma32(lt, kh8, bl8[p]);
+            lt = mma32(lt, kl8, bh8[p]);
+            if (!MAP) {
+              at = mma32(at, kh8, qh8[p]);
+              at = mma32(at, kh8, ql8[p]);
+              at = mma32(at, kl8, qh8[p]);
+            }
+          }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) lt[r] = 4 * g + r < c ? lt[r] : 0.f;
+        *(f32x4*)&sm.r.Lm[c][4 * g] = lt;
+        if (!MAP) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) at[r] = 4 * g + r <= c ? at[r] : 0.f;
+          uint32_t h0, h1, l0, l1;
+          split2(at[0], at[1], h0, l0);
+          split2(at[2], at[3], h1, l1);
+          af = pack8(h0, h1, l0, l1);
+        }
+      }
+      // ---- v_e = w*v - (b k e^Lam) S and q S, both tokens 4g + i of the lane's columns
+      f32x4 qs[NVT];
+#pragma unroll
+      for (int t = 0; t < NCT; ++t) {
+        if (!MAP) qs[t < NVT ? t : 0] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+          uint32_t h[4], l[4];
+#pragma unroll
+          for (int e = 0; e < 8; e += 2) {
+            const int l0 = 8 * p + e, l1 = l0 + 1;
+            split2(Sr[l0 % NKT][t][l0 / NKT], Sr[l1 % NKT][t][l1 / NKT], h[e / 2], l[e / 2]);
+          }
+          const i16x8 sh = pack8(h[0], h[1], h[2], h[3]), sl = pack8(l[0], l[1], l[2], l[3]);
+          ve[t] = mma32(ve[t], bh8[p], sh);
+          ve[t] = mma32(ve[t], bh8[p], sl);
+          ve[t] = mma32(ve[t], bl8[p], sh);
+          if (!MAP) {
+            f32x4& q_ = qs[t < NVT ? t : 0];
+            q_ = mma32(q_, qh8[p], sh);
+            q_ = mma32(q_, qh8[p], sl);
+            q_ = mma32(q_, ql8[p], sh);
+          }
+        }
+      }
+      f32x4 el[NL / 4];
+#pragma unroll
+      for (int l = 0; l < NL / 4; ++l) el[l] = *(const f32x4*)&sm.r.elast[NL * g + 4 * l];
+      if (wide) {   // S' = e^{Lam_15} S + (k e^{Lam_15 - Lam})^T u
+        asm volatile("");   // keeps this a branch
+#pragma unroll
+        for (int t = 0; t < NCT; ++t)
+#pragma unroll
+          for (int kt = 0; kt < NKT; ++kt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) Sr[kt][t][i] *= el[(NKT * i + kt) / 4][(NKT * i + kt) % 4];
+#pragma unroll
+        for (int l = 0; l < NL / 4; ++l) el[l] = f32x4{1.f, 1.f, 1.f, 1.f};
+      }
+      wave_fence();
+      // ---- (I + L) u = v_e: one column per lane, u[4G + i] = token 4G + i
+      float u[SC];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        uint32_t x[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) x[t] = t < NCT ? __float_as_uint(ve[t < NCT ? t : 0][i]) : 0u;
+        transpose4(x);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) u[4 * t + i] = __uint_as_float(x[t]);
+      }
+#pragma unroll
+      for (int jb = 0; jb < 4; ++jb) {
+#pragma unroll
+        for (int i = 4 * jb + 1; i < SC; ++i) {
+          const f32x4 lr = *(const f32x4*)&sm.r.Lm[i][4 * jb];   // broadcast
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (4 * jb + r < i) u[i] = fmaf(lr[r], u[4 * jb + r], u[i]);
+        }
+      }
+      // the next rows: from here on the registers have room for them
+      prefetch(min(cc + 1, c_end - 1));
+      // ---- u as B operands: hi and lo pairs back to tokens 4g + i of the lane's columns
+      uint32_t uh[2][4], ul[2][4];
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+#pragma unroll
+        for (int G = 0; G < 4; ++G) split2(u[4 * G + 2 * m], u[4 * G + 2 * m + 1], uh[m][G], ul[m][G]);
+        transpose4(uh[m]);
+        transpose4(ul[m]);
+      }
+#pragma unroll
+      for (int t = 0; t < NCT; ++t) {
+        const i16x8 uh8 = pack8(uh[0][t], uh[1][t], uh[0][t], uh[1][t]);
+        const i16x8 ul8 = pack8(ul[0][t], ul[1][t], ul[0][t], ul[1][t]);
+        if (!MAP) {
+          f32x4 o = qs[t < NVT ? t : 0];
+          o = mma32(o, af, uh8);
+          ob[t < NVT ? t : 0] = mma32(o, af, ul8);
+        }
+#pragma unroll
+        for (int kt = 0; kt < NKT; ++kt) {
+          f32x4 s = Sr[kt][t];
+          s = mma32(s, kf[kt], uh8);
+          s = mma32(s, kf[kt], ul8);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) s[i] *= el[(NKT * i + kt) / 4][(NKT * i + kt) % 4];
+          Sr[kt][t] = s;
+        }
+      }
+    }
+    ot0 = t0;
+    if (MAP) {
+      uint32_t nz = 0;
+#pragma unroll
+      for (int kt = 0; kt < NKT; ++kt)
+#pragma unroll
+        for (int t = 0; t < NCT; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) nz |= __float_as_uint(Sr[kt][t][i]);
+      if (__ballot((nz << 1) != 0u) == 0ull) return cc + 1 - c_begin;
+    }
+  }
+  flush();
+  return -1;
+}
+
+// The new conv history of head hi: the last three conv inputs, from the projections or, for
+// fewer than three tokens, the old history (all read before any is written: the two may be
+// the same buffers).
+__device__ __forceinline__ void sub_new_history(const SubArgs& a, int lane, int bi, int hi) {
+  const int ch = hi * 64 + lane;
+  float x[3][3];
+#pragma unroll
+  for (int s = 0; s < 3; ++s)
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+      const int t = a.L - 3 + m;
+      x[s][m] = 0.f;
+      if (t >= 0) x[s][m] = bf16_bits_to_f32(a.px[s][(int64_t)bi * a.pxs0[s] + (int64_t)t * a.pxs1[s] + ch]);
+      else if (a.ph[s])
+        x[s][m] = bf16_bits_to_f32(a.ph[s][(int64_t)bi * a.phs0[s] + (int64_t)ch * a.phs1[s] + (int64_t)(t + 3) * a.phs2[s]]);
+    }
+#pragma unroll
+  for (int s = 0; s < 3; ++s)
+#pragma unroll
+    for (int m = 0; m < 3; ++m)
+      store_elem(a.nh[s], a.nhdt[s], bi * a.nhs0[s] + ch * a.nhs1[s] + m * a.nhs2[s], x[s][m]);
+}
+
+// One wave per workgroup.  SUB_MAIN: BH * nseg * nvh output waves, then BH * (nseg - 1) *
+// (d_k / 64) transition waves of the segments k >= 1.  SUB_FIX: the output waves of the
+// segments k >= 1.  Two waves per SIMD (256 VGPRs); d_k = 128 holds twice the state per
+// lane and runs one.
+template <bool F32IN, bool G16, bool GCH, bool PRO, int DK, int DV>
+__global__ __launch_bounds__(64, DK == 128 ? 1 : 2) void dgda_sub_kernel(SubArgs a) {
   static_assert(!PRO || (DK == 64 && DV == 64), "the fused prologue takes 64-channel heads");
   static_assert((DK == 32 || DK == 64 || DK == 128) && (DV == 32 || DV == 64), "head sizes");
-  constexpr int NKT = DK / 16;                   // 16-row tiles of the key side
-  constexpr int PK = SubSmem<AGG, PRO, DK, DV>::PK;
-  constexpr int AW = DV + DK;                    // row length of a segment map [N | M]
-  constexpr int NG = (DK > DV ? DK : DV) / 4;    // four-channel groups staged per token
-  constexpr int NPASS = NG > 16 ? NG / 16 : 1;   // staging passes of the 256 stagers (d_k = 128: two)
-  constexpr int NSTG = NG >= 16 ? 256 : 16 * NG; // stager threads
-  constexpr int NOW = DV / 16;                   // waves holding state columns (aggregate pass: the N waves)
-  constexpr int NMW = DK / 16;                   // aggregate pass: the M waves
-  constexpr bool HAS_NOCOL = !AGG && DV < 64;    // output passes with d_v = 32: waves 2, 3 hold no columns
-  const int wave = tid >> 6, lane = tid & 63;
-  const int g = lane >> 4, c16 = lane & 15;
+  constexpr int NKT = DK / 16, NVT = DV / 16;
+  constexpr int MC = DK < 64 ? DK : 64, NMT = MC / 16, NCG = DK / MC;   // transition columns per wave, waves per map
+  __shared__ SubSmem<PRO, DK> sm;
+  const int lane = threadIdx.x;
+  const int g = lane >> 4, c = lane & 15;
+  const int nout = a.mode == SUB_FIX ? a.BH * (a.nseg - 1) * a.nvh : a.BH * a.nseg * a.nvh;
+  const int AW = a.dvt + DK;
+  int id = blockIdx.x;
+  const bool map = id >= nout;
+  int k, bh, part;
+  if (map) {
+    id -= nout;
+    part = id % NCG;
+    id /= NCG;
+    bh = id / (a.nseg - 1);
+    k = id % (a.nseg - 1) + 1;
+  } else {
+    part = id % a.nvh;
+    id /= a.nvh;
+    if (a.mode == SUB_FIX) {
+      bh = id / (a.nseg - 1);
+      k = id % (a.nseg - 1) + 1;
+    } else {
+      bh = id / a.nseg;
+      k = id % a.nseg;
+    }
+  }
+  const int c0 = k * a.seglen;
+  int c1 = min(c0 + a.seglen, a.nchunks);
+  const bool last = k == a.nseg - 1;
   const int bi = bh / a.H, hi = bh % a.H;
-  const int64_t sidx = (int64_t)bh * a.nseg_max + k;
-  const bool last = k == n - 1;
-  if (!AGG && a.mode == SUB_ZERO && k > 0 && a.zc[sidx] < 0) return;  // M never vanished: the fix-up runs it
-  if (!AGG && a.mode == SUB_FIX && a.zc[sidx] >= 0) c_end = c_begin + a.zc[sidx];
-  const bool pred_final = !AGG && a.mode == SUB_FIX && (k == 1 || a.zc[sidx - 1] >= 0);
+  int* zc = a.zc + 2 * ((int64_t)bh * a.nseg + k);
+  if constexpr (PRO) {
+    for (int i = lane; i < 3 * 4 * 64; i += 64) {
+      const int s = i >> 8, j = (i >> 6) & 3, cl = i & 63;
+      sm.cw[s][j][cl] = load_elem(a.cw[s], a.cwdt, (int64_t)(hi * 64 + cl) * a.cwsc[s] + j * a.cwst[s]);
+    }
+    wave_fence();
+  }
 
-  // ---- start state: Sr[kt][i] = S[16 kt + 4g + i][col0 + c16]
-  f32x4 Sr[NKT];
-  const bool is_m = AGG && wave >= NOW;        // aggregate pass: M part of [N | M]
-  const bool nocol = HAS_NOCOL && wave >= NOW;
-  const int col0 = 16 * (is_m ? wave - NOW : (nocol ? 0 : wave));
-  const int col = col0 + c16;
+  if (map) {
+    const int col = MC * part + NMT * c;
+    f32x4 Sr[NKT][NMT];
+#pragma unroll
+    for (int kt = 0; kt < NKT; ++kt)
+#pragma unroll
+      for (int t = 0; t < NMT; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) Sr[kt][t][i] = (DK / 4) * g + NKT * i + kt == col + t ? 1.f : 0.f;
+    const int z = sub_run<true, F32IN, G16, GCH, PRO, DK, DV>(a, sm, lane, bh, 0, c0, c1, Sr);
+    if (lane == 0) {
+      zc[part] = z;
+      if (NCG == 1) zc[1] = z;
+    }
+    if (z < 0 && !last) {
+      uint32_t* dst = (uint32_t*)(a.agg + ((int64_t)bh * a.nseg + k) * DK * AW + DK * a.dvt) + col / 2;
+#pragma unroll
+      for (int kt = 0; kt < NKT; ++kt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int t = 0; t < NMT; t += 2) {
+            uint32_t* row = dst + ((DK / 4) * g + NKT * i + kt) * DK + t / 2;
+            split2(Sr[kt][t][i], Sr[kt][t + 1][i], row[0], row[DK / 2]);
+          }
+    }
+    return;
+  }
+
+  const int col = DV * part + NVT * c;
+  f32x4 Sr[NKT][NVT];
   auto fill = [&](auto load) {
 #pragma unroll
     for (int kt = 0; kt < NKT; ++kt)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) Sr[kt][i] = load(16 * kt + 4 * g + i);
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int t = 0; t < NVT; ++t) Sr[kt][t][i] = load((DK / 4) * g + NKT * i + kt, t);
   };
-  if (AGG) {
-    fill([&](int r) { return (is_m && r == col) ? 1.f : 0.f; });
-  } else if (nocol) {
-    fill([&](int) { return 0.f; });
+  // the state in slot s of the sequence
+  auto slot = [&](int s) {
+    return (f32x4*)(a.agg + ((int64_t)bh * a.nseg + s) * DK * AW + DK * DV * part) + lane * NKT;
+  };
+  auto fetch = [&](const f32x4* src) {
+#pragma unroll
+    for (int t = 0; t < NVT; ++t)
+#pragma unroll
+      for (int kt = 0; kt < NKT; ++kt) Sr[kt][t] = src[64 * NKT * t + kt];
+  };
+  int z = -1;
+  if (a.mode == SUB_FIX) {
+    z = zc[0] < 0 || zc[1] < 0 ? -1 : max(zc[0], zc[1]);
+    if (z >= 0) c1 = c0 + z;
+    fetch(slot(k - 1));
   } else if (k == 0 && a.has_s0) {
-    const int64_t o = bi * a.s0.s0 + hi * a.s0.s1 + col * a.s0.s3, rs = a.s0.s2;
-    if (a.s0.dt == MABA_F32) fill([&](int r) { return ((const float*)a.s0.p)[o + r * rs]; });
-    else if (a.s0.dt == MABA_BF16) fill([&](int r) { return bf16_bits_to_f32(((const uint16_t*)a.s0.p)[o + r * rs]); });
-    else fill([&](int r) { return __half2float(((const __half*)a.s0.p)[o + r * rs]); });
-  } else if (k == 0 || a.mode == SUB_ZERO) {
-    fill([&](int) { return 0.f; });
-  } else if (pred_final) {
-    const float* src = a.agg + (sidx - 1) * DK * AW + col;   // S_k = N_{k-1}
-    fill([&](int r) { return src[r * AW]; });
+    const int64_t o = bi * a.s0.s0 + hi * a.s0.s1 + col * a.s0.s3, rs = a.s0.s2, cs = a.s0.s3;
+    if (a.s0.dt == MABA_F32) fill([&](int r, int t) { return ((const float*)a.s0.p)[o + r * rs + t * cs]; });
+    else if (a.s0.dt == MABA_BF16) fill([&](int r, int t) { return bf16_bits_to_f32(((const uint16_t*)a.s0.p)[o + r * rs + t * cs]); });
+    else fill([&](int r, int t) { return __half2float(((const __half*)a.s0.p)[o + r * rs + t * cs]); });
   } else {
-    // the predecessor's M did not vanish: from the last exact N_j apply the maps of the
-    // segments between
-    const int* zc = a.zc + (int64_t)bh * a.nseg_max;
-    int j = k - 1;
-    while (j > 0 && zc[j] < 0) --j;
-    const float* agg = a.agg + (int64_t)bh * a.nseg_max * DK * AW;
-    const float* src = agg + (int64_t)j * DK * AW + col;
-    fill([&](int r) { return src[r * AW]; });
-    for (int m = j + 1; m < k; ++m) apply_map<DK, DV>(agg + (int64_t)m * DK * AW, Sr, col0, c16, g);
+    fill([&](int, int) { return 0.f; });
   }
-  // the slab's loads complete here: inside the loop the compiler would otherwise count
-  // them as pending and wait for every outstanding load (the prefetch) before using it
-#pragma unroll
-  for (int kt = 0; kt < NKT; ++kt)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(Sr[kt][i]));
-
-  const int64_t qb = (int64_t)bi * a.qs0 + (int64_t)hi * a.qs1;
-  const int64_t kb = (int64_t)bi * a.ks0 + (int64_t)hi * a.ks1;
-  const int64_t vb = (int64_t)bi * a.vs0 + (int64_t)hi * a.vs1;
-  const int64_t gb = (int64_t)bi * a.gs0 + (int64_t)hi * a.gs1;
-  const int64_t bb = (int64_t)bi * a.bs0 + (int64_t)hi * a.bs1;
-  const int64_t wb = (int64_t)bi * a.ws0 + (int64_t)hi * a.ws1;
-  const int64_t obase = (int64_t)bi * a.os0 + (int64_t)hi * a.os1 + col;
-
-  // ---- register prefetch of one sub-chunk's inputs: item (token st, channels c4..c4+3),
-  // tokens along the 16 lanes of a DPP row; pass pp covers channel groups 16 pp .. 16 pp + 15
-  // (key-side rows below d_k, value-side rows below d_v: both bounds fall on wave boundaries)
-  const bool stager = tid < NSTG;
-  const int st = tid & 15;
-  const int c4 = (tid >> 4) * 4;                 // pass 0; pass pp adds 64 pp
-  Raw4<F32IN> pq[NPASS] = {}, pk[NPASS] = {}, pv[NPASS] = {};
-  Raw4<!G16> pg[NPASS] = {}, pb[NPASS] = {}, pw[NPASS] = {};
-  // fused prologue: conv taps of tokens t-3 .. t (bf16 bits; taps before token 0 are
-  // loaded at token 0 and replaced by the history in the first sub-chunk), the gate
-  // projections and SiLU(conv k) of the staged token.  The head's conv weights go to LDS
-  // once per segment (the previous segment's last reads of them were before its last
-  // post-staging barrier).
-  i16x4 tq[4] = {}, tk[4] = {}, tv[4] = {}, xg[3] = {};
-  f32x4 kc = {};
-  const int ch = hi * 64 + c4;   // the stager's first channel of the projection rows
+  sub_run<false, F32IN, G16, GCH, PRO, DK, DV>(a, sm, lane, bh, col, c0, c1, Sr);
   if constexpr (PRO) {
-    for (int i = tid; i < 3 * 4 * 64; i += blockDim.x) {
-      const int s = i >> 8, j = (i >> 6) & 3, cl = i & 63;
-      sm.cw[s][j][cl] = load_elem(a.cw[s], a.cwdt, (int64_t)(hi * 64 + cl) * a.cwsc[s] + j * a.cwst[s]);
-    }
-    lds_barrier();
+    // after the sequence's first segment has read the old history, which this may overwrite
+    if (last && part == 0 && (a.nseg == 1 || a.mode == SUB_FIX)) sub_new_history(a, lane, bi, hi);
   }
-  // row tr + st of projection s at the stager's channels: a uniform base pointer plus a
-  // 32-bit lane offset, clamped to row 0 (rows before token 0 are replaced by the history)
-  auto prow = [&](int s, int tr) {
-    const uint16_t* base = a.px[s] + (int64_t)bi * a.pxs0[s];
-    return *(const i16x4*)(base + max(st * a.pxs1[s] + ch + tr * a.pxs1[s], ch));
-  };
-  auto prefetch = [&](int cc) {
-    const int tok = cc * SC + st;
-    if (!stager || tok >= a.L) return;
-    if constexpr (PRO) {
-      const int t0 = cc * SC;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if (!AGG) tq[j] = prow(0, t0 - 3 + j);
-        tk[j] = prow(1, t0 - 3 + j);
-        tv[j] = prow(2, t0 - 3 + j);
-      }
-#pragma unroll
-      for (int s = 0; s < 3; ++s) xg[s] = prow(3 + s, t0);
-      return;
-    }
-#pragma unroll
-    for (int pp = 0; pp < NPASS; ++pp) {
-      const int cp = c4 + 64 * pp;
-      if (cp < DK) {
-        pk[pp] = load_raw4<F32IN>(a.k, kb + (int64_t)tok * a.ks2 + cp);
-        if (!AGG) pq[pp] = load_raw4<F32IN>(a.q, qb + (int64_t)tok * a.qs2 + cp);
-        pg[pp] = load_gate4<G16>(a.gp, gb + (int64_t)tok * a.gs2, a.gs3, cp);
-        pb[pp] = load_gate4<G16>(a.bp, bb + (int64_t)tok * a.bs2, a.bs3, cp);
-      }
-      if (cp < DV) {
-        pv[pp] = load_raw4<F32IN>(a.vp, vb + (int64_t)tok * a.vs2 + cp);
-        pw[pp] = load_gate4<G16>(a.wp, wb + (int64_t)tok * a.ws2, a.ws3, cp);
-      }
-    }
-  };
-  prefetch(c_begin);
-
-  // outputs of a sub-chunk are stored during the next one's staging, before its prefetch:
-  // vmcnt counts stores, and a store issued just before the staging's wait for the
-  // prefetched rows would make that wait cover the store's latency
-  f32x4 obuf = {0.f, 0.f, 0.f, 0.f};
-  int ot0 = -1, ont = 0;
-  auto flush = [&]() {
-    if (AGG || ot0 < 0) return;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int t = 4 * g + i;
-      if (t < ont) {
-        const int64_t off = obase + (int64_t)(ot0 + t) * a.os2;
-        if (OBF) ((uint16_t*)a.op)[off] = a.of16 ? __half_as_ushort(__float2half(obuf[i])) : f32_to_bf16_bits(obuf[i]);
-        else ((float*)a.op)[off] = obuf[i];
-      }
-    }
-  };
-  // fused prologue: SiLU(depthwise conv) of the stager's four channels of stream s from
-  // the taps (oldest first)
-  auto conv4 = [&](int s, const i16x4 (&t)[4]) {
-    f32x4 w[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) w[j] = *(const f32x4*)&sm.cw[s][j][c4];
-    f32x4 y;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      float acc = w[3][e] * bf16_val(t[3][e]);
-      acc = fmaf(w[2][e], bf16_val(t[2][e]), acc);
-      acc = fmaf(w[1][e], bf16_val(t[1][e]), acc);
-      acc = fmaf(w[0][e], bf16_val(t[0][e]), acc);
-      y[e] = pro_silu(acc);
-    }
-    return y;
-  };
-  // taps before token 0 (first sub-chunk of the sequence) come from the history, or are zero
-  auto hist_taps = [&](int s, i16x4 (&t)[4]) {
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      if (st - 3 + j >= 0) continue;
-      i16x4 h = {0, 0, 0, 0};
-      if (a.ph[s]) {
-        const uint16_t* hp = a.ph[s] + (int64_t)bi * a.phs0[s] + (int64_t)ch * a.phs1[s] + (int64_t)(st + j) * a.phs2[s];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) h[e] = (short)hp[(int64_t)e * a.phs1[s]];
-      }
-      t[j] = h;
-    }
-  };
-  // before the loop-top barrier of sub-chunk cc: SiLU(conv k) of the prefetched taps and the
-  // wave's |k|^2 partial per token (lanes 16 m + st hold channel groups 4 wave + m of token st)
-  auto pre_norm = [&](int cc) {
-    if constexpr (PRO) {
-      if (!stager) return;
-      if (cc == 0) {
-        if (!AGG) hist_taps(0, tq);
-        hist_taps(1, tk);
-        hist_taps(2, tv);
-      }
-      kc = conv4(1, tk);
-      float ss = kc[0] * kc[0] + kc[1] * kc[1] + kc[2] * kc[2] + kc[3] * kc[3];
-      ss += __shfl_xor(ss, 16);
-      ss += __shfl_xor(ss, 32);
-      if (lane < 16) sm.nrm[cc & 1][wave][lane] = ss;
-    }
-  };
-
-  bool idle = nocol;                     // aggregate pass, M waves: the slab is exactly zero
-  if (AGG && tid < NMW) s_mzero[tid] = 0;
-  if (tid == 0) sm.big[c_begin & 1] = 0;   // read after the first loop-top barrier
-  int c_stop = -1;
-
-  for (int c = c_begin; c < c_end; ++c) {
-    const int t0 = c * SC;
-    const int nt = min(SC, a.L - t0);
-    pre_norm(c);
-    lds_barrier();   // the previous sub-chunk is done with the shared buffers
-    if (AGG) {
-      bool allz = true;
-#pragma unroll
-      for (int m = 0; m < NMW; ++m) allz = allz && s_mzero[m] != 0;
-      if (allz) {   // workgroup-uniform
-        c_stop = c;
-        break;
-      }
-    }
-    // ---- (1) stage and scale.  The 16 lanes of a DPP row hold the 16 tokens of one
-    // four-channel group, so the per-channel prefix Lam over the sub-chunk is a row scan
-    // in registers.  Tokens past the end stage as zeros (no decay, no write).
-    if (stager) {
-      const bool on = st < nt;
-      const f32x4 z = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int pp = 0; pp < NPASS; ++pp) {
-        const int cp = c4 + 64 * pp;
-        f32x4 rk, rv, rq, rg, rb, rw;
-        if constexpr (PRO) {
-          const float n2 = (sm.nrm[c & 1][0][st] + sm.nrm[c & 1][1][st]) + (sm.nrm[c & 1][2][st] + sm.nrm[c & 1][3][st]);
-          rk = kc * pro_knorm_inv(n2, a.eps);
-          rv = conv4(2, tv);
-          rq = AGG ? z : conv4(0, tq);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            rg[i] = pro_log_decay(bf16_val(xg[0][i]));
-            rb[i] = pro_sigmoid(bf16_val(xg[1][i]));
-            rw[i] = pro_sigmoid(bf16_val(xg[2][i]));
-          }
-        } else {
-          const bool f16 = a.f16 != 0;
-          rk = raw_f32<F32IN>(pk[pp], f16); rv = raw_f32<F32IN>(pv[pp], f16);
-          rq = AGG ? z : raw_f32<F32IN>(pq[pp], f16);
-          rg = raw_f32<!G16>(pg[pp], f16); rb = raw_f32<!G16>(pb[pp], f16); rw = raw_f32<!G16>(pw[pp], f16);
-        }
-        if (cp < DV) {
-          f32x4 wv;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) wv[i] = on ? rw[i] * rv[i] : 0.f;
-          *(f32x4*)&sm.WV[st][cp] = wv;
-        }
-        if (cp >= DK) continue;
-        const f32x4 kk = on ? rk : z;
-        f32x4 la, bk, lam, l15;
-        float mx = 0.f;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float l = a.use_log ? rg[i] : __logf(fmaxf(rg[i], 1e-20f));
-          la[i] = on ? l : 0.f;
-          bk[i] = on ? rb[i] * rk[i] : 0.f;
-          lam[i] = row16_incl_scan(la[i]);
-          l15[i] = __shfl(lam[i], lane | 15);
-          mx = fmaxf(mx, fabsf(lam[i]));
-        }
-        if (!(mx <= SUB_MFMA_RANGE)) sm.big[c & 1] = 1;   // benign race: every writer stores 1
-        // fp32 rows for the exact pair-by-pair path
-        *(f32x4*)&sm.K[st][cp] = kk;
-        *(f32x4*)&sm.BK[st][cp] = bk;
-        *(f32x4*)&sm.LA[st][cp] = lam;
-        if (!AGG) *(f32x4*)&sm.Q[st][cp] = on ? rq : z;
-        // scaled operands, split into bf16 hi + lo; e^{-Lam} is used only when |Lam| <= 64
-        f32x4 e, ki, kcs, bke;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          e[i] = __expf(lam[i]);
-          ki[i] = kk[i] * __expf(-lam[i]);
-          kcs[i] = kk[i] * __expf(l15[i] - lam[i]);
-          bke[i] = bk[i] * e[i];
-        }
-        if (st == SC - 1) *(f32x4*)&sm.elast[cp] = e;
-        i16x4 h, l;
-        split4(bke, h, l);
-        *(i16x4*)(sm.BKEh + st * PK + cp) = h;
-        *(i16x4*)(sm.BKEl + st * PK + cp) = l;
-        split4(ki, h, l);
-        *(i16x4*)(sm.KIh + st * PK + cp) = h;
-        *(i16x4*)(sm.KIl + st * PK + cp) = l;
-        if (!AGG) {
-          split4((on ? rq : z) * e, h, l);
-          *(i16x4*)(sm.QEh + st * PK + cp) = h;
-          *(i16x4*)(sm.QEl + st * PK + cp) = l;
-        }
-        split4(kcs, h, l);   // transposed: row = channel, column = token
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          sm.KCh[(cp + i) * TP + st] = h[i];
-          sm.KCl[(cp + i) * TP + st] = l[i];
-        }
-      }
-    }
-    if (tid == 0) sm.big[(c + 1) & 1] = 0;   // last read in the previous sub-chunk
-    flush();
-    if (c + 1 < c_end) prefetch(c + 1);
-    lds_barrier();
-    const bool big = sm.big[c & 1] != 0;   // workgroup-uniform
-
-    // ---- (4) L and its inverse (wave 0), A (wave 1); every wave: v_e and q S for its columns
-    // tile of X (rows i) times KI^T (columns j): lane (c16, g) gets rows 4g + r of column j = c16
-    auto tile_mfma = [&](const short* Xh, const short* Xl) {
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int p = 0; p < DK / 32; ++p) {
-        const i16x8 xh = lds8(Xh, c16, 32 * p + 8 * g, PK), xl = lds8(Xl, c16, 32 * p + 8 * g, PK);
-        const i16x8 kh = lds8(sm.KIh, c16, 32 * p + 8 * g, PK), kl = lds8(sm.KIl, c16, 32 * p + 8 * g, PK);
-        acc = mma32(acc, kh, xh);   // D[j][i]: rows of KI as A, rows of X as B
-        acc = mma32(acc, kh, xl);
-        acc = mma32(acc, kl, xh);
-      }
-      return acc;   // lane (c16, g), element r: X_i . KI_j with i = c16, j = 4g + r
-    };
-    if (big) {
-      // strong decay: L and A pair by pair in fp32, exact exponentials (all 256 threads of
-      // the first four waves, pair (i, j) = (t / 16, t % 16))
-      if (tid < SC * SC) {
-        const int i = tid >> 4, j = tid & 15;
-        float lv = 0.f, av = 0.f;
-        if (j <= i) {
-          for (int cc = 0; cc < DK; ++cc) {
-            const float d = __expf(sm.LA[i][cc] - sm.LA[j][cc]) * sm.K[j][cc];
-            lv = fmaf(sm.BK[i][cc], d, lv);
-            if (!AGG) av = fmaf(sm.Q[i][cc], d, av);
-          }
-        }
-        sm.Lq[i][j & 3][j >> 2] = j < i ? lv : 0.f;
-        if (!AGG) {
-          const short hb = bf16_rn(av);
-          sm.Ah[i * TP + j] = hb;
-          sm.Al[i * TP + j] = bf16_rn(av - bf16_val(hb));
-        }
-      }
-      lds_barrier();
-    } else if (wave == 0) {
-      const f32x4 d = tile_mfma(sm.BKEh, sm.BKEl);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) sm.Lq[c16][r][g] = (4 * g + r < c16) ? d[r] : 0.f;   // L[c16][4g + r]
-    } else if (!AGG && wave == 1) {
-      const f32x4 d = tile_mfma(sm.QEh, sm.QEl);
-      f32x4 v;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) v[r] = (4 * g + r <= c16) ? d[r] : 0.f;
-      i16x4 h, l;
-      split4(v, h, l);
-      *(i16x4*)(sm.Ah + c16 * TP + 4 * g) = h;   // row i = c16, columns j = 4g .. 4g + 3
-      *(i16x4*)(sm.Al + c16 * TP + 4 * g) = l;
-    }
-    if (wave == 0) {
-      // T = (I + L)^-1 by forward substitution, x_i = [i == j] - sum_{m<i} L_im x_m for
-      // column j: the four lanes 4j .. 4j+3 split the sum by m mod 4 (lane p keeps x_m for
-      // m = p, p + 4, ...) and add their parts with two quad DPP steps, so a step costs
-      // four FMAs and two DPP adds.  L[i][m] = 0 for m >= i and x_m = 0 until computed,
-      // so the products need no guards.  (Wave 0 reads its own LDS writes above in order.)
-      const int jc = lane >> 2, p = lane & 3;
-      auto qadd = [](float v, auto ctrl_c) {
-        return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(ctrl_c)::value,
-                                                              0xf, 0xf, false));
-      };
-      float xm[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int i = 0; i < SC; ++i) {
-        const f32x4 lv = *(const f32x4*)&sm.Lq[i][p][0];   // L[i][p + 4 r], r = 0..3
-        float part = (p == 0 && i == jc) ? 1.f : 0.f;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) part = fmaf(-lv[r], xm[r], part);
-        part = qadd(part, std::integral_constant<int, 0xB1>{});   // quad_perm [1,0,3,2]
-        part = qadd(part, std::integral_constant<int, 0x4E>{});   // quad_perm [2,3,0,1]
-        if (p == (i & 3)) xm[i >> 2] = part;
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {   // T[p + 4r][jc]
-        const short hb = bf16_rn(xm[r]);
-        sm.Th[(p + 4 * r) * TP + jc] = hb;
-        sm.Tl[(p + 4 * r) * TP + jc] = bf16_rn(xm[r] - bf16_val(hb));
-      }
-    }
-    // v_e = w*v - (b k e^Lam) S and q S: permuted K over the slab's row groups, lane
-    // (c16, g) gets tokens 4g + i of column col
-    i16x4 Sh[NKT], Sl[NKT];
-#pragma unroll
-    for (int kt = 0; kt < NKT; ++kt) split4(Sr[kt], Sh[kt], Sl[kt]);
-    auto state_product = [&](const short* Xh, const short* Xl) {
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int p = 0; p < DK / 32; ++p) {
-        const i16x8 xh = lds4x2(Xh, c16, 32 * p + 4 * g, PK), xl = lds4x2(Xl, c16, 32 * p + 4 * g, PK);
-        const i16x8 bh8 = cat8(Sh[2 * p], Sh[2 * p + 1]), bl8 = cat8(Sl[2 * p], Sl[2 * p + 1]);
-        acc = mma32(acc, xh, bh8);
-        acc = mma32(acc, xh, bl8);
-        acc = mma32(acc, xl, bh8);
-      }
-      return acc;
-    };
-    f32x4 ve = {0.f, 0.f, 0.f, 0.f}, qs = ve;
-    if (!idle) {
-      ve = state_product(sm.BKEh, sm.BKEl);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) ve[i] = (is_m ? 0.f : sm.WV[4 * g + i][col]) - ve[i];
-    }
-    if (!AGG && !idle) qs = state_product(sm.QEh, sm.QEl);
-    lds_barrier();   // T (and A) are ready
-
-    // ---- (5) u = T v_e, (6) o = q S + A u, (7) S' = diag(e^{Lam_15}) S + K_C^T u
-    if (idle) continue;
-    i16x4 vh, vl;
-    split4(ve, vh, vl);
-    f32x4 u = {0.f, 0.f, 0.f, 0.f};
-    {
-      const i16x4 th = lds4(sm.Th, c16, 4 * g, TP), tl = lds4(sm.Tl, c16, 4 * g, TP);   // T[c16][4g..]
-      // D[m][n] = sum_k T[m][k] v_e[k][n]: A-operand rows of T, B-operand the v_e fragment
-      u = mma16(u, th, vh);
-      u = mma16(u, th, vl);
-      u = mma16(u, tl, vh);
-    }
-    i16x4 uh, ul;
-    split4(u, uh, ul);
-    if (!AGG) {
-      const i16x4 ah = lds4(sm.Ah, c16, 4 * g, TP), al = lds4(sm.Al, c16, 4 * g, TP);
-      f32x4 o = qs;
-      o = mma16(o, ah, uh);
-      o = mma16(o, ah, ul);
-      o = mma16(o, al, uh);
-      obuf = o;
-      ot0 = t0;
-      ont = nt;
-    }
-#pragma unroll
-    for (int kt = 0; kt < NKT; ++kt) {
-      const f32x4 el = *(const f32x4*)(sm.elast + 16 * kt + 4 * g);
-      f32x4 acc = Sr[kt] * el;
-      const i16x4 kh = lds4(sm.KCh, 16 * kt + c16, 4 * g, TP), kl = lds4(sm.KCl, 16 * kt + c16, 4 * g, TP);
-      acc = mma16(acc, kh, uh);
-      acc = mma16(acc, kh, ul);
-      acc = mma16(acc, kl, uh);
-      Sr[kt] = acc;
-    }
-    if (AGG && is_m) {
-      bool nz = false;
-#pragma unroll
-      for (int kt = 0; kt < NKT; ++kt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) nz |= Sr[kt][i] != 0.f;
-      idle = __ballot(nz) == 0ull;
-      if (lane == 0) s_mzero[wave - NOW] = idle;   // read after the next loop-top barrier
-    }
-  }
-
-  flush();   // the last sub-chunk's outputs
-  if (nocol) return;
-  // ---- segment results
   auto drain = [&](auto put) {
 #pragma unroll
     for (int kt = 0; kt < NKT; ++kt)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) put(16 * kt + 4 * g + i, Sr[kt][i]);
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int t = 0; t < NVT; ++t) put((DK / 4) * g + NKT * i + kt, t, Sr[kt][t][i]);
   };
-  if (AGG) {
-    if (tid == 0) a.zc[sidx] = c_stop >= 0 ? c_stop - c_begin : -1;
-    if (c_stop < 0) {  // M never vanished: [N | M] for the fix-up pass
-      float* dst = a.agg + sidx * DK * AW + (is_m ? DV : 0) + col;
-      drain([&](int r, float v) { dst[r * AW] = v; });
-    }
-  } else if (a.mode == SUB_ZERO && !last) {  // N_k for the fix-up pass
-    float* dst = a.agg + sidx * DK * AW + col;
-    drain([&](int r, float v) { dst[r * AW] = v; });
-  } else if (last && !(a.mode == SUB_FIX && a.zc[sidx] >= 0)) {
-    const int64_t o = bi * a.sf.s0 + hi * a.sf.s1 + col * a.sf.s3, rs = a.sf.s2;
-    if (a.sf.dt == MABA_F32) drain([&](int r, float v) { ((float*)a.sf.p)[o + r * rs] = v; });
+  if (last && (a.nseg == 1 || a.mode == SUB_FIX)) {
+    // (never in the launch that reads the initial state from another wave: the two may be one buffer)
+    if (z >= 0) fetch(slot(k));   // the zero start's end state is the true one
+    const int64_t o = bi * a.sf.s0 + hi * a.sf.s1 + col * a.sf.s3, rs = a.sf.s2, cs = a.sf.s3;
+    if (a.sf.dt == MABA_F32) drain([&](int r, int t, float v) { ((float*)a.sf.p)[o + r * rs + t * cs] = v; });
     else if (a.sf.dt == MABA_BF16)
-      drain([&](int r, float v) { ((uint16_t*)a.sf.p)[o + r * rs] = f32_to_bf16_bits(v); });
-    else drain([&](int r, float v) { ((__half*)a.sf.p)[o + r * rs] = __float2half(v); });
+      drain([&](int r, int t, float v) { ((uint16_t*)a.sf.p)[o + r * rs + t * cs] = f32_to_bf16_bits(v); });
+    else drain([&](int r, int t, float v) { ((__half*)a.sf.p)[o + r * rs + t * cs] = __float2half(v); });
+  } else if (a.mode == SUB_MAIN) {   // N_k
+    f32x4* dst = slot(k);
+#pragma unroll
+    for (int t = 0; t < NVT; ++t)
+#pragma unroll
+      for (int kt = 0; kt < NKT; ++kt) dst[64 * NKT * t + kt] = Sr[kt][t];
   }
 }
 
-// Output passes: 256 threads (four waves).  Aggregate pass: one wave per 16 columns of
-// [N | M], (d_v + d_k) / 16 waves.
-template <bool AGG, bool F32IN, bool G16, bool OBF, bool PRO, int DK, int DV>
-__global__ __launch_bounds__(AGG ? 4 * (DK + DV) : 256, AGG ? 1 : 2) void dgda_sub_kernel(SubArgs a) {
-  __shared__ SubSmem<AGG, PRO, DK, DV> sm;
-  __shared__ int s_mzero[DK / 16];
-  // Aggregate and fix-up passes: one workgroup per segment k >= 1.  Output pass: slot
-  // w covers the sub-chunks [U w, U w + U) of the (b,h)-major order, one segment per
-  // sequence it touches.
-  const bool per_segment = AGG || a.mode == SUB_FIX;
-  const int64_t total = (int64_t)a.BH * a.nchunks;
-  int64_t G = per_segment ? 0 : (int64_t)blockIdx.x * a.U;
-  const int64_t Gend = per_segment ? 1 : min(G + a.U, total);
-  while (G < Gend) {
-    int bh, k, n, c0, c1;
-    if (per_segment) {
-      const int per = a.nseg_max - 1;
-      bh = blockIdx.x / per;
-      k = blockIdx.x % per + 1;
-      n = seg_count_of(a.nchunks, a.U, bh);
-      if (k >= n) return;
-      seg_range_of(a.nchunks, a.U, bh, k, n, c0, c1);
-      G = Gend;
-    } else {
-      bh = (int)(G / a.nchunks);
-      const int64_t s = (int64_t)bh * a.nchunks;
-      c0 = (int)(G - s);
-      c1 = (int)(min(Gend, s + a.nchunks) - s);
-      k = c0 == 0 ? 0 : (int)(blockIdx.x - s / a.U);
-      n = seg_count_of(a.nchunks, a.U, bh);
-      G = s + c1;
-    }
-    // the thread index and the argument pointer pass through empty asm statements so
-    // that nothing derived from them is held across the segments
-    int tid = threadIdx.x;
-    asm volatile("" : "+v"(tid));
-    KSubArgs* ap = (KSubArgs*)__builtin_amdgcn_kernarg_segment_ptr();
-    asm volatile("" : "+s"(ap));
-    sub_segment<AGG, F32IN, G16, OBF, PRO, DK, DV>(*ap, sm, s_mzero, tid, bh, k, n, c0, c1);
+// Start states: slot k of a sequence holds N_k, segment k's end state from a zero start
+// (from the initial state for k = 0), and becomes the true one, S_{k+1} = M_k S_k + N_k,
+// where M_k survived (else N_k already is it).  One wave per 16 columns of one sequence
+// walks its slots in order; M (stored split) and S as bf16 hi + lo, three products.  A
+// slot's loads do not depend on the walk, so they run DEPTH slots ahead (what a wave may
+// have outstanding, 63 operations, allows no more).
+template <int DK>
+__global__ __launch_bounds__(64, 1) void dgda_sub_scan_kernel(SubArgs a) {
+  constexpr int NKT = DK / 16, NP = DK / 32, NL = DK / 4;
+  constexpr int DEPTH = DK == 128 ? 1 : 3;
+  const int lane = threadIdx.x;
+  const int g = lane >> 4, c = lane & 15;
+  const int bh = blockIdx.x, AW = a.dvt + DK;
+  const int* zc = a.zc + 2 * (int64_t)bh * a.nseg;
+  float* agg = a.agg + (int64_t)bh * a.nseg * DK * AW;
+  const int64_t slot = (int64_t)DK * AW;
+  const int own = blockIdx.y * 64 * 4 * NKT + lane * 4 * NKT;   // a tile of 16 columns, as sub_run's waves hold it
+  const int kend = a.nseg - 1;   // slots 1 .. kend - 1 (the last segment's end state starts nothing)
+
+  // which slots survived; most calls have none and end here
+  __shared__ uint8_t alive[SUB_MAX_SEG];
+  int any = 0;
+  for (int k = threadIdx.x; k < kend; k += blockDim.x) {
+    alive[k] = k >= 1 && (zc[2 * k] < 0 || zc[2 * k + 1] < 0);
+    any |= alive[k];
   }
-}
+  if (!__syncthreads_or(any)) return;
 
-
-// The aggregate, zero-start and fix-up passes (one zero-start pass when every sequence
-// fits one slot).  PRO: the fused-prologue inputs (bf16 projections).  f32in: fp32 q, k,
-// v; g16: 16-bit gates in q's format (only with 16-bit q, k, v); obf: 16-bit output.
-// The caller has set the workspace pointers for d_k x (d_v + d_k) segment maps.
-template <bool PRO, int DK, int DV>
-int run_sub_passes(SubArgs& a, bool f32in, bool g16, bool obf, hipStream_t stream) {
-#define MABA_SUB_K(AGG, F, G, O, P) dgda_sub_kernel<AGG, F, G, O, P, DK, DV>
-  auto launch_out = [&](int mode) {
-    a.mode = mode;
-    const dim3 grid(mode == SUB_ZERO ? (unsigned)ceil_div((int64_t)a.BH * a.nchunks, a.U)
-                                     : (unsigned)(a.BH * (a.nseg_max - 1)));
-    if constexpr (PRO) {
-      if (obf) hipLaunchKernelGGL((MABA_SUB_K(false, false, false, true, true)), grid, dim3(256), 0, stream, a);
-      else hipLaunchKernelGGL((MABA_SUB_K(false, false, false, false, true)), grid, dim3(256), 0, stream, a);
-    } else if (f32in) {
-      if (obf) hipLaunchKernelGGL((MABA_SUB_K(false, true, false, true, false)), grid, dim3(256), 0, stream, a);
-      else hipLaunchKernelGGL((MABA_SUB_K(false, true, false, false, false)), grid, dim3(256), 0, stream, a);
-    } else if (g16) {
-      if (obf) hipLaunchKernelGGL((MABA_SUB_K(false, false, true, true, false)), grid, dim3(256), 0, stream, a);
-      else hipLaunchKernelGGL((MABA_SUB_K(false, false, true, false, false)), grid, dim3(256), 0, stream, a);
-    } else {
-      if (obf) hipLaunchKernelGGL((MABA_SUB_K(false, false, false, true, false)), grid, dim3(256), 0, stream, a);
-      else hipLaunchKernelGGL((MABA_SUB_K(false, false, false, false, false)), grid, dim3(256), 0, stream, a);
+  // tile kt: rows NKT m + kt, so element i of the lane is row NL g + NKT i + kt, as in sub_run
+  struct Slot { f32x4 n[NKT]; i16x8 mh[NKT][NP], ml[NKT][NP]; } buf[DEPTH];
+  auto load = [&](Slot& s, int k) {
+    const float* X = agg + min(k, kend - 1) * slot;
+#pragma unroll
+    for (int kt = 0; kt < NKT; ++kt) {
+      s.n[kt] = *(const f32x4*)(X + own + 4 * kt);
+      const short* mrow = (const short*)(X + DK * a.dvt + (NKT * c + kt) * DK) + NL * g;
+#pragma unroll
+      for (int p = 0; p < NP; ++p) {
+        s.mh[kt][p] = *(const i16x8*)(mrow + 8 * p);
+        s.ml[kt][p] = *(const i16x8*)(mrow + DK + 8 * p);
+      }
     }
-    return check_launch("dgda_prefill/sub-chunk output");
   };
-  if (a.nseg_max == 1) {
-    a.zc = nullptr;
-    return launch_out(SUB_ZERO);
+  f32x4 Sr[NKT];
+#pragma unroll
+  for (int kt = 0; kt < NKT; ++kt) Sr[kt] = *(const f32x4*)(agg + own + 4 * kt);
+#pragma unroll
+  for (int d = 0; d < DEPTH; ++d) load(buf[d], 1 + d);
+  // The step is straight-line code (a vanished slot's products are dropped and its N stored
+  // back), so that the wait for one slot's loads is not a wait for the later slots'.
+  auto step = [&](Slot& b, int k, bool alive) {
+    i16x8 sh[NP], sl[NP];
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      uint32_t h[4], l[4];
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) {
+        const int l0 = 8 * p + e, l1 = l0 + 1;
+        split2(Sr[l0 % NKT][l0 / NKT], Sr[l1 % NKT][l1 / NKT], h[e / 2], l[e / 2]);
+      }
+      sh[p] = pack8(h[0], h[1], h[2], h[3]);
+      sl[p] = pack8(l[0], l[1], l[2], l[3]);
+    }
+    float* X = agg + k * slot;
+#pragma unroll
+    for (int kt = 0; kt < NKT; ++kt) {
+      f32x4 acc = b.n[kt];
+#pragma unroll
+      for (int p = 0; p < NP; ++p) {
+        acc = mma32(acc, b.mh[kt][p], sh[p]);
+        acc = mma32(acc, b.mh[kt][p], sl[p]);
+        acc = mma32(acc, b.ml[kt][p], sh[p]);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) Sr[kt][i] = alive ? acc[i] : b.n[kt][i];
+      *(f32x4*)(X + own + 4 * kt) = Sr[kt];
+    }
+  };
+  int k = 1;
+  for (; k + DEPTH <= kend; k += DEPTH) {
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+      step(buf[d], k + d, alive[k + d]);
+      load(buf[d], k + d + DEPTH);
+    }
   }
-  a.mode = SUB_ZERO;
-  const dim3 agrid((unsigned)(a.BH * (a.nseg_max - 1))), ablock(4 * (DK + DV));
-  if constexpr (PRO) hipLaunchKernelGGL((MABA_SUB_K(true, false, false, true, true)), agrid, ablock, 0, stream, a);
-  else if (f32in) hipLaunchKernelGGL((MABA_SUB_K(true, true, false, true, false)), agrid, ablock, 0, stream, a);
-  else if (g16) hipLaunchKernelGGL((MABA_SUB_K(true, false, true, true, false)), agrid, ablock, 0, stream, a);
-  else hipLaunchKernelGGL((MABA_SUB_K(true, false, false, true, false)), agrid, ablock, 0, stream, a);
+#pragma unroll
+  for (int d = 0; d < DEPTH; ++d) {
+    if (k + d >= kend) break;
+    step(buf[d], k + d, alive[k + d]);
+  }
+}
+
+// The launches of one prefill.  PRO: the fused-prologue inputs (bf16 projections).  f32in:
+// fp32 q, k, v; g16: 16-bit gates in q's format (only with 16-bit q, k, v); gch: every gate
+// per channel.
+template <bool PRO, int DK, int DV>
+int run_sub_passes(SubArgs& a, bool f32in, bool g16, bool gch, hipStream_t stream) {
+  constexpr int NCG = DK > 64 ? DK / 64 : 1;
+  auto launch = [&](int mode) {
+    a.mode = mode;
+    const int64_t per = (int64_t)a.BH * a.nvh;
+    const dim3 grid((unsigned)(mode == SUB_MAIN ? per * a.nseg + (int64_t)a.BH * (a.nseg - 1) * NCG : per * (a.nseg - 1)));
+#define MABA_SUB_K(F, G, C) hipLaunchKernelGGL((dgda_sub_kernel<F, G, C, PRO, DK, DV>), grid, dim3(64), 0, stream, a)
+    if constexpr (PRO) {
+      MABA_SUB_K(false, false, true);
+    } else if (f32in) {
+      if (gch) MABA_SUB_K(true, false, true);
+      else MABA_SUB_K(true, false, false);
+    } else if (g16) {
+      if (gch) MABA_SUB_K(false, true, true);
+      else MABA_SUB_K(false, true, false);
+    } else {
+      if (gch) MABA_SUB_K(false, false, true);
+      else MABA_SUB_K(false, false, false);
+    }
 #undef MABA_SUB_K
-  int rc = check_launch("dgda_prefill/sub-chunk aggregate");
-  if (rc) return rc;
-  if ((rc = launch_out(SUB_ZERO))) return rc;
-  return launch_out(SUB_FIX);
+    return check_launch("dgda_prefill/sub-chunk");
+  };
+  int rc = launch(SUB_MAIN);
+  if (rc || a.nseg == 1) return rc;
+  if (a.nseg > 2) {
+    hipLaunchKernelGGL((dgda_sub_scan_kernel<DK>), dim3((unsigned)a.BH, (unsigned)(a.dvt / 16)), dim3(64), 0, stream, a);
+    if ((rc = check_launch("dgda_prefill/sub-chunk scan"))) return rc;
+  }
+  return launch(SUB_FIX);
 }
 
 // One translation unit per d_k instantiates the kernels (dgda_sub_k32.hip, dgda_sub.hip,
-// dgda_sub_k128.hip), so that they compile in parallel; dv is 32 or 64.
-int run_sub_k32(SubArgs& a, int dv, bool f32in, bool g16, bool obf, hipStream_t stream);
-int run_sub_k64(SubArgs& a, int dv, bool f32in, bool g16, bool obf, hipStream_t stream);
-int run_sub_k128(SubArgs& a, int dv, bool f32in, bool g16, bool obf, hipStream_t stream);
+// dgda_sub_k128.hip), so that they compile in parallel; dv is 32 or 64 columns.
+int run_sub_k32(SubArgs& a, int dv, bool f32in, bool g16, bool gch, hipStream_t stream);
+int run_sub_k64(SubArgs& a, int dv, bool f32in, bool g16, bool gch, hipStream_t stream);
+int run_sub_k128(SubArgs& a, int dv, bool f32in, bool g16, bool gch, hipStream_t stream);
 
 }  // namespace maba

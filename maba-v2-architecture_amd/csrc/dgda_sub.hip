@@ -3,6 +3,8 @@
 // d_k = 64 and the fused layer prologue entry point (maba_hip_dgda_layer_prefill).
 #include "dgda_sub.h"
 
+#include <algorithm>
+
 namespace maba {
 
 // ------------------------------------------------------------------ host side
@@ -13,10 +15,12 @@ static bool fits32s(const maba_tensor* t) {
     if (t->stride[d] < 0 || t->stride[d] > INT32_MAX) return false;
   return true;
 }
+// the kernels address the 16 rows of a sub-chunk with 32-bit byte offsets
+static bool rows_fit(int64_t row_stride) { return row_stride <= (INT32_MAX - 4096) / (SC * 4); }
 // gate with channel stride 0 (per token) or 1 (per channel, 16-byte aligned rows), fp32 or
 // (16-bit q, k, v) in q's dtype
 static bool sub_gate_ok(const maba_tensor* t, int gdt) {
-  if (!t || t->dtype != gdt || !fits32s(t)) return false;
+  if (!t || t->dtype != gdt || !fits32s(t) || !rows_fit(t->stride[2])) return false;
   if (t->stride[3] == 0) return true;
   if (t->stride[3] != 1 || !al16s(t->data)) return false;
   for (int d = 0; d < 3; ++d)
@@ -35,7 +39,7 @@ bool dgda_sub_supported(const maba_tensor* q, const maba_tensor* k, const maba_t
   const int dt = q->dtype;
   if (!sub_io_dtype(dt) || k->dtype != dt || v->dtype != dt) return false;
   for (const maba_tensor* t : {q, k, v}) {   // 4-element (8- or 16-byte) loads
-    if (t->stride[3] != 1 || !al16s(t->data) || !fits32s(t)) return false;
+    if (t->stride[3] != 1 || !al16s(t->data) || !fits32s(t) || !rows_fit(t->stride[2])) return false;
     for (int d = 0; d < 3; ++d)
       if (t->shape[d] > 1 && t->stride[d] % 4 != 0) return false;
   }
@@ -48,23 +52,70 @@ bool dgda_sub_supported(const maba_tensor* q, const maba_tensor* k, const maba_t
   return q->shape[2] <= ((int64_t)1 << 30);
 }
 
-static SlotGeom sub_geom(int64_t BH, int64_t L) {
-  const int64_t nch = ceil_div(L, SC) > 0 ? ceil_div(L, SC) : 1;
-  return slot_geom(BH, nch, SUB_MIN_U);
+// ---- segments per sequence
+// Sub-chunks per segment at least.  Shorter ones no longer gain: a segment's end costs a step
+// of the scan where transitions survive (0.7 us against 3.5 us per sub-chunk twice), and where
+// they vanish it costs up to their 3 to 10 sub-chunks again.  B=1 H=10 T=2048 fp32: 87 us at
+// 16, 58 at 8, 46 at 4; slow decay at T=4096: 144, 103, 109 (6: 99).
+constexpr int64_t SUB_MIN_LEN = 5;
+// Sub-chunks per segment from which two waves per SIMD pay: the second wave gains up to 8 %
+// (B=4 H=10 T=32768 per-channel bf16: 436 us against 470), and twice as many segments cost
+// their re-runs (the fused layer at B=1 T=32768, 10 sub-chunks each: 493 us against 412).
+constexpr int64_t SUB_LEN_2 = 32;
+
+static int64_t sub_chunks(int64_t L) { return ceil_div(L, SC); }
+static int sub_groups(int64_t dv) { return dv == 128 ? 2 : 1; }   // groups of value columns, a wave each
+static size_t sub_slot_bytes(int64_t dk, int64_t dv) { return (size_t)(dk * (dv + dk)) * sizeof(float) + 2 * sizeof(int); }
+static size_t sub_bytes(int64_t BH, int64_t nseg, int64_t dk, int64_t dv) {
+  return nseg <= 1 ? 16 : (size_t)(BH * nseg) * sub_slot_bytes(dk, dv);
 }
 
-// d_v = 128 runs as two d_v = 64 calls, one after the other on the stream, which share
-// the workspace.
-static int64_t sub_dv_call(int64_t dv) { return dv == 128 ? 64 : dv; }
+// The segments a call is cut into, given the workspace's size: one wave per SIMD, or two (see
+// SUB_LEN_2; always at d_k = 32, whose waves hold a quarter of the state, never at d_k = 128,
+// whose state leaves registers for one), and no more than the workspace holds.
+static void sub_split(int64_t BH, int64_t L, int64_t dk, int64_t dv, size_t ws_bytes, int& nseg, int& seglen) {
+  const int64_t nch = sub_chunks(L);
+  const int64_t waves = BH > 0 ? BH * sub_groups(dv) : 1, simds = 4 * (int64_t)device_cu_count();
+  const bool two = dk == 32 || (dk == 64 && nch * waves >= SUB_LEN_2 * 2 * simds);
+  int64_t n = (two ? 2 : 1) * simds / waves;
+  if (n > ceil_div(nch, SUB_MIN_LEN)) n = ceil_div(nch, SUB_MIN_LEN);
+  const int64_t fit = (int64_t)(ws_bytes / ((size_t)(BH > 0 ? BH : 1) * sub_slot_bytes(dk, dv)));
+  if (n > fit) n = fit;
+  if (n > SUB_MAX_SEG) n = SUB_MAX_SEG;
+  if (n < 2) n = 1;
+  const int64_t len = nch > 0 ? ceil_div(nch, n) : 0;
+  seglen = (int)len;
+  nseg = len > 0 ? (int)ceil_div(nch, len) : 1;
+}
 
+// The size the query promises to be enough; what fits in it, sub_split works out.
 size_t dgda_sub_workspace(int64_t BH, int64_t L, int64_t dk, int64_t dv) {
-  const SlotGeom gm = sub_geom(BH, L);
+  const SlotGeom gm = slot_geom(BH, sub_chunks(L) > 0 ? sub_chunks(L) : 1, 64);
   if (gm.nseg_max <= 1) return 16;
-  const int64_t nseg = gm.nseg_max;
-  return (size_t)(BH * nseg * dk * (sub_dv_call(dv) + dk)) * sizeof(float) + (size_t)(BH * nseg) * sizeof(int);
+  const int64_t dvc = dv == 128 ? 64 : dv;
+  return (size_t)(BH * gm.nseg_max * dk * (dvc + dk)) * sizeof(float) + (size_t)(BH * gm.nseg_max) * sizeof(int);
 }
 
-static int64_t esz(int dt) { return dt == MABA_F32 ? 4 : 2; }
+// The size with which a call is cut as finely as pays.
+size_t dgda_sub_workspace_preferred(int64_t BH, int64_t L, int64_t dk, int64_t dv) {
+  int nseg, len;
+  sub_split(BH, L, dk, dv, SIZE_MAX, nseg, len);
+  return sub_bytes(BH, nseg, dk, dv);
+}
+
+static void sub_place(SubArgs& a, int64_t BH, int64_t L, int64_t dk, int64_t dv, void* ws, size_t ws_bytes) {
+  sub_split(BH, L, dk, dv, ws_bytes, a.nseg, a.seglen);
+  a.nchunks = (int)sub_chunks(L);
+  a.nvh = sub_groups(dv);
+  a.dvt = (int)dv;
+  a.agg = (float*)ws;
+  a.zc = (int*)(a.agg + BH * a.nseg * dk * (dv + dk));
+}
+
+// One vector store per lane and token: aligned rows.
+static int sub_out_vec(const maba_tensor* out) {
+  return al16s(out->data) && out->stride[0] % 4 == 0 && out->stride[1] % 4 == 0 && out->stride[2] % 4 == 0;
+}
 
 int launch_dgda_sub(const maba_tensor* q, const maba_tensor* k, const maba_tensor* v,
                     const maba_tensor* gate, int use_log, const maba_tensor* b,
@@ -84,46 +135,26 @@ int launch_dgda_sub(const maba_tensor* q, const maba_tensor* k, const maba_tenso
   a.wp = w->data; a.ws0 = (int)w->stride[0]; a.ws1 = (int)w->stride[1];
   a.ws2 = (int)w->stride[2]; a.ws3 = (int)w->stride[3];
   a.s0 = view4(s0);
-  a.op = out->data; a.os0 = (int)out->stride[0]; a.os1 = (int)out->stride[1]; a.os2 = (int)out->stride[2];
+  a.op = out->data; a.odt = out->dtype;
+  a.os0 = (int)out->stride[0]; a.os1 = (int)out->stride[1]; a.os2 = (int)out->stride[2];
+  a.ovec = sub_out_vec(out);
   a.sf = mview4(sf);
   a.H = (int)H; a.L = (int)L; a.BH = (int)BH;
-  a.nchunks = (int)(ceil_div(L, SC) > 0 ? ceil_div(L, SC) : 1);
-  const SlotGeom gm = sub_geom(BH, L);
-  a.U = gm.U;
-  a.nseg_max = gm.nseg_max;
   a.use_log = use_log; a.has_s0 = s0 != nullptr;
-  a.f16 = q->dtype == MABA_F16; a.of16 = out->dtype == MABA_F16;
-  const size_t need = dgda_sub_workspace(BH, L, dk, dv);
-  if (ws_bytes < need) return fail(MABA_ERR_WORKSPACE, "dgda_prefill: workspace too small");
-  const int64_t nsegs = BH * a.nseg_max, dvc = sub_dv_call(dv);
-  a.agg = (float*)ws;
-  a.zc = (int*)(a.agg + nsegs * dk * (dvc + dk));
-  const bool f32in = q->dtype == MABA_F32, g16 = gate->dtype != MABA_F32, o16 = out->dtype != MABA_F32;
-  auto run = [&](SubArgs& x) {
-    if (dk == 32) return run_sub_k32(x, (int)dvc, f32in, g16, o16, stream);
-    if (dk == 64) return run_sub_k64(x, (int)dvc, f32in, g16, o16, stream);
-    return run_sub_k128(x, (int)dvc, f32in, g16, o16, stream);
-  };
-  if (dv != 128) return run(a);
-  // the two halves of the value columns: v, w, the output and the states start 64
-  // columns further in the second call
-  for (int half = 0; half < 2; ++half) {
-    SubArgs h = a;
-    const int64_t c = 64 * half;
-    h.vp = (const char*)v->data + c * esz(v->dtype);
-    h.wp = (const char*)w->data + c * w->stride[3] * esz(w->dtype);
-    h.op = (char*)out->data + c * esz(out->dtype);
-    if (s0) h.s0.p = (const char*)s0->data + c * s0->stride[3] * esz(s0->dtype);
-    h.sf.p = (char*)sf->data + c * sf->stride[3] * esz(sf->dtype);
-    const int rc = run(h);
-    if (rc) return rc;
-  }
-  return MABA_OK;
+  a.f16 = q->dtype == MABA_F16;
+  if (ws_bytes < dgda_sub_workspace(BH, L, dk, dv)) return fail(MABA_ERR_WORKSPACE, "dgda_prefill: workspace too small");
+  sub_place(a, BH, L, dk, dv, ws, ws_bytes);
+  const bool f32in = q->dtype == MABA_F32, g16 = gate->dtype != MABA_F32;
+  const bool gch = a.gs3 == 1 && a.bs3 == 1 && a.ws3 == 1;
+  const int dvc = dv == 128 ? 64 : (int)dv;
+  if (dk == 32) return run_sub_k32(a, dvc, f32in, g16, gch, stream);
+  if (dk == 64) return run_sub_k64(a, dvc, f32in, g16, gch, stream);
+  return run_sub_k128(a, dvc, f32in, g16, gch, stream);
 }
 
-int run_sub_k64(SubArgs& a, int dv, bool f32in, bool g16, bool obf, hipStream_t stream) {
-  return dv == 32 ? run_sub_passes<false, 64, 32>(a, f32in, g16, obf, stream)
-                  : run_sub_passes<false, 64, 64>(a, f32in, g16, obf, stream);
+int run_sub_k64(SubArgs& a, int dv, bool f32in, bool g16, bool gch, hipStream_t stream) {
+  return dv == 32 ? run_sub_passes<false, 64, 32>(a, f32in, g16, gch, stream)
+                  : run_sub_passes<false, 64, 64>(a, f32in, g16, gch, stream);
 }
 
 }  // namespace maba
@@ -131,7 +162,7 @@ int run_sub_k64(SubArgs& a, int dv, bool f32in, bool g16, bool obf, hipStream_t 
 using namespace maba;
 
 extern "C" size_t maba_hip_dgda_layer_prefill_workspace_size(int64_t B, int64_t H, int64_t L) {
-  return dgda_sub_workspace(B * H, L, 64, 64);
+  return std::max(dgda_sub_workspace(B * H, L, 64, 64), dgda_sub_workspace_preferred(B * H, L, 64, 64));
 }
 
 extern "C" int maba_hip_dgda_layer_prefill(const maba_tensor* const* xs, const maba_tensor* const* conv_w,
@@ -196,20 +227,18 @@ extern "C" int maba_hip_dgda_layer_prefill(const maba_tensor* const* xs, const m
   }
   a.eps = eps;
   a.s0 = view4(initial_state);
-  a.op = out->data; a.os0 = (int)out->stride[0]; a.os1 = (int)out->stride[1]; a.os2 = (int)out->stride[2];
+  for (int s = 0; s < 3; ++s) {
+    a.nh[s] = new_hist[s]->data; a.nhdt[s] = new_hist[s]->dtype;
+    a.nhs0[s] = new_hist[s]->stride[0]; a.nhs1[s] = new_hist[s]->stride[1]; a.nhs2[s] = new_hist[s]->stride[2];
+  }
+  a.op = out->data; a.odt = out->dtype;
+  a.os0 = (int)out->stride[0]; a.os1 = (int)out->stride[1]; a.os2 = (int)out->stride[2];
+  a.ovec = sub_out_vec(out);
   a.sf = mview4(final_state);
   a.H = (int)H; a.L = (int)L; a.BH = (int)BH;
-  a.nchunks = (int)ceil_div(L, SC);
-  const SlotGeom gm = sub_geom(BH, L);
-  a.U = gm.U;
-  a.nseg_max = gm.nseg_max;
   a.use_log = 1; a.has_s0 = initial_state != nullptr;
-  const int64_t nsegs = BH * a.nseg_max;
-  a.agg = (float*)workspace;
-  a.zc = (int*)(a.agg + nsegs * 64 * 128);
-  hipStream_t st = (hipStream_t)stream;
-  const int rc = run_sub_passes<true, 64, 64>(a, false, false, out->dtype == MABA_BF16, st);
-  if (rc) return rc;
-  // after the passes, which read the old history: the new one may overwrite it in place
-  return launch_dgda_new_history(xs, hist, new_hist, st);
+  sub_place(a, BH, L, 64, 64, workspace, workspace_bytes);
+  // the new history is written by the last launch, after the first one has read the old: it
+  // may overwrite it in place
+  return run_sub_passes<true, 64, 64>(a, false, false, true, (hipStream_t)stream);
 }

@@ -3,9 +3,9 @@
 
 namespace maba {
 
-int run_sub_k128(SubArgs& a, int dv, bool f32in, bool g16, bool obf, hipStream_t stream) {
-  return dv == 32 ? run_sub_passes<false, 128, 32>(a, f32in, g16, obf, stream)
-                  : run_sub_passes<false, 128, 64>(a, f32in, g16, obf, stream);
+int run_sub_k128(SubArgs& a, int dv, bool f32in, bool g16, bool gch, hipStream_t stream) {
+  return dv == 32 ? run_sub_passes<false, 128, 32>(a, f32in, g16, gch, stream)
+                  : run_sub_passes<false, 128, 64>(a, f32in, g16, gch, stream);
 }
 
 }  // namespace maba

@@ -36,6 +36,7 @@ EXPORTED_SYMBOLS = (
     "maba_hip_last_error",
     "maba_hip_abi_version",
     "maba_hip_dgda_prefill_workspace_size",
+    "maba_hip_dgda_prefill_workspace_preferred",
     "maba_hip_dgda_prefill",
     "maba_hip_dgda_step",
     "maba_hip_compute_centroids",
@@ -92,6 +93,7 @@ def _declare(lib) -> None:
         "maba_hip_last_error": ([], ctypes.c_char_p),
         "maba_hip_abi_version": ([], i),
         "maba_hip_dgda_prefill_workspace_size": ([T, T, T, T], sz),
+        "maba_hip_dgda_prefill_workspace_preferred": ([T, T, T, T], sz),
         "maba_hip_dgda_prefill": ([T, T, T, T, T, T, T, T, T, T, i, vp, sz, vp], i),
         "maba_hip_dgda_step": ([T, T, T, T, T, T, T, T, T, T, vp], i),
         "maba_hip_compute_centroids": ([T, T, i, vp], i),

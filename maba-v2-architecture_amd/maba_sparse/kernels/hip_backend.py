@@ -72,7 +72,7 @@ def hip_dgda_prefill(q, k, v, alpha=None, b=None, w=None, chunk_size: int = 16, 
     ds0 = N.desc(initial_state)
     dout, dst = N.desc(out), N.desc(state)
     gate = dla if log_alpha is not None else da
-    nbytes = lib.maba_hip_dgda_prefill_workspace_size(dq, dvv, gate, db)
+    nbytes = lib.maba_hip_dgda_prefill_workspace_preferred(dq, dvv, gate, db)
     ws = _workspace(nbytes, dev)
     rc = lib.maba_hip_dgda_prefill(dq, dk_, dvv, da, dla, db, dw, ds0, dout, dst, int(chunk_size),
                                    ws.data_ptr(), ws.numel(), N.stream_ptr(dev))

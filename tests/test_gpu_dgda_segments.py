@@ -1,0 +1,114 @@
+"""How the sub-chunk DGDA prefill cuts a sequence: segments as the workspace allows, in-place
+buffers across the launches, and sub-chunks on both sides of the decay range its matrix products
+take.  Tolerances as in test_gpu_dgda_prefill.py: rtol = atol = 2e-3 against the float64
+recurrence; where only the cut differs, the last bits of fp32 sums of products split to 16
+mantissa bits (observed 1e-5)."""
+import numpy as np
+import pytest
+import torch
+
+from _helpers import assert_close, dgda_inputs, oracle_dgda_args, to_np
+from oracle import dgda as odgda
+
+pytestmark = pytest.mark.gpu
+
+
+def _call(inp, nbytes, s0=None, sf=None):
+    """maba_hip_dgda_prefill with a workspace of ``nbytes``."""
+    from maba_sparse import _native as N
+    lib = N.load()
+    q, v = inp["q"], inp["v"]
+    B, H, L, dk = q.shape
+    dv = v.shape[3]
+    out = torch.empty(B, H, L, dv, device=q.device)
+    sf = torch.empty(B, H, dk, dv, device=q.device) if sf is None else sf
+    ws = torch.full((max(int(nbytes), 16),), 0xff, dtype=torch.uint8, device=q.device)   # NaN patterns
+    rc = lib.maba_hip_dgda_prefill(N.desc(q), N.desc(inp["k"]), N.desc(v), None, N.desc(inp["log_alpha"]),
+                                   N.desc(inp["b"]), N.desc(inp["w"]), N.desc(s0), N.desc(out), N.desc(sf), 16,
+                                   ws.data_ptr(), int(nbytes), N.stream_ptr(q.device))
+    N.check(rc, "dgda_prefill")
+    return out, sf
+
+
+def _sizes(inp):
+    from maba_sparse import _native as N
+    lib = N.load()
+    d = [N.desc(inp[n]) for n in ("q", "v", "log_alpha", "b")]
+    return lib.maba_hip_dgda_prefill_workspace_size(*d), lib.maba_hip_dgda_prefill_workspace_preferred(*d)
+
+
+@pytest.mark.parametrize("dk,dv", [(64, 64), (32, 32), (128, 128)])
+@pytest.mark.parametrize("decay", ["baseline", "slow"])
+def test_segments_follow_the_workspace(dev, dk, dv, decay):
+    """The least workspace, the preferred one and two between give the recurrence's result."""
+    inp = dgda_inputs(1, 2, 1300, dk=dk, dv=dv, seed=3, decay=decay, gates="channel", device=dev, with_state=True)
+    eo, eS = odgda.dgda_prefill_seq(**oracle_dgda_args(inp))
+    least, best = _sizes(inp)
+    assert 16 < least < best
+    for nbytes in (least, (least + best) // 2, best - 1, best):
+        o, S = _call(inp, nbytes, s0=inp["initial_state"])
+        assert_close(o, eo, 2e-3, 2e-3, f"out {nbytes}")
+        assert_close(S, eS, 2e-3, 2e-3, f"state {nbytes}")
+
+
+@pytest.mark.parametrize("decay", ["baseline", "slow"])
+def test_state_in_place_across_segments(dev, decay):
+    inp = dgda_inputs(2, 3, 900, seed=5, decay=decay, gates="channel", device=dev, with_state=True)
+    _, best = _sizes(inp)
+    o, S = _call(inp, best, s0=inp["initial_state"])
+    buf = inp["initial_state"].clone()
+    o2, S2 = _call(inp, best, s0=buf, sf=buf)
+    assert torch.equal(o, o2) and torch.equal(S, S2)
+
+
+@pytest.mark.parametrize("L", [1, 2, 3, 17, 700])
+def test_layer_history_in_place(dev, L):
+    """The new conv history over the old one's buffers, one segment and several."""
+    from maba_sparse.kernels import hip_backend as hb
+    g = torch.Generator().manual_seed(L)
+    rn = lambda *s: torch.randn(*s, generator=g).bfloat16().to(dev)  # noqa: E731
+    projs, convs = rn(2, L, 6 * 128).split(128, dim=-1), [rn(128, 1, 4) for _ in range(3)]
+    hist = [rn(2, 128, 3) for _ in range(3)]
+    o, S, new = hb.hip_dgda_layer_prefill(projs, convs, hist)
+    for s in range(3):
+        want = torch.cat([hist[s].transpose(1, 2), projs[s]], dim=1)[:, -3:].transpose(1, 2)
+        assert torch.equal(new[s], want)
+    buf = [h.clone() for h in hist]
+    o2, S2, new2 = hb.hip_dgda_layer_prefill(projs, convs, buf, out_history=buf)
+    assert torch.equal(o, o2) and torch.equal(S, S2) and all(torch.equal(a, b) for a, b in zip(new, new2))
+
+
+@pytest.mark.parametrize("per_token", [-3.999, -4.001, -8.0, -30.0, -200.0, 3.999, 4.001])
+@pytest.mark.parametrize("dk", [32, 64, 128])
+def test_decay_range_of_the_products(dev, per_token, dk):
+    """One channel in four decays by ``per_token`` at every token, so a sub-chunk's range is sixteen
+    times that: 64 is where the products end and the pairwise sums begin.  Growth is kept to one
+    sub-chunk with a written state of order one."""
+    L = 16 if per_token > 0 else 70
+    inp = dgda_inputs(1, 2, L, dk=dk, dv=64, seed=9, decay="slow", gates="channel", qkv_dtype=torch.float32, device=dev)
+    la = inp["log_alpha"].clone()
+    la[..., ::4] = per_token
+    inp["log_alpha"] = la
+    eo, eS = odgda.dgda_prefill_seq(**oracle_dgda_args(inp))
+    o, S = _call(inp, _sizes(inp)[1])
+    for a, e in ((o, eo), (S, eS)):   # relative to the largest value: growth reaches e^64
+        scale = max(1.0, float(np.abs(e).max()))
+        assert_close(a / scale, e / scale, 2e-3, 2e-3, f"{per_token}")
+
+
+def test_layer_strong_decay_gates(dev):
+    """Decay projections far up: every sub-chunk of the fused layer leaves the products' range, its
+    decays at the e^-14 floor."""
+    from maba_sparse.kernels import hip_backend as hb
+    g = torch.Generator().manual_seed(2)
+    rn = lambda *s: torch.randn(*s, generator=g).bfloat16()  # noqa: E731
+    x = list(rn(1, 300, 6 * 64).split(64, dim=-1))
+    x[3] = (x[3].float() * 40).bfloat16()
+    convs = [rn(64, 1, 4) for _ in range(3)]
+    o, S, _ = hb.hip_dgda_layer_prefill([t.to(dev).contiguous() for t in x], [w.to(dev) for w in convs],
+                                        state_dtype=torch.float32)
+    f = lambda t: t.double().numpy()  # noqa: E731
+    q, k, v, la, _, b, w, _ = odgda.layer_prologue(*[f(t) for t in x], *[f(c[:, 0]) for c in convs], n_heads=1)
+    eo, eS = odgda.dgda_prefill_seq(*(t[:, None] for t in (q, k, v)), alpha=np.exp(la)[:, None], b=b[:, None], w=w[:, None])
+    assert_close(o.float().view(1, 300, 1, 64).transpose(1, 2), eo, 1e-2, 1e-2, "out")   # bf16 output
+    assert_close(S, eS, 2e-3, 2e-3, "state")

@@ -118,6 +118,26 @@ __device__ __forceinline__ float wave_incl_scan(float x) {
   return x;
 }
 
+// Exchanges a's upper 32 lanes with b's lower 32 (swap32), a's odd 16-lane rows with b's
+// even ones (swap16).
+__device__ __forceinline__ void swap32(uint32_t& a, uint32_t& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  a = r[0]; b = r[1];
+}
+__device__ __forceinline__ void swap16(uint32_t& a, uint32_t& b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+  a = r[0]; b = r[1];
+}
+// Largest over the four lane groups, in every lane.
+__device__ __forceinline__ float group_max(float x) {
+  uint32_t a = __float_as_uint(x), b = a;
+  swap32(a, b);
+  const float s = fmaxf(__uint_as_float(a), __uint_as_float(b));
+  a = b = __float_as_uint(s);
+  swap16(a, b);
+  return fmaxf(__uint_as_float(a), __uint_as_float(b));
+}
+
 // LDS-only barrier: waits for this wave's LDS operations, not for its outstanding
 // global loads (the next chunk's prefetch stays in flight across it).
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }

@@ -29,7 +29,7 @@
 // is VALU issue: per sub-chunk at d_k = d_v = 64 about 1,100 VALU instructions (fused layer
 // 1,700, 200 of them transcendental) beside 100 MFMAs, so that one wave per SIMD takes 3.5 us
 // (6.5 us) and two take hardly less time each.  Before and after, whole calls: B=4 H=10
-// T=8192 d=128 fp16 1,377 -> 525 us; B=1 H=10 T=2048 fp32 212 -> 51 us; the fused layer's
+// T=8192 d=128 fp16 1,377 -> 403 us; B=1 H=10 T=2048 fp32 212 -> 51 us; the fused layer's
 // launches at B=4 T=32768 1,150 -> 680 us, at B=1 T=1000 310 -> 100 us.
 //
 // Layouts.  NKT = d_k / 16, NCT = columns / 16.  Lane (c = lane & 15, g = lane >> 4):
@@ -132,14 +132,12 @@ __device__ __forceinline__ Row<F32, N> load_row(const char* p) {
   }
   return r;
 }
-template <bool F32, int N>
-__device__ __forceinline__ float row_at(const Row<F32, N>& r, int j, bool f16) {
+// Element j; 16-bit ones are fp16 (F16) or bf16.
+template <bool F16, bool F32, int N>
+__device__ __forceinline__ float row_at(const Row<F32, N>& r, int j) {
   if constexpr (F32) return __uint_as_float(r.w[j]);
-  else {
-    const uint32_t h = (j & 1) ? r.w[j / 2] >> 16 : r.w[j / 2] & 0xffffu;
-    if (f16) return __half2float(__ushort_as_half((unsigned short)h));
-    return __uint_as_float((j & 1) ? r.w[j / 2] & 0xffff0000u : r.w[j / 2] << 16);
-  }
+  else if constexpr (F16) return __half2float(__ushort_as_half((unsigned short)(r.w[j / 2] >> (16 * (j & 1)))));
+  else return __uint_as_float((j & 1) ? r.w[j / 2] & 0xffff0000u : r.w[j / 2] << 16);
 }
 // N gate values of one token at channel stride cs (0 or 1), p at the first, as raw elements.
 template <bool G16, bool GCH, int N>
@@ -162,16 +160,6 @@ __device__ __forceinline__ Row<!G16, N> load_gate(const char* p, int cs) {
 
 // ------------------------------------------------------------------ lane-group moves
 
-// Exchanges a's upper 32 lanes with b's lower 32 (swap32), a's odd 16-lane rows with b's
-// even ones (swap16).
-__device__ __forceinline__ void swap32(uint32_t& a, uint32_t& b) {
-  const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
-  a = r[0]; b = r[1];
-}
-__device__ __forceinline__ void swap16(uint32_t& a, uint32_t& b) {
-  const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
-  a = r[0]; b = r[1];
-}
 // x[t] of lane group g  <->  x[g] of lane group t (4 x 4 transpose; its own inverse).
 __device__ __forceinline__ void transpose4(uint32_t (&x)[4]) {
   swap32(x[0], x[2]);
@@ -338,7 +326,7 @@ __device__ __forceinline__ int sub_run(const SubArgs& a, SubSmem<PRO, DK>& sm, i
     for (int e = 0; e < 4; ++e) {
       float x[7];
 #pragma unroll
-      for (int m = 0; m < 7; ++m) x[m] = row_at<false, 4>(t[m], e, false);
+      for (int m = 0; m < 7; ++m) x[m] = row_at<false>(t[m], e);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         float acc = w[3][e] * x[i + 3];
@@ -406,8 +394,8 @@ __device__ __forceinline__ int sub_run(const SubArgs& a, SubSmem<PRO, DK>& sm, i
         for (int j = 0; j < NKT; ++j) {
           kk[i][j] *= inv;
           // the decay e^max(-softplus(x), -14) = max(1 / (1 + e^x), e^-14)
-          la[i][j] = fmaxf(fast_rcp(1.f + fast_exp(row_at<false, 4>(xg[0][i], j, false))), DECAY_MIN);
-          be[i][j] = pro_sigmoid(row_at<false, 4>(xg[1][i], j, false));
+          la[i][j] = fmaxf(fast_rcp(1.f + fast_exp(row_at<false>(xg[0][i], j))), DECAY_MIN);
+          be[i][j] = pro_sigmoid(row_at<false>(xg[1][i], j));
         }
       }
       if (!MAP) {
@@ -416,26 +404,34 @@ __device__ __forceinline__ int sub_run(const SubArgs& a, SubSmem<PRO, DK>& sm, i
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
-          for (int j = 0; j < NVT; ++j) ve[j][i] = pro_sigmoid(row_at<false, 4>(xg[2][i], j, false)) * vv[i][j];
+          for (int j = 0; j < NVT; ++j) ve[j][i] = pro_sigmoid(row_at<false>(xg[2][i], j)) * vv[i][j];
         conv(0, tq, qq);
       }
     } else {
-      const bool f16 = a.f16 != 0;
+      auto convert = [&](auto f16_c) {
+        constexpr bool F16 = decltype(f16_c)::value;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < 4; ++i) {
 #pragma unroll
-        for (int j = 0; j < NKT; ++j) {
-          kk[i][j] = row_at(pk[i], j, f16);
-          be[i][j] = row_at(pb[i], j, f16);
-          const float x = row_at(pg[i], j, f16);
-          la[i][j] = a.use_log ? x * LOG2E : __builtin_amdgcn_logf(fmaxf(x, 1e-20f));
-          if (!MAP) qq[i][j] = row_at(pq[i], j, f16);
+          for (int j = 0; j < NKT; ++j) {
+            kk[i][j] = row_at<F16>(pk[i], j);
+            be[i][j] = row_at<F16>(pb[i], j);
+            la[i][j] = row_at<F16>(pg[i], j);
+            if (!MAP) qq[i][j] = row_at<F16>(pq[i], j);
+          }
+          if (!MAP) {
+#pragma unroll
+            for (int j = 0; j < NVT; ++j) ve[j][i] = row_at<F16>(pw[i], j) * row_at<F16>(pv[i], j);
+          }
         }
-        if (!MAP) {
+      };
+      if (!F32IN && a.f16) convert(std::true_type{});   // one branch, not one per element
+      else convert(std::false_type{});
 #pragma unroll
-          for (int j = 0; j < NVT; ++j) ve[j][i] = row_at(pw[i], j, f16) * row_at(pv[i], j, f16);
-        }
-      }
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < NKT; ++j)
+          la[i][j] = a.use_log ? la[i][j] * LOG2E : __builtin_amdgcn_logf(fmaxf(la[i][j], 1e-20f));
     }
     if (MAP) {
 #pragma unroll

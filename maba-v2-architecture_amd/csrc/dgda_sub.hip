@@ -64,31 +64,38 @@ constexpr int64_t SUB_MIN_LEN = 5;
 constexpr int64_t SUB_LEN_2 = 32;
 
 static int64_t sub_chunks(int64_t L) { return ceil_div(L, SC); }
-static int sub_groups(int64_t dv) { return dv == 128 ? 2 : 1; }   // groups of value columns, a wave each
 static size_t sub_slot_bytes(int64_t dk, int64_t dv) { return (size_t)(dk * (dv + dk)) * sizeof(float) + 2 * sizeof(int); }
-static size_t sub_bytes(int64_t BH, int64_t nseg, int64_t dk, int64_t dv) {
-  return nseg <= 1 ? 16 : (size_t)(BH * nseg) * sub_slot_bytes(dk, dv);
-}
 
-// The segments a call is cut into, given the workspace's size: one wave per SIMD, or two (see
-// SUB_LEN_2; always at d_k = 32, whose waves hold a quarter of the state, never at d_k = 128,
-// whose state leaves registers for one), and no more than the workspace holds.
-static void sub_split(int64_t BH, int64_t L, int64_t dk, int64_t dv, size_t ws_bytes, int& nseg, int& seglen) {
+// How a call is cut: nseg segments of seglen sub-chunks, cols value columns per wave.
+struct SubCut { int nseg, seglen, cols; };
+
+// As many segments as fill one wave per SIMD, or two (see SUB_LEN_2; always at d_k = 32, whose
+// waves hold a quarter of the state, never at d_k = 128, whose state leaves registers for one),
+// and no more than the workspace holds.  Where that leaves half the SIMDs without work a wave
+// takes 32 columns instead of 64 (narrow; not in the fused layer, whose staging is most of a
+// sub-chunk): the key side is done twice, but a sub-chunk takes a wave less time (B=2 H=10
+// bf16: T=160 54 -> 37 us, T=1000 57 -> 48 us).
+static SubCut sub_cut(int64_t BH, int64_t L, int64_t dk, int64_t dv, size_t ws_bytes, bool narrow) {
   const int64_t nch = sub_chunks(L);
-  const int64_t waves = BH > 0 ? BH * sub_groups(dv) : 1, simds = 4 * (int64_t)device_cu_count();
+  const int64_t simds = 4 * (int64_t)device_cu_count();
+  const int64_t waves = (BH > 0 ? BH : 1) * (dv == 128 ? 2 : 1);
   const bool two = dk == 32 || (dk == 64 && nch * waves >= SUB_LEN_2 * 2 * simds);
   int64_t n = (two ? 2 : 1) * simds / waves;
   if (n > ceil_div(nch, SUB_MIN_LEN)) n = ceil_div(nch, SUB_MIN_LEN);
   const int64_t fit = (int64_t)(ws_bytes / ((size_t)(BH > 0 ? BH : 1) * sub_slot_bytes(dk, dv)));
   if (n > fit) n = fit;
   if (n > SUB_MAX_SEG) n = SUB_MAX_SEG;
-  if (n < 2) n = 1;
+  // two short segments take no less time one after the other (the second's re-run) than one
+  if (n < 2 || (n == 2 && nch < 4 * SUB_MIN_LEN)) n = 1;
   const int64_t len = nch > 0 ? ceil_div(nch, n) : 0;
-  seglen = (int)len;
-  nseg = len > 0 ? (int)ceil_div(nch, len) : 1;
+  SubCut c;
+  c.seglen = (int)len;
+  c.nseg = len > 0 ? (int)ceil_div(nch, len) : 1;
+  c.cols = dv == 32 || (narrow && 2 * waves * c.nseg <= simds) ? 32 : 64;
+  return c;
 }
 
-// The size the query promises to be enough; what fits in it, sub_split works out.
+// The size the query promises to be enough; what fits in it, sub_cut works out.
 size_t dgda_sub_workspace(int64_t BH, int64_t L, int64_t dk, int64_t dv) {
   const SlotGeom gm = slot_geom(BH, sub_chunks(L) > 0 ? sub_chunks(L) : 1, 64);
   if (gm.nseg_max <= 1) return 16;
@@ -98,18 +105,21 @@ size_t dgda_sub_workspace(int64_t BH, int64_t L, int64_t dk, int64_t dv) {
 
 // The size with which a call is cut as finely as pays.
 size_t dgda_sub_workspace_preferred(int64_t BH, int64_t L, int64_t dk, int64_t dv) {
-  int nseg, len;
-  sub_split(BH, L, dk, dv, SIZE_MAX, nseg, len);
-  return sub_bytes(BH, nseg, dk, dv);
+  const SubCut c = sub_cut(BH, L, dk, dv, SIZE_MAX, true);
+  return c.nseg == 1 ? 16 : (size_t)(BH * c.nseg) * sub_slot_bytes(dk, dv);
 }
 
-static void sub_place(SubArgs& a, int64_t BH, int64_t L, int64_t dk, int64_t dv, void* ws, size_t ws_bytes) {
-  sub_split(BH, L, dk, dv, ws_bytes, a.nseg, a.seglen);
+// Returns the columns per wave.
+static int sub_place(SubArgs& a, int64_t BH, int64_t L, int64_t dk, int64_t dv, void* ws, size_t ws_bytes, bool narrow) {
+  const SubCut c = sub_cut(BH, L, dk, dv, ws_bytes, narrow);
+  a.nseg = c.nseg;
+  a.seglen = c.seglen;
   a.nchunks = (int)sub_chunks(L);
-  a.nvh = sub_groups(dv);
+  a.nvh = (int)(dv / c.cols);
   a.dvt = (int)dv;
   a.agg = (float*)ws;
   a.zc = (int*)(a.agg + BH * a.nseg * dk * (dv + dk));
+  return c.cols;
 }
 
 // One vector store per lane and token: aligned rows.
@@ -143,13 +153,12 @@ int launch_dgda_sub(const maba_tensor* q, const maba_tensor* k, const maba_tenso
   a.use_log = use_log; a.has_s0 = s0 != nullptr;
   a.f16 = q->dtype == MABA_F16;
   if (ws_bytes < dgda_sub_workspace(BH, L, dk, dv)) return fail(MABA_ERR_WORKSPACE, "dgda_prefill: workspace too small");
-  sub_place(a, BH, L, dk, dv, ws, ws_bytes);
+  const int cols = sub_place(a, BH, L, dk, dv, ws, ws_bytes, true);
   const bool f32in = q->dtype == MABA_F32, g16 = gate->dtype != MABA_F32;
   const bool gch = a.gs3 == 1 && a.bs3 == 1 && a.ws3 == 1;
-  const int dvc = dv == 128 ? 64 : (int)dv;
-  if (dk == 32) return run_sub_k32(a, dvc, f32in, g16, gch, stream);
-  if (dk == 64) return run_sub_k64(a, dvc, f32in, g16, gch, stream);
-  return run_sub_k128(a, dvc, f32in, g16, gch, stream);
+  if (dk == 32) return run_sub_k32(a, cols, f32in, g16, gch, stream);
+  if (dk == 64) return run_sub_k64(a, cols, f32in, g16, gch, stream);
+  return run_sub_k128(a, cols, f32in, g16, gch, stream);
 }
 
 int run_sub_k64(SubArgs& a, int dv, bool f32in, bool g16, bool gch, hipStream_t stream) {
@@ -237,7 +246,7 @@ extern "C" int maba_hip_dgda_layer_prefill(const maba_tensor* const* xs, const m
   a.sf = mview4(final_state);
   a.H = (int)H; a.L = (int)L; a.BH = (int)BH;
   a.use_log = 1; a.has_s0 = initial_state != nullptr;
-  sub_place(a, BH, L, 64, 64, workspace, workspace_bytes);
+  sub_place(a, BH, L, 64, 64, workspace, workspace_bytes, false);
   // the new history is written by the last launch, after the first one has read the old: it
   // may overwrite it in place
   return run_sub_passes<true, 64, 64>(a, false, false, true, (hipStream_t)stream);

@@ -23,6 +23,27 @@
 //                                        tile, B: the probabilities in bf16 hi + lo)
 // with an online softmax per query and stream; each sparse key is weighted by how often the
 // lane's query lists its block.  A wave skips the tiles none of its queries weights.
+//
+// The kernel is bound by VALU issue, not by its products (a tile's 24 MFMAs are 384 cycles of
+// the matrix unit), so the softmax is kept to one FMA, one maximum, one exp2, one addition and
+// the hi/lo split per score:
+//  * the running reference m of a query moves only when a score passes it by 2^8 (the sums
+//    hold that easily in fp32); only then do lanes exchange maxima and the sums rescale;
+//  * a key's weight is folded into the exponent as its log2, so an unlisted block is a bias of
+//    -inf and a block listed once costs nothing;
+//  * the probabilities' sum is a product with a row of ones, on the matrix unit;
+//  * which union entries a query lists is a row of bits in LDS, one word per 32 entries, in
+//    place of comparing the entry with all of the query's slots (which remains for unions
+//    beyond PF_QWORDS words and for queries that list a block twice);
+//  * a tile inside every query's range skips the row masks, and the staging addresses are a
+//    uniform base and a 32-bit lane offset.
+// Measured at B=1 H=10 dh=64 T=32768, top-32 (start of each pair: a maximum and a rescale per
+// tile, counted slots, 64-bit addresses, padded rows): random queries, 5.1 K distinct blocks
+// per 16 of them, 3.82 -> 2.63 ms; neighbouring queries alike 1.13 -> 0.82 ms.  VALU
+// instructions per call 1,234 M -> 700 M, a quarter of the SIMDs' cycles MFMA.  Tiles loaded
+// straight to LDS three ahead, with 64 or 128 queries per workgroup, measured the same on
+// random queries and 12 to 20 % slower on alike ones (two workgroups per CU instead of three):
+// issue bounds it, not latency.
 #include <algorithm>
 
 #include "dgda_common.h"
@@ -32,6 +53,8 @@ namespace maba {
 constexpr int PF_MAXK = 64;          // index slots per query
 constexpr int PF_WORDS = 512;        // bitmap words per workgroup: blocks below 16384
 constexpr int PF_LIST = 64 * PF_MAXK;   // the union of a workgroup's 64 queries' slots
+constexpr int PF_QWORDS = 16;        // words of a query's row of union bits (512 entries)
+constexpr float PF_SLACK = 8.f;      // a score may pass the running reference by 2^8
 
 typedef __attribute__((ext_vector_type(8))) short pf16x8;
 typedef __attribute__((ext_vector_type(4))) short pf16x4;
@@ -51,13 +74,15 @@ struct PfArgs {
   float scale;
 };
 
-// Transposed LDS read: lane j of 16-lane group g addressing row r0 + 4g + j/4, column
-// c0 + 4(j%4) of a row-major tile receives the column fragment tile[r0 + 4g + r][c0 + j],
-// r = 0..3.
-__device__ __forceinline__ pf16x4 pf_ldsT4(const short* tile, int pitch, int r0, int c0, int c16, int g) {
-  const short* p = tile + (r0 + 4 * g + (c16 >> 2)) * pitch + c0 + 4 * (c16 & 3);
-  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) pf16x4*)p);
-}
+// LDS tiles: rows of dh without padding, the 16-byte chunks of row r exchanged so that neither
+// the staging writes, nor a b128 read of one chunk of 16 consecutive rows (keys), nor a
+// transposed b64 read of two chunks of 8 consecutive rows (values) meets a bank twice: NP rows
+// of 64 banks hold 4 NP chunks; keys xor the chunk with r / (4 / NP), values with twice that.
+// (With rows padded by 8 elements the conflicts were a quarter of the LDS's time.)
+template <int NP>
+__device__ __forceinline__ constexpr int pf_kswz(int r) { return (r / (4 / NP)) & (4 * NP - 1); }
+template <int NP>
+__device__ __forceinline__ constexpr int pf_vswz(int r) { return 2 * ((r / (4 / NP)) & (2 * NP - 1)); }
 
 // Bits 4 rb + i of the lane's 16 tile rows j = 16 rb + 4 g + i that lie in [lo, hi]
 // (tile-relative, either bound may fall outside [0, 63]).
@@ -70,19 +95,23 @@ __device__ __forceinline__ uint32_t pf_range_bits(int lo, int hi, int g) {
          (((m1 >> (16 + sh)) & 0xfu) << 12);
 }
 
-// Running softmax state of one stream for the lane's query (m in log2 units).
+// Running softmax state of one stream for the lane's query: the reference m (log2 units), the
+// sum l of the probabilities (in each element), the values.
 template <int NDT>
 struct PfAcc {
-  float m, l;
+  float m;
+  f32x4 l;
   f32x4 z[NDT];   // O^T[16 dt + 4g + i][query c16]
 };
 
-template <int NP>   // dh = 32 NP
+// dh = 32 NP.  FAR: rows 2^24 bytes apart or more, whose offsets take 64 bits.
+template <int NP, bool FAR>
 __global__ __launch_bounds__(256, NP == 4 ? 2 : 3) void maba_sa_prefill_kernel(PfArgs a) {
   constexpr int DH = 32 * NP;
-  constexpr int TP = DH + 8;      // row pitch (bf16) of the LDS key and value tiles
   constexpr int NDT = DH / 16;
-  constexpr int TE = 64 * TP;
+  constexpr int NC = 4 * NP;      // 16-byte chunks per row
+  constexpr int RP = 256 / NC;    // rows per staging pass of the workgroup
+  constexpr int TE = 64 * DH;
   __shared__ __attribute__((aligned(16))) short s_k[2][TE];
   __shared__ __attribute__((aligned(16))) short s_v[2][TE];
   __shared__ uint32_t s_bits[PF_WORDS];
@@ -92,18 +121,26 @@ __global__ __launch_bounds__(256, NP == 4 ? 2 : 3) void maba_sa_prefill_kernel(P
   // set-up's last barrier): the list position of each bitmap word's first block, the list length.
   int* s_wpre = (int*)&s_v[1][0];
   int* s_nlist = s_wpre + PF_WORDS;
-  static_assert((PF_WORDS + 1) * 4 <= TE * 2, "set-up tables fit one value buffer");
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  int* s_count = s_nlist + 1;   // some query lists a block twice: slots are counted
+  static_assert((PF_WORDS + 2) * 4 <= TE * 2, "set-up tables fit one value buffer");
+  // per query, the list entries it lists, behind the entries of a list that short
+  uint32_t (*s_qbits)[PF_QWORDS] = (uint32_t (*)[PF_QWORDS])(s_list + 32 * PF_QWORDS);
+  static_assert(64 * PF_QWORDS * 4 + 32 * PF_QWORDS * 2 <= PF_LIST * 2, "the rows of bits fit behind the list");
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int g = lane >> 4, c16 = lane & 15;
   const int64_t b = blockIdx.z;
   const int h = blockIdx.y;
-  const int64_t tw0 = (int64_t)blockIdx.x * 64;                // the workgroup's first query (< Lq)
+  // the workgroup's first query (< Lq): the last groups see the most keys and start first
+  const int64_t tw0 = (int64_t)(gridDim.x - 1 - blockIdx.x) * 64;
   const int64_t tq0 = tw0 + wave * 16;                         // the wave's first query
   const bool qvalid = tq0 + c16 < a.Lq;
   const int64_t tq = qvalid ? tq0 + c16 : a.Lq - 1;            // extra columns repeat the last query
   const int64_t off = a.Lkv - a.Lq;
   const int pos = (int)(off + tq);   // key positions fit 32 bits: Lkv <= PF_WORDS * 32 * 64
   const int64_t wpos_lo = off + tw0;
+  // the wave's own first and last position: a tile inside every query's range needs no row masks
+  const int vpos_lo = __builtin_amdgcn_readfirstlane((int)(off + min(tq0, a.Lq - 1)));
+  const int vpos_hi = __builtin_amdgcn_readfirstlane((int)(off + min(tq0 + 15, a.Lq - 1)));
   const int64_t wpos_hi = off + min(tw0 + 63, a.Lq - 1);
 
   pf16x8 qb[NP];   // lane (query c16, group g): dims 32 p + 8 g .. +7
@@ -188,122 +225,186 @@ __global__ __launch_bounds__(256, NP == 4 ? 2 : 3) void maba_sa_prefill_kernel(P
   const int64_t e_hi = min(a.nc - 1, (wpos_hi + 1) / a.pool - 1);
   const int n_hca = e_hi >= 0 ? (int)(e_hi / 64 + 1) : 0;
   for (int wd = tid; wd < 4 * (PF_LIST / 32); wd += 256) (&s_need[0][0])[wd] = 0u;
+  if (tid == 0) *s_count = 0;
   __syncthreads();
-  const int n_sp = *s_nlist;
+  const int n_sp = __builtin_amdgcn_readfirstlane(*s_nlist);
+  const bool is_short = n_sp <= 32 * PF_QWORDS;
+  if (is_short) {
+    for (int wd = tid; wd < 64 * PF_QWORDS; wd += 256) (&s_qbits[0][0])[wd] = 0u;
+  }
+  __syncthreads();
   if (qvalid) {   // mark the list entries of the lane's slots for its wave
 #pragma unroll
     for (int r = 0; r < PF_MAXK / 4; ++r) {
       const int bk = (int)((myblk[r >> 1] >> (16 * (r & 1))) & 0xffffu);
       if (bk < nbl) {
         const int u = s_wpre[bk >> 5] + __popc(s_bits[bk >> 5] & ((1u << (bk & 31)) - 1u));
-        atomicOr(&s_need[wave][u >> 5], 1u << (u & 31));
+        const uint32_t bit = 1u << (u & 31);
+        atomicOr(&s_need[wave][u >> 5], bit);
+        if (is_short && (atomicOr(&s_qbits[16 * wave + c16][u >> 5], bit) & bit)) *s_count = 1;
       }
     }
   }
   __syncthreads();
+  const bool by_bits = is_short && *s_count == 0;
   const int n_ls = n_loc + n_sp;
   const int nt = n_ls + n_hca;
 
-  // ---- tile staging: thread tid copies row tid / 4, 16-byte chunks (tid % 4) + 4 p, of the
-  // key and value tiles; the next tile's loads are in flight while the current one computes.
+  // ---- tile staging: thread tid copies chunk tid % NC of rows tid / NC + RP p of the key and
+  // value tiles; the next tile's loads are in flight while the current one computes.  Tile
+  // bases are uniform, a lane adds its byte offset, its row clamped to the last one (such rows
+  // are masked).
   const uint16_t* kbase = a.k + b * a.ksb + h * a.ksh;
   const uint16_t* vbase = a.v + b * a.vsb + h * a.vsh;
   const uint16_t* khbase = a.kh ? a.kh + b * a.khb + h * a.khh : nullptr;
   const uint16_t* vhbase = a.vh ? a.vh + b * a.vhb + h * a.vhh : nullptr;
-  const int srow = tid >> 2, spart = tid & 3;
+  const int srow = tid / NC, sch = tid % NC;
+  short* kw = &s_k[0][0] + (srow * NC + (sch ^ pf_kswz<NP>(srow))) * 8;
+  short* vw = &s_v[0][0] + (srow * NC + (sch ^ pf_vswz<NP>(srow))) * 8;
   pf16x8 pk[NP], pv[NP];
   auto fetch = [&](int i) {
     const uint16_t* kr;
     const uint16_t* vr;
+    int64_t ks, vs;
+    int last;
     if (i < n_ls) {
       const int64_t tb = i < n_st ? 64 * (int64_t)i
-                       : i < n_loc ? wt0 + 64 * (int64_t)(i - n_st) : 64 * (int64_t)s_list[i - n_loc];
-      const int64_t j = min(tb + srow, a.Lkv - 1);
-      kr = kbase + j * a.kst;
-      vr = vbase + j * a.vst;
+                       : i < n_loc ? wt0 + 64 * (int64_t)(i - n_st)
+                                   : 64 * (int64_t)__builtin_amdgcn_readfirstlane((int)s_list[i - n_loc]);
+      kr = kbase + tb * a.kst;
+      vr = vbase + tb * a.vst;
+      ks = a.kst; vs = a.vst;
+      last = (int)min(a.Lkv - 1 - tb, (int64_t)63);
     } else {
-      const int64_t e = min(64 * (int64_t)(i - n_ls) + srow, a.nc - 1);
-      kr = khbase + e * a.khe;
-      vr = vhbase + e * a.vhe;
+      const int64_t e0 = 64 * (int64_t)(i - n_ls);
+      kr = khbase + e0 * a.khe;
+      vr = vhbase + e0 * a.vhe;
+      ks = a.khe; vs = a.vhe;
+      last = (int)min(a.nc - 1 - e0, (int64_t)63);
     }
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
-      pk[p] = *(const pf16x8*)(kr + 8 * (spart + 4 * p));
-      pv[p] = *(const pf16x8*)(vr + 8 * (spart + 4 * p));
+      const int r = min(srow + RP * p, last);
+      if constexpr (FAR) {
+        pk[p] = *(const pf16x8*)(kr + r * ks + 8 * sch);
+        pv[p] = *(const pf16x8*)(vr + r * vs + 8 * sch);
+      } else {
+        pk[p] = *(const pf16x8*)((const char*)kr + (__umul24(r, (uint32_t)ks * 2u) + 16u * sch));
+        pv[p] = *(const pf16x8*)((const char*)vr + (__umul24(r, (uint32_t)vs * 2u) + 16u * sch));
+      }
     }
   };
-  auto stash = [&](int buf) {
+  auto stash = [&](int buf) {   // pf_kswz and pf_vswz repeat every RP rows
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
-      *(pf16x8*)(s_k[buf] + srow * TP + 8 * (spart + 4 * p)) = pk[p];
-      *(pf16x8*)(s_v[buf] + srow * TP + 8 * (spart + 4 * p)) = pv[p];
+      *(pf16x8*)(kw + buf * TE + RP * p * DH) = pk[p];
+      *(pf16x8*)(vw + buf * TE + RP * p * DH) = pv[p];
     }
+  };
+  // the lane's read addresses: key rows 16 rb + c16, chunk 4 p + g; value rows
+  // 16 rb + 4 g + c16 / 4, columns 16 dt + 4 (c16 % 4) .. (transposed: the lane receives column
+  // c16 of rows 4 g .. 4 g + 3)
+  const short* kl[NP];
+  const short* vl[NDT];
+#pragma unroll
+  for (int p = 0; p < NP; ++p) kl[p] = &s_k[0][0] + (c16 * NC + ((4 * p + g) ^ pf_kswz<NP>(c16))) * 8;
+  {
+    const int r = 4 * g + (c16 >> 2);
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt)
+      vl[dt] = &s_v[0][0] + (r * NC + ((2 * dt + ((c16 >> 1) & 1)) ^ pf_vswz<NP>(r))) * 8 + 4 * (c16 & 1);
+  }
+  auto vT = [](const short* p) {
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) pf16x4*)p);
   };
 
   // One 64-key tile from LDS buffer buf: the lane's rows with bit 4 rb + i of vmask set
-  // (row 16 rb + 4 g + i) have weight fc, the others 0.  A wave none of whose queries weights
-  // any row skips the tile: for such a lane the tile would leave (m, l, z) exactly as they
-  // are.  Scores are scaled to log2 units (scale * log2 e) so that each probability is one
-  // exp2; a tile whose 64 rows are valid for every lane of the wave skips the masking.
+  // (row 16 rb + 4 g + i) have weight 2^lw, the others 0 (lw = -inf: all of them).  A wave none
+  // of whose queries weights any row skips the tile: for such a lane the tile would leave its
+  // state exactly as it is.  Scores are taken in log2 units (scale * log2 e); rows are masked one
+  // by one only where some lane weights a part of the tile.
   const float sl2 = a.scale * 1.4426950408889634f;
-  auto tile = [&](PfAcc<NDT>& st, int buf, float fc, uint32_t vmask) {
-    if (!qvalid || !(fc > 0.f)) vmask = 0u;
+  auto tile = [&](PfAcc<NDT>& st, int buf, float lw, uint32_t vmask) {
+    if (!qvalid || lw == -INFINITY) vmask = 0u;
+    if (vmask == 0u) lw = -INFINITY;
     if (__ballot(vmask != 0u) == 0ull) return;   // wave-uniform
-    const bool full = __ballot(qvalid && vmask != 0xffffu) == 0ull;
-    const short* ks = s_k[buf];
-    const short* vt = s_v[buf];
-    f32x4 sc[4];
+    const bool part = __ballot(vmask != 0u && vmask != 0xffffu) != 0ull;
+    f32x4 sc[4], x[4];
 #pragma unroll
     for (int rb = 0; rb < 4; ++rb) {
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int p = 0; p < NP; ++p) {
-        const pf16x8 kv = *(const pf16x8*)(ks + (16 * rb + c16) * TP + 32 * p + 8 * g);
+        const pf16x8 kv = *(const pf16x8*)(kl[p] + buf * TE + 16 * rb * DH);
         acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kv),
                                                       __builtin_bit_cast(bf16x8, qb[p]), acc, 0, 0, 0);
       }
       sc[rb] = acc;
     }
-    // lane (query c16, g) holds the scores of keys 16 rb + 4 g + i
-    float tmax = -INFINITY;
+    // lane (query c16, g) holds the scores of keys 16 rb + 4 g + i; x: relative to the reference
+    auto relative = [&]() {
+      const float bias = lw == -INFINITY ? -INFINITY : st.m == -INFINITY ? lw : lw - st.m;
 #pragma unroll
-    for (int rb = 0; rb < 4; ++rb)
+      for (int rb = 0; rb < 4; ++rb)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float x = (full || ((vmask >> (4 * rb + i)) & 1u)) ? sc[rb][i] * sl2 : -INFINITY;
-        sc[rb][i] = x;
-        tmax = fmaxf(tmax, x);
+        for (int i = 0; i < 4; ++i) x[rb][i] = fmaf(sc[rb][i], sl2, bias);
+      if (part) {
+        uint32_t vm = vmask;
+        asm volatile("" : "+v"(vm));   // the bit tests stay in this branch
+#pragma unroll
+        for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) x[rb][i] = ((vm >> (4 * rb + i)) & 1u) ? x[rb][i] : -INFINITY;
       }
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 16));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
-    const float m_new = fmaxf(st.m, tmax);
-    const float corr = (m_new == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f(st.m - m_new);
-    const float m_sub = (m_new == -INFINITY) ? 0.f : m_new;
-    float psum = 0.f;
+    };
+    auto largest = [&]() {
+      float mx = -INFINITY;
+#pragma unroll
+      for (int rb = 0; rb < 4; ++rb) mx = fmaxf(fmaxf(mx, fmaxf(x[rb][0], x[rb][1])), fmaxf(x[rb][2], x[rb][3]));
+      return mx;
+    };
+    relative();
+    const float mx = largest();
+    if (__ballot(mx > PF_SLACK || (st.m == -INFINITY && lw != -INFINITY)) != 0ull) {
+      // some query's reference moves: to the largest score so far, in all of its lanes
+      const float base = st.m == -INFINITY ? 0.f : st.m;
+      float top = lw == -INFINITY ? -INFINITY : mx - lw + base;
+      top = group_max(top);
+      const float m_new = fmaxf(st.m, top);
+      const float corr = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(st.m - m_new);
+      st.m = m_new;
+      st.l *= corr;   // every element is the query's sum
+#pragma unroll
+      for (int dt = 0; dt < NDT; ++dt) st.z[dt] *= corr;
+      relative();
+    }
     i16x4 ph[4], pl[4];
 #pragma unroll
     for (int rb = 0; rb < 4; ++rb) {
       f32x4 pe;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        pe[i] = fc * __builtin_amdgcn_exp2f(sc[rb][i] - m_sub);   // exp2(-inf) = 0 for masked keys
-        psum += pe[i];
-      }
+      for (int i = 0; i < 4; ++i) pe[i] = __builtin_amdgcn_exp2f(x[rb][i]);   // exp2(-inf) = 0 for masked keys
       split4(pe, ph[rb], pl[rb]);
     }
-    psum += __shfl_xor(psum, 16);
-    psum += __shfl_xor(psum, 32);
-    st.l = st.l * corr + psum;
-    st.m = m_new;
-    // O^T[dim][query] = corr O^T + V^T P over the 64 keys as two 32-key steps whose key order
+    // l += the probabilities' sum, as a product with a row of ones
+    {
+      const short one = 0x3f80;
+      const pf16x8 ones = {one, one, one, one, one, one, one, one};
+#pragma unroll
+      for (int p2 = 0; p2 < 2; ++p2) {
+        st.l = mma32(st.l, ones, cat8(ph[2 * p2], ph[2 * p2 + 1]));
+        st.l = mma32(st.l, ones, cat8(pl[2 * p2], pl[2 * p2 + 1]));
+      }
+    }
+    // O^T[dim][query] += V^T P over the 64 keys as two 32-key steps whose key order
     // (16 rb + 4 g + i, rb in {2 p2, 2 p2 + 1}) matches the probabilities this lane holds
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt) {
-      f32x4 acc = st.z[dt] * corr;
+      f32x4 acc = st.z[dt];
 #pragma unroll
       for (int p2 = 0; p2 < 2; ++p2) {
-        const pf16x4 a0 = pf_ldsT4(vt, TP, 32 * p2, 16 * dt, c16, g);
-        const pf16x4 a1 = pf_ldsT4(vt, TP, 32 * p2 + 16, 16 * dt, c16, g);
+        const pf16x4 a0 = vT(vl[dt] + buf * TE + 32 * p2 * DH);
+        const pf16x4 a1 = vT(vl[dt] + buf * TE + (32 * p2 + 16) * DH);
         const pf16x8 av = {a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
         const i16x8 bh = cat8(ph[2 * p2], ph[2 * p2 + 1]), bl = cat8(pl[2 * p2], pl[2 * p2 + 1]);
         acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, av), __builtin_bit_cast(bf16x8, bh),
@@ -316,24 +417,24 @@ __global__ __launch_bounds__(256, NP == 4 ? 2 : 3) void maba_sa_prefill_kernel(P
   };
   auto reset = [&](PfAcc<NDT>& st) {
     st.m = -INFINITY;
-    st.l = 0.f;
+    st.l = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt) st.z[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
   };
   auto fold = [&](const PfAcc<NDT>& st, float gs) {   // o += g_s z_s / l_s
-    const float w = st.l > 0.f ? gs / st.l : 0.f;
+    const float w = st.l[0] > 0.f ? gs / st.l[0] : 0.f;
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt) o[dt] += st.z[dt] * w;
   };
   // tiles [i, i_end): prefetch tile i + 1 (of whichever stream), compute tile i, stage the
-  // prefetched tile into the other buffer, one barrier per tile.  weight_of(i) gives tile i's
-  // weight for the lane's query and mask_of(i) its row mask (pf_range_bits).
+  // prefetched tile into the other buffer, one barrier per tile.  weight_of(i) gives the log2 of
+  // tile i's weight for the lane's query and mask_of(i) its row mask (pf_range_bits).
   int i = 0;
   auto run = [&](PfAcc<NDT>& st, int i_end, auto weight_of, auto mask_of) {
     for (; i < i_end; ++i) {
       if (i + 1 < nt) fetch(i + 1);
-      const float fc = weight_of(i);
-      tile(st, i & 1, fc, fc > 0.f ? mask_of(i) : 0u);
+      const float lw = weight_of(i);
+      tile(st, i & 1, lw, lw != -INFINITY ? mask_of(i) : 0u);
       if (i + 1 < nt) stash((i + 1) & 1);
       __syncthreads();
     }
@@ -348,20 +449,26 @@ __global__ __launch_bounds__(256, NP == 4 ? 2 : 3) void maba_sa_prefill_kernel(P
   // ---- local stream: sink tiles hold keys [0, min(sink_end, pos + 1)); window tiles the keys
   // in (pos - window, pos] and the sinks below min(ns, pos + 1)
   reset(st);
-  run(st, n_loc, [](int) { return 1.f; }, [&](int ti) {
+  run(st, n_loc, [](int) { return 0.f; }, [&](int ti) {
     if (ti < n_st) return pf_range_bits(-64 * ti, min((int)sink_end - 1, pos) - 64 * ti, g);
     const int tb = (int)wt0 + 64 * (ti - n_st);
+    if (tb + 63 <= vpos_lo && tb > vpos_hi - a.window) return 0xffffu;
     return pf_range_bits(pos - a.window + 1 - tb, pos - tb, g) |
            pf_range_bits(-tb, min((int)ns - 1, pos) - tb, g);
   });
   fold(st, g0);
 
   // ---- sparse stream: each key weighted by how often the lane's query lists its block; a
-  // wave skips the entries none of its queries lists without counting
+  // wave skips the entries none of its queries lists
   reset(st);
+  uint32_t word = 0u;
   run(st, n_ls, [&](int ti) {
     const int u = ti - n_loc;
-    if (((s_need[wave][u >> 5] >> (u & 31)) & 1u) == 0u) return 0.f;   // wave-uniform
+    if (by_bits) {
+      if ((u & 31) == 0) word = s_qbits[16 * wave + c16][u >> 5];
+      return ((word >> (u & 31)) & 1u) ? 0.f : -INFINITY;
+    }
+    if (((s_need[wave][u >> 5] >> (u & 31)) & 1u) == 0u) return -INFINITY;   // wave-uniform
     const int blk = s_list[u];
     int cnt = 0;
 #pragma unroll
@@ -369,15 +476,22 @@ __global__ __launch_bounds__(256, NP == 4 ? 2 : 3) void maba_sa_prefill_kernel(P
       cnt += (int)((myblk[m] & 0xffffu) == (uint32_t)blk) + (int)((myblk[m] >> 16) == (uint32_t)blk);
     cnt += __shfl_xor(cnt, 16);
     cnt += __shfl_xor(cnt, 32);
-    return (float)cnt;
-  }, [&](int ti) { return pf_range_bits(0, pos - 64 * (int)s_list[ti - n_loc], g); });
+    return cnt > 0 ? __builtin_amdgcn_logf((float)cnt) : -INFINITY;
+  }, [&](int ti) {
+    const int tb = 64 * __builtin_amdgcn_readfirstlane((int)s_list[ti - n_loc]);
+    return tb + 63 <= vpos_lo ? 0xffffu : pf_range_bits(0, pos - tb, g);
+  });
   fold(st, g1);
 
   // ---- HCA stream: means e <= e_max, the last complete block's mean before the lane's query;
   // early queries take their row
   reset(st);
   const int e_max = (int)min(a.nc - 1, (int64_t)((pos + 1) / a.pool) - 1);
-  run(st, nt, [](int) { return 1.f; }, [&](int ti) { return pf_range_bits(0, e_max - 64 * (ti - n_ls), g); });
+  const int ve_max = (int)min(a.nc - 1, (int64_t)((vpos_lo + 1) / a.pool) - 1);
+  run(st, nt, [](int) { return 0.f; }, [&](int ti) {
+    const int e0 = 64 * (ti - n_ls);
+    return e0 + 63 <= ve_max ? 0xffffu : pf_range_bits(0, e_max - e0, g);
+  });
   if (pos < a.pool - 1) {   // running mean of c[0..pos] through W_v (the caller's row)
     const bool have = a.early && tq < a.n_early;
 #pragma unroll
@@ -486,10 +600,16 @@ extern "C" int maba_hip_maba_sa_prefill(const maba_tensor* q, const maba_tensor*
   a.K = (int)K; a.window = window; a.n_sink = n_sink; a.pool = pool; a.scale = scale;
   hipStream_t s = (hipStream_t)stream;
   const dim3 grid((unsigned)ceil_div(Lq, 64), (unsigned)H, (unsigned)B);
-  switch (dh) {
-    case 32: hipLaunchKernelGGL(maba_sa_prefill_kernel<1>, grid, dim3(256), 0, s, a); break;
-    case 64: hipLaunchKernelGGL(maba_sa_prefill_kernel<2>, grid, dim3(256), 0, s, a); break;
-    default: hipLaunchKernelGGL(maba_sa_prefill_kernel<4>, grid, dim3(256), 0, s, a); break;
-  }
+  auto far = [](int64_t st) { return st < 0 || st >= (1 << 23); };   // elements
+  auto launch = [&](auto far_c) {
+    constexpr bool FAR = decltype(far_c)::value;
+    switch (dh) {
+      case 32: hipLaunchKernelGGL((maba_sa_prefill_kernel<1, FAR>), grid, dim3(256), 0, s, a); break;
+      case 64: hipLaunchKernelGGL((maba_sa_prefill_kernel<2, FAR>), grid, dim3(256), 0, s, a); break;
+      default: hipLaunchKernelGGL((maba_sa_prefill_kernel<4, FAR>), grid, dim3(256), 0, s, a); break;
+    }
+  };
+  if (far(a.kst) || far(a.vst) || far(a.khe) || far(a.vhe)) launch(std::true_type{});
+  else launch(std::false_type{});
   return check_launch("maba_sa_prefill");
 }

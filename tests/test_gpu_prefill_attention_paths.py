@@ -1,0 +1,66 @@
+"""Branches of the head-space MABA-SA prefill that only some selections or shapes take, against
+the float64 oracle (rtol = atol = 2e-3, as test_gpu_prefill_attention.py): distinct blocks read
+from bits, a union too long for them, references that move far, rows whose offsets need 64 bits."""
+import pytest
+import torch
+
+from _helpers import assert_close, to_np
+from oracle import sparse_attn as osa
+from test_gpu_prefill_attention import _case, _hip
+
+pytestmark = pytest.mark.gpu
+
+
+def _distinct(B, Lq, nb, K, seed):
+    g = torch.Generator().manual_seed(seed)
+    return torch.rand(B, Lq, nb, generator=g).argsort(dim=-1)[..., :K]
+
+
+def _check(dev, case, scale, what, **kw):
+    q, k, v, kh, vh, early, idx, gate = case
+    d = lambda t: None if t is None else t.to(dev)  # noqa: E731
+    out = _hip().hip_maba_sa_prefill(*(d(t) for t in case), scale=scale, out_dtype=torch.float32, **kw)
+    exp = osa.maba_sa_prefill_heads(*(to_np(t) if t is not None else None for t in (q, k, v, kh, vh, early)), idx.numpy(),
+                                    to_np(gate), window=kw.get("window", 128), n_sink=kw.get("n_sink", 4), scale=scale)
+    assert_close(out, exp, 2e-3, 2e-3, what)
+
+
+@pytest.mark.parametrize("dh", [32, 64, 128])
+@pytest.mark.parametrize("Lq,Lkv,K", [(100, 100, 1), (100, 2500, 7), (65, 4160, 64)])
+def test_distinct_blocks(dev, dh, Lq, Lkv, K):
+    case = list(_case(1, 2, Lq, Lkv, dh, K, dh + Lkv))
+    case[6] = _distinct(1, Lq, (Lkv + 63) // 64, K, 1)
+    _check(dev, case, dh ** -0.5, f"distinct {dh} {Lkv}")
+
+
+def test_union_beyond_the_bits(dev):
+    """64 queries of 64 distinct blocks each among 700: more than 512 in the union."""
+    Lq, Lkv = 64, 64 * 700
+    case = list(_case(1, 1, Lq, Lkv, 64, 64, 3))
+    case[6] = _distinct(1, Lq, 700, 64, 2)
+    assert case[6].unique().numel() > 512
+    _check(dev, case, 0.125, "long union")
+
+
+@pytest.mark.parametrize("scale", [4.0, 0.0, -1.0])
+@pytest.mark.parametrize("dup", [False, True])
+def test_references_that_move(dev, scale, dup):
+    """Scores of hundreds of log2 units, so the running reference moves at most tiles; scores all
+    equal; a negative scale (masked keys stay masked)."""
+    case = list(_case(1, 2, 150, 1000, 64, 8, 7, dup=dup))
+    if not dup:
+        case[6] = _distinct(1, 150, 16, 8, 4)
+    _check(dev, case, scale, f"scale {scale}")
+
+
+def test_far_rows(dev):
+    """Key rows 2^23 elements apart."""
+    q, k, v, kh, vh, early, idx, gate = _case(1, 1, 70, 70, 64, 2, 9)
+    buf = torch.empty(70, 1 << 23, dtype=torch.bfloat16, device=dev)
+    far = buf[:, :64].view(1, 1, 70, 64)
+    far.copy_(k)
+    d = lambda t: None if t is None else t.to(dev)  # noqa: E731
+    args = [d(t) for t in (q, k, v, kh, vh, early, idx, gate)]
+    want = _hip().hip_maba_sa_prefill(*args, scale=0.125)
+    args[1] = far
+    assert torch.equal(_hip().hip_maba_sa_prefill(*args, scale=0.125), want)

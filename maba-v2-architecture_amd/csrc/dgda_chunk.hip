@@ -14,7 +14,7 @@
 //
 // Sequence parallelism (only B*H = 40 recurrences at the BASELINE shape, but
 // 256 CUs): the (b,h)-major sequence of all B*H*nchunks chunks is cut into slots
-// of U chunks, U = max(CPS, ceil(total / (2 * CUs))), so that the output pass runs
+// of U chunks, U = max(CPS_FINE, ceil(total / (2 * CUs))), so that the output pass runs
 // exactly one wave of workgroups (two per CU) of equal length.  A segment is the
 // part of one (b,h) sequence inside one slot; each (b,h) has up to nseg_max.
 //   pass 1 (dgda_chunk_kernel<AGG>) runs every segment but the first of each (b,h)
@@ -48,7 +48,9 @@ namespace maba {
 constexpr int CH = 64;        // chunk length (tokens)
 constexpr int DK = 64;        // key / value head size
 constexpr int TPITCH = 20;    // bf16 row pitch of the 16x16 inverse blocks
-constexpr int CPS = 16;       // chunks per segment
+constexpr int CPS = 16;       // chunks per slot at least, with the least workspace
+constexpr int CPS_FINE = 4;   // and with the preferred one
+constexpr int SHORT_CHUNKS = 14;   // up to here a sequence stays whole (chunk_geom)
 // The aggregate pass's bound (see chunk_segment): chunks probed, the log-decay at which the start
 // state no longer counts, and the largest b |k|^2 taken as a contraction (2, less a margin for
 // the rounding of the fp32 sums).
@@ -92,9 +94,6 @@ struct ChunkArgs {
 };
 
 __device__ __forceinline__ int seg_count(const ChunkArgs& a, int bh) { return seg_count_of(a.nchunks, a.U, bh); }
-__device__ __forceinline__ void seg_range(const ChunkArgs& a, int bh, int k, int n, int& c0, int& c1) {
-  seg_range_of(a.nchunks, a.U, bh, k, n, c0, c1);
-}
 
 // Lower-triangular 64x64 matrices are stored as their 10 lower 16x16 tiles
 // (tile (I,J), J <= I, at index I(I+1)/2 + J), rows padded to TPITCH.
@@ -684,7 +683,7 @@ template <bool AGG, bool WTOK, bool OBF>
 __global__ __launch_bounds__(AGG ? 512 : 256, AGG ? 1 : 2) void dgda_chunk_kernel(ChunkArgs a) {
   __shared__ ChunkSmem<AGG> sm;
   __shared__ int s_mzero[5];   // [0, 4): the M slabs' zero flags; [4]: the bound's chunk count
-  // Pass 1 and OUT_FIX: one workgroup per segment k >= 1.  OUT_ZERO: slot w covers
+  // Pass 1 and OUT_FIX: the segments k >= 1, one workgroup per slot.  OUT_ZERO: slot w covers
   // the chunks [U w, U w + U) of the (b,h)-major order, one segment per sequence it
   // touches.  Both walk the same loop so the segment body is inlined once.
   const bool per_segment = AGG || a.mode == OUT_FIX;
@@ -694,12 +693,21 @@ __global__ __launch_bounds__(AGG ? 512 : 256, AGG ? 1 : 2) void dgda_chunk_kerne
   while (G < Gend) {
     int bh, k, n, c0, c1;
     if (per_segment) {
-      const int per = a.nseg_max - 1;
-      bh = blockIdx.x / per;
-      k = blockIdx.x % per + 1;
+      // A segment k >= 1 starts where its slot does, so the slots that start inside a sequence
+      // are these segments, and the grid has no more workgroups than fit in one round of the
+      // output pass or two of the aggregate (with a workgroup per sequence and possible segment
+      // there was a third: B=1 T=32768, decay that remembers, 424 us against 378).  Every eighth
+      // workgroup goes to the same XCD; each eight of them are rotated by one, or the slots that
+      // start a sequence (which end here) could all be one XCD's.
+      int64_t w = blockIdx.x;
+      if ((w | 7) < gridDim.x) w = (w & ~(int64_t)7) | ((w + (w >> 3)) & 7);
+      const int64_t start = w * a.U;
+      bh = (int)(start / a.nchunks);
+      c0 = (int)(start - (int64_t)bh * a.nchunks);
+      if (c0 == 0) return;
+      k = (int)(w - (int64_t)bh * a.nchunks / a.U);
       n = seg_count(a, bh);
-      if (k >= n) return;
-      seg_range(a, bh, k, n, c0, c1);
+      c1 = (int)min((int64_t)a.nchunks, c0 + a.U);
       G = Gend;
     } else {
       bh = (int)(G / a.nchunks);
@@ -751,16 +759,33 @@ bool dgda_chunk_supported(const maba_tensor* q, const maba_tensor* k, const maba
   return true;
 }
 
-static SlotGeom chunk_geom(int64_t BH, int64_t L) {
-  const int64_t nch = ceil_div(L, CH) > 0 ? ceil_div(L, CH) : 1;
-  return slot_geom(BH, nch, CPS);
+static size_t chunk_geom_bytes(const SlotGeom& gm, int64_t BH) {
+  if (gm.nseg_max <= 1) return 16;
+  const int64_t nseg = BH * gm.nseg_max;
+  return (size_t)(nseg * 64 * 128) * sizeof(float) + (size_t)nseg * sizeof(int);
 }
 
-size_t dgda_chunk_workspace(int64_t BH, int64_t L) {
-  const SlotGeom gm = chunk_geom(BH, L);
-  if (gm.nseg_max <= 1) return 16;
-  const int64_t nseg = gm.nseg_max;
-  return (size_t)(BH * nseg * 64 * 128) * sizeof(float) + (size_t)(BH * nseg) * sizeof(int);
+// Slots of CPS chunks at least, or of CPS_FINE where the workspace holds that many segments: a
+// workgroup takes about 4.6 us per chunk however few there are, so slots of 16 chunks leave an
+// idle chip waiting for them (CPS 16 -> 4, us, decay that vanishes / that remembers: B=1 H=10
+// T=2048 85 -> 38 / 211 -> 79; B=2 T=5000 92 -> 51 / 218 -> 156; B=2 T=10007 93 -> 66 /
+// 228 -> 198; B=4 T=8192 105 -> 80 / 330 -> 240; no change at T=32768).  2 measured as 4 where
+// maps vanish and slower with many surviving ones (B=1 T=5000 161 against 100), 8 slower.
+// A sequence that CPS leaves whole is cut where that costs nothing even if every map survives
+// and each segment runs twice: from 15 chunks (B=4 T=1000 75 -> 38 / 75 -> 71, but 11 chunks
+// 53 -> 39 / 53 -> 68), and while each slot has a CU (B=8 T=1000, 320 slots: 75 -> 46 / 75 -> 104).
+static SlotGeom chunk_geom(int64_t BH, int64_t L, size_t ws_bytes) {
+  const int64_t nch = ceil_div(L, CH) > 0 ? ceil_div(L, CH) : 1;
+  const SlotGeom coarse = slot_geom(BH, nch, CPS), fine = slot_geom(BH, nch, CPS_FINE);
+  const bool pays = coarse.nseg_max > 1 ||
+                    (nch > SHORT_CHUNKS && ceil_div(BH * nch, fine.U) <= device_cu_count());
+  return pays && chunk_geom_bytes(fine, BH) <= ws_bytes ? fine : coarse;
+}
+
+// The size the query promises to be enough, and the one with which a call is cut as finely as pays.
+size_t dgda_chunk_workspace(int64_t BH, int64_t L) { return chunk_geom_bytes(chunk_geom(BH, L, 0), BH); }
+size_t dgda_chunk_workspace_preferred(int64_t BH, int64_t L) {
+  return chunk_geom_bytes(chunk_geom(BH, L, SIZE_MAX), BH);
 }
 
 int launch_dgda_chunk(const maba_tensor* q, const maba_tensor* k, const maba_tensor* v,
@@ -786,7 +811,7 @@ int launch_dgda_chunk(const maba_tensor* q, const maba_tensor* k, const maba_ten
   a.sf = mview4(sf);
   a.H = (int)H; a.L = (int)L; a.BH = (int)BH;
   a.nchunks = (int)(ceil_div(L, CH) > 0 ? ceil_div(L, CH) : 1);
-  const SlotGeom gm = chunk_geom(BH, L);
+  const SlotGeom gm = chunk_geom(BH, L, ws_bytes);
   a.U = gm.U;
   a.nseg_max = gm.nseg_max;
   a.use_log = use_log; a.has_s0 = s0 != nullptr;
@@ -796,9 +821,9 @@ int launch_dgda_chunk(const maba_tensor* q, const maba_tensor* k, const maba_ten
   a.agg = (float*)ws;
   a.zc = (int*)(a.agg + nsegs * 64 * 128);
   const bool obf = out->dtype == MABA_BF16;
+  const dim3 grid((unsigned)ceil_div(BH * a.nchunks, a.U));   // one workgroup per slot
   auto launch_out = [&](int mode) {
     a.mode = mode;
-    const dim3 grid(mode == OUT_ZERO ? (unsigned)ceil_div(BH * a.nchunks, a.U) : (unsigned)(BH * (a.nseg_max - 1)));
     if (a.w_tok && obf) hipLaunchKernelGGL((dgda_chunk_kernel<false, true, true>), grid, dim3(256), 0, stream, a);
     else if (a.w_tok) hipLaunchKernelGGL((dgda_chunk_kernel<false, true, false>), grid, dim3(256), 0, stream, a);
     else if (obf) hipLaunchKernelGGL((dgda_chunk_kernel<false, false, true>), grid, dim3(256), 0, stream, a);
@@ -810,9 +835,8 @@ int launch_dgda_chunk(const maba_tensor* q, const maba_tensor* k, const maba_ten
     return launch_out(OUT_ZERO);
   }
   a.mode = OUT_ZERO;
-  const dim3 agrid((unsigned)(BH * (a.nseg_max - 1)));
-  if (a.w_tok) hipLaunchKernelGGL((dgda_chunk_kernel<true, true, true>), agrid, dim3(512), 0, stream, a);
-  else hipLaunchKernelGGL((dgda_chunk_kernel<true, false, true>), agrid, dim3(512), 0, stream, a);
+  if (a.w_tok) hipLaunchKernelGGL((dgda_chunk_kernel<true, true, true>), grid, dim3(512), 0, stream, a);
+  else hipLaunchKernelGGL((dgda_chunk_kernel<true, false, true>), grid, dim3(512), 0, stream, a);
   int rc = check_launch("dgda_prefill/aggregate");
   if (rc) return rc;
   if ((rc = launch_out(OUT_ZERO))) return rc;

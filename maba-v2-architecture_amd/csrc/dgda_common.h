@@ -179,11 +179,6 @@ __device__ __forceinline__ int seg_count_of(int nchunks, int64_t U, int bh) {
   const int64_t s = (int64_t)bh * nchunks;
   return (int)((s + nchunks - 1) / U - s / U + 1);
 }
-__device__ __forceinline__ void seg_range_of(int nchunks, int64_t U, int bh, int k, int n, int& c0, int& c1) {
-  const int64_t s = (int64_t)bh * nchunks, f = s / U;
-  c0 = k == 0 ? 0 : (int)(U * (f + k) - s);
-  c1 = k == n - 1 ? nchunks : (int)(U * (f + k + 1) - s);
-}
 
 // Slot geometry: U chunks per slot, at most nseg_max segments per sequence (1 when
 // every sequence fits one slot: then slots are aligned to sequences).  Two output

@@ -113,6 +113,7 @@ bool dgda_chunk_strides_fit(const maba_tensor* t);
 bool dgda_chunk_supported(const maba_tensor* q, const maba_tensor* k, const maba_tensor* v,
                           const maba_tensor* gate, const maba_tensor* b);
 size_t dgda_chunk_workspace(int64_t BH, int64_t L);
+size_t dgda_chunk_workspace_preferred(int64_t BH, int64_t L);
 int launch_dgda_chunk(const maba_tensor* q, const maba_tensor* k, const maba_tensor* v,
                       const maba_tensor* gate, int use_log, const maba_tensor* b,
                       const maba_tensor* w, const maba_tensor* s0, maba_tensor* out,
@@ -148,7 +149,9 @@ extern "C" size_t maba_hip_dgda_prefill_workspace_size(const maba_tensor* q, con
 extern "C" size_t maba_hip_dgda_prefill_workspace_preferred(const maba_tensor* q, const maba_tensor* v,
                                                            const maba_tensor* gate, const maba_tensor* b) {
   size_t n = maba_hip_dgda_prefill_workspace_size(q, v, gate, b);
-  if (n && dgda_sub_supported(q, q, v, gate, b, nullptr, nullptr) && !dgda_chunk_supported(q, q, v, gate, b))
+  if (n && dgda_chunk_supported(q, q, v, gate, b))
+    n = std::max(n, dgda_chunk_workspace_preferred(q->shape[0] * q->shape[1], q->shape[2]));
+  else if (n && dgda_sub_supported(q, q, v, gate, b, nullptr, nullptr))
     n = std::max(n, dgda_sub_workspace_preferred(q->shape[0] * q->shape[1], q->shape[2], q->shape[3], v->shape[3]));
   return n;
 }

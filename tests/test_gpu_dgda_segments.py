@@ -51,6 +51,23 @@ def test_segments_follow_the_workspace(dev, dk, dv, decay):
         assert_close(S, eS, 2e-3, 2e-3, f"state {nbytes}")
 
 
+@pytest.mark.parametrize("B,H,L", [(1, 1, 14 * 64), (1, 2, 14 * 64 + 1), (2, 3, 16 * 64), (3, 1, 16 * 64 + 1), (1, 3, 2100),
+                                   (65, 1, 1000)])
+@pytest.mark.parametrize("decay", ["baseline", "slow"])
+def test_chunk_segments_follow_the_workspace(dev, B, H, L, decay):
+    """Per-token gates: slots of four chunks with the preferred workspace, of sixteen with any
+    smaller one, at the lengths where the cut begins and changes."""
+    inp = dgda_inputs(B, H, L, seed=7, decay=decay, gates="scalar", device=dev, with_state=True)
+    assert inp["log_alpha"].stride(3) == 0 and inp["q"].dtype == torch.bfloat16
+    least, best = _sizes(inp)
+    assert (best > least) == (14 * 64 < L and B * H < 65)
+    eo, eS = odgda.dgda_prefill_seq(**oracle_dgda_args(inp))
+    for nbytes in sorted({least, best - 1, best} - {least - 1}):
+        o, S = _call(inp, nbytes, s0=inp["initial_state"])
+        assert_close(o, eo, 2e-3, 2e-3, f"out {nbytes}")
+        assert_close(S, eS, 2e-3, 2e-3, f"state {nbytes}")
+
+
 @pytest.mark.parametrize("decay", ["baseline", "slow"])
 def test_state_in_place_across_segments(dev, decay):
     inp = dgda_inputs(2, 3, 900, seed=5, decay=decay, gates="channel", device=dev, with_state=True)

@@ -34,6 +34,7 @@
  *                                   dense masks and the gate; inline torch code)
  *   maba_hip_maba_sa_prefill_latent the same streams over the latent cache with the
  *                                   absorbed projections
+ *   maba_hip_prefill_union          no counterpart: which of the two forms above pays
  *   maba_hip_dgda_prologue          layers/dgda.py:103-121,186-207 (the DGDA
  *                                   layer's conv + SiLU with carried history,
  *                                   gate activations and key normalisation;
@@ -255,6 +256,14 @@ int maba_hip_maba_sa_prefill_latent(const maba_tensor* q_lat, const maba_tensor*
                                     const maba_tensor* hca, const maba_tensor* idx,
                                     const maba_tensor* gate, float scale, int window, int n_sink,
                                     int block_size, int pool, maba_tensor* out_lat, void* stream);
+
+/*
+ * How far 16 consecutive queries share their selected blocks: the numbers of distinct blocks
+ * (below 16384; all other values count as one) among idx [B,Lq,K] (int64, K <= 64) of every
+ * complete 16 queries of a batch element, summed; out [n] (int32, 1 <= n <= 65535) receives n
+ * parts of the sum.  maba_hip_maba_sa_prefill's time grows with it, the latent form's does not.
+ */
+int maba_hip_prefill_union(const maba_tensor* idx, maba_tensor* out, void* stream);
 
 /*
  * DGDA layer prologue.  xs[0..5]: the q, k, v, alpha, erase and write projections

@@ -521,6 +521,53 @@ __global__ __launch_bounds__(256, NP == 4 ? 2 : 3) void maba_sa_prefill_kernel(P
   }
 }
 
+// How many distinct blocks each 16 consecutive queries list, summed per workgroup: what the choice
+// between this kernel and the latent one goes by.  A wave takes 16 queries at a time and marks
+// their slots in its LDS bitmap; the lane that sets a bit counts it, and afterwards the words it
+// touched are cleared.  Latency-bound: 11 us for the 6.3 MB of indices at T=24571 K=32, where a
+// segmented sort of the 16 K slots (48 us), the compare of neighbours, its sum and their means had
+// the layer's call at 1,111 us, now 1,050.
+struct PfUnionArgs {
+  const int64_t* idx; int64_t isb, ist, isk;
+  int32_t* out;                       // one count per workgroup
+  int64_t gpb, groups;                // 16-query groups per batch element, in all
+  int K;
+};
+
+__global__ __launch_bounds__(256) void prefill_union_kernel(PfUnionArgs a) {
+  __shared__ uint32_t s_bits[4][PF_WORDS + 1];   // the last word: indices that are no block
+  __shared__ int s_sum[4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  uint32_t* bits = s_bits[wave];
+  for (int w = lane; w <= PF_WORDS; w += 64) bits[w] = 0u;
+  __syncthreads();
+  int n = 0;
+  const int slots = 16 * a.K;
+  for (int64_t gi = (int64_t)blockIdx.x * 4 + wave; gi < a.groups; gi += (int64_t)gridDim.x * 4) {
+    const int64_t base = (gi / a.gpb) * a.isb + (gi % a.gpb) * 16 * a.ist;
+    int blk[PF_MAXK / 4];
+#pragma unroll
+    for (int r = 0; r < PF_MAXK / 4; ++r) {   // all loads in flight
+      const int sl = lane + 64 * r;
+      const int64_t v = sl < slots ? a.idx[base + (sl / a.K) * a.ist + (sl % a.K) * a.isk] : -1;
+      blk[r] = sl >= slots ? -1 : v >= 0 && v < PF_WORDS * 32 ? (int)v : PF_WORDS * 32;
+    }
+#pragma unroll
+    for (int r = 0; r < PF_MAXK / 4; ++r)
+      if (blk[r] >= 0) n += (atomicOr(&bits[blk[r] >> 5], 1u << (blk[r] & 31)) >> (blk[r] & 31) & 1u) == 0u;
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int r = 0; r < PF_MAXK / 4; ++r)   // after every mark: a wave's LDS operations stay in order
+      if (blk[r] >= 0) bits[blk[r] >> 5] = 0u;
+    __builtin_amdgcn_wave_barrier();
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
+  if (lane == 0) s_sum[wave] = n;
+  __syncthreads();
+  if (threadIdx.x == 0) a.out[blockIdx.x] = s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3];
+}
+
 static bool pf_rows_ok(const maba_tensor* t, int64_t B, int64_t H, int64_t n, int64_t dh) {
   if (!t || t->ndim != 4 || t->dtype != MABA_BF16) return false;
   if (t->shape[0] != B || t->shape[1] != H || t->shape[2] != n || t->shape[3] != dh) return false;
@@ -612,4 +659,21 @@ extern "C" int maba_hip_maba_sa_prefill(const maba_tensor* q, const maba_tensor*
   if (far(a.kst) || far(a.vst) || far(a.khe) || far(a.vhe)) launch(std::true_type{});
   else launch(std::false_type{});
   return check_launch("maba_sa_prefill");
+}
+
+extern "C" int maba_hip_prefill_union(const maba_tensor* idx, maba_tensor* out, void* stream) {
+  if (!idx || idx->ndim != 3) return fail(MABA_ERR_INVALID, "prefill_union: idx must be [B,Lq,K]");
+  if (!out || out->ndim != 1) return fail(MABA_ERR_INVALID, "prefill_union: out must be 1D");
+  if (idx->dtype != MABA_I64 || out->dtype != MABA_I32)
+    return fail(MABA_ERR_DTYPE, "prefill_union: idx must be int64 and out int32");
+  const int64_t B = idx->shape[0], Lq = idx->shape[1], K = idx->shape[2], n = out->shape[0];
+  if (K < 1 || K > PF_MAXK) return fail(MABA_ERR_UNSUPPORTED, "prefill_union: 1 to %d index slots", PF_MAXK);
+  if (n < 1 || n > 65535 || (n > 1 && out->stride[0] != 1))
+    return fail(MABA_ERR_INVALID, "prefill_union: out must hold 1 to 65535 contiguous counts");
+  PfUnionArgs a;
+  a.idx = (const int64_t*)idx->data; a.isb = idx->stride[0]; a.ist = idx->stride[1]; a.isk = idx->stride[2];
+  a.out = (int32_t*)out->data;
+  a.gpb = Lq / 16; a.groups = B * a.gpb; a.K = (int)K;
+  hipLaunchKernelGGL(prefill_union_kernel, dim3((unsigned)n), dim3(256), 0, (hipStream_t)stream, a);
+  return check_launch("prefill_union");
 }

@@ -461,6 +461,17 @@ def hip_maba_sa_prefill_latent(q_lat, c_kv, hca, idx, gate_logits, scale: float,
     return out
 
 
+def hip_prefill_union(idx) -> torch.Tensor:
+    """The number of distinct blocks each complete 16 consecutive queries of ``idx [B, Lq, K]``
+    (int64) list, summed over them, in int32 parts whose sum is the total."""
+    dev = N.require_device([idx], "prefill_union")
+    groups = idx.shape[0] * (idx.shape[1] // 16)
+    # four groups per workgroup, one round of workgroups
+    out = torch.empty(max(1, min(1024, -(-groups // 4))), dtype=torch.int32, device=dev)
+    N.check(N.load().maba_hip_prefill_union(N.desc(idx), N.desc(out), N.stream_ptr(dev)), "prefill_union")
+    return out
+
+
 def hip_dgda_layer_step(projections, conv_weights, history, state, eps: float = 1e-6, out=None):
     """One decode token of the DGDA layer after its input projection (layers/dgda.py:103-121,
     186-207, then the step of dispatcher.py:330-396) in one launch: ``projections`` are the

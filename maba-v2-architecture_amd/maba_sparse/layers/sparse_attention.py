@@ -299,7 +299,7 @@ class MabaSparseAttention(WeightCacheMixin, nn.Module):
         queries at 32k tokens give 5.1 K, at 64k 6.5 K, at 128k 7.6 K), and neighbouring queries
         of a trained or randomly initialised model select nearly the same blocks (about 3 K, where
         the head-space kernel is 2.5 times faster).  The union is counted on the GPU from ``idx``
-        (one segmented sort); ``self.prefill_form`` may force either."""
+        (``hip_prefill_union``; elsewhere one segmented sort); ``self.prefill_form`` may force either."""
         if self.prefill_form != "auto":
             return self.prefill_form
         B, Lq, K = idx.shape
@@ -307,6 +307,10 @@ class MabaSparseAttention(WeightCacheMixin, nn.Module):
             return "heads"
         if Lq < 16:
             return "latent"
+        if idx.device.type == "cuda" and get_backend(idx.device) == "hip" and K <= 64:
+            from maba_sparse.kernels import hip_backend as hb
+            distinct = sum(hb.hip_prefill_union(idx).tolist()) / max(1, B * (Lq // 16))
+            return "heads" if distinct < self.prefill_union_limit * K else "latent"
         grp = idx[:, : (Lq // 16) * 16].reshape(B, Lq // 16, 16 * K).sort(dim=-1).values
         distinct = (grp[..., 1:] != grp[..., :-1]).sum(dim=-1).float().mean().item() + 1.0
         return "heads" if distinct < self.prefill_union_limit * K else "latent"

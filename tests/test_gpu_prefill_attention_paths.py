@@ -64,3 +64,19 @@ def test_far_rows(dev):
     want = _hip().hip_maba_sa_prefill(*args, scale=0.125)
     args[1] = far
     assert torch.equal(_hip().hip_maba_sa_prefill(*args, scale=0.125), want)
+
+
+@pytest.mark.parametrize("B,Lq,K,nb", [(1, 16, 1, 1), (1, 31, 32, 40), (2, 200, 64, 16384), (3, 77, 5, 33), (1, 70000, 7, 900)])
+def test_prefill_union_counts(dev, B, Lq, K, nb):
+    """Distinct blocks per 16 queries, dense and permuted index strides, more groups than one
+    round of workgroups, and values that are no block (counted as one)."""
+    from maba_sparse.kernels import hip_backend as hb
+    g = torch.Generator().manual_seed(B + Lq)
+    idx = torch.randint(0, nb, (B, Lq, K), generator=g)
+    idx[:, 3::16, 0] = nb - 1
+    if Lq == 77:
+        idx[:, ::5, 1] = -1
+    want = sum(len(set(r)) for r in idx[:, : Lq // 16 * 16].reshape(-1, 16 * K).tolist())
+    d = idx.to(dev)
+    assert sum(hb.hip_prefill_union(d).tolist()) == want
+    assert sum(hb.hip_prefill_union(d.permute(2, 0, 1).contiguous().permute(1, 2, 0)).tolist()) == want

@@ -35,7 +35,7 @@ from maba_sparse.layers.indexer import DGIndexer, _Growing
 
 # Fused prefill: the head-space kernel is taken while 16 consecutive queries list fewer than
 # this many distinct blocks, in units of top_k (the measured crossover with the latent kernel)
-PREFILL_UNION_LIMIT = 5.25
+PREFILL_UNION_LIMIT = 6.9
 
 
 class LatentCache:
@@ -295,10 +295,11 @@ class MabaSparseAttention(WeightCacheMixin, nn.Module):
         blocks, staged once per tile and computed by each 16-query wave that lists it (16
         queries share every key tile, per head).  Its cost grows with the union of 16
         consecutive queries' blocks, the latent kernel's does not: measured at 10 heads of 64,
-        d_c 128, top-32, the two are equal near 5.25 K distinct blocks per 16 queries (random
-        queries at 32k tokens give 5.1 K, at 64k 6.5 K, at 128k 7.6 K), and neighbouring queries
-        of a trained or randomly initialised model select nearly the same blocks (about 3 K, where
-        the head-space kernel is 2.5 times faster).  The union is counted on the GPU from ``idx``
+        d_c 128, top-32 (heads / latent, ms): random queries at 32k tokens, 5.1 K distinct blocks
+        per 16 queries, 2.83 / 4.05; at 64k, 6.5 K, 7.63 / 8.52; at 128k, 7.6 K, 21.2 / 18.8, and
+        with queries partly alike, 4.9 K, 11.0 / 18.8, so the two are equal near 7 K.  Neighbouring
+        queries of a trained or randomly initialised model select nearly the same blocks (about 3 K).
+        The union is counted on the GPU from ``idx``
         (``hip_prefill_union``; elsewhere one segmented sort); ``self.prefill_form`` may force either."""
         if self.prefill_form != "auto":
             return self.prefill_form
@@ -364,7 +365,7 @@ class MabaSparseAttention(WeightCacheMixin, nn.Module):
             early = heads(self.v_up_proj(cm[:, off: off + n_early]), n_early)
         return dispatch_maba_sa_prefill(q, k, v, kh, vh, early, idx, self.stream_gate(x), scale=self.scale,
                                         window=self.window_size, n_sink=self.n_sink_tokens,
-                                        block_size=self.block_size, pool=r)
+                                        block_size=self.block_size, pool=r, token_major=True)
 
     # ------------------------------------------------------------ prefill (dense)
     def _dense_streams(self, x, q, c_full, idx):

@@ -62,10 +62,10 @@
 // element.  A lane loads the seven rows its four tokens' taps cover.
 #pragma once
 #include "dgda_common.h"
+#include "dgda_rows.h"
 
 namespace maba {
 
-constexpr int SC = 16;                   // tokens per sub-chunk
 constexpr int SUB_MAX_SEG = 2048;         // segments per sequence at most
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr float SUB_MFMA_RANGE = 64.f * LOG2E;   // largest |Lam| within a sub-chunk on the MFMA path, in log2 units
@@ -277,16 +277,15 @@ __device__ __forceinline__ int sub_run(const SubArgs& a, SubSmem<PRO, DK>& sm, i
       rows(4, xg[1], 0, integral_constant<int, 4>{});
       if (!MAP) rows(5, xg[2], 0, integral_constant<int, 4>{});
     } else {
-      const int last = a.L - 1 - t0;
       const char* bk = base(a.k, a.ks0, a.ks1, a.ks2, ES, t0);
       const char* bv = base(a.vp, a.vs0, a.vs1, a.vs2, ES, t0);
       const char* bg = base(a.gp, a.gs0, a.gs1, a.gs2, EG, t0);
       const char* bb = base(a.bp, a.bs0, a.bs1, a.bs2, EG, t0);
       const char* bw = base(a.wp, a.ws0, a.ws1, a.ws2, EG, t0);
       auto rows = [&](const char* p, int S, int chb, auto& x, auto load) {
-        const int lane0 = 4 * g * S + chb, end = last * S + chb;
+        const uint32_t lane0 = 4 * g * S + chb, end = row_end(a.L - 1 - t0, SC - 1, S, chb);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) x[i] = load(p + (uint32_t)min(lane0 + i * S, end));
+        for (int i = 0; i < 4; ++i) x[i] = load(p + row_offset(lane0, i, S, end));
       };
       auto lk = [](const char* p) { return load_row<F32IN, NKT>(p); };
       auto lv = [](const char* p) { return load_row<F32IN, NVT>(p); };

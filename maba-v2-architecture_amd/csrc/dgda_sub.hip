@@ -15,7 +15,7 @@ static bool fits32s(const maba_tensor* t) {
     if (t->stride[d] < 0 || t->stride[d] > INT32_MAX) return false;
   return true;
 }
-// the kernels address the 16 rows of a sub-chunk with 32-bit byte offsets
+// the kernels address the 16 rows of a sub-chunk with 32-bit byte offsets (row_end)
 static bool rows_fit(int64_t row_stride) { return row_stride <= (INT32_MAX - 4096) / (SC * 4); }
 // gate with channel stride 0 (per token) or 1 (per channel, 16-byte aligned rows), fp32 or
 // (16-bit q, k, v) in q's dtype

@@ -129,3 +129,18 @@ def test_layer_strong_decay_gates(dev):
     eo, eS = odgda.dgda_prefill_seq(*(t[:, None] for t in (q, k, v)), alpha=np.exp(la)[:, None], b=b[:, None], w=w[:, None])
     assert_close(o.float().view(1, 300, 1, 64).transpose(1, 2), eo, 1e-2, 1e-2, "out")   # bf16 output
     assert_close(S, eS, 2e-3, 2e-3, "state")
+
+
+def test_rows_beyond_32_bits(dev):
+    """600 tokens 4 MiB apart: the sequence's bytes leave 32 bits, a sub-chunk's do not."""
+    inp = dgda_inputs(1, 2, 600, seed=4, decay="slow", gates="channel", qkv_dtype=torch.float32, device=dev)
+    buf = torch.empty(600, 1 << 20, device=dev)
+    far = {}
+    for i, n in enumerate(("q", "k", "v", "log_alpha", "b", "w")):
+        far[n] = buf[:, 128 * i: 128 * (i + 1)].view(1, 600, 2, 64).transpose(1, 2)
+        far[n].copy_(inp[n])
+    best = _sizes(inp)[1]
+    assert _sizes(far)[1] == best > 16   # the same kernel and cut
+    o, S = _call(inp, best)
+    o2, S2 = _call(far, best)
+    assert torch.equal(o, o2) and torch.equal(S, S2)

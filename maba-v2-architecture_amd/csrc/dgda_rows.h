@@ -13,7 +13,8 @@ constexpr int SC = 16;   // tokens per sub-chunk
 constexpr uint32_t row_end(int left, int most, int step, int first) {
   return (uint32_t)(left < most ? left : most) * (uint32_t)step + (uint32_t)first;
 }
-// Offset of row `row` after the lane's first one, at most `end`.
+// Offset of row `row` after the lane's first one, at most `end`; a row before the base (the fused
+// layer's conv taps ahead of token 0) wraps and is `end` too.
 constexpr uint32_t row_offset(uint32_t lane0, int row, int step, uint32_t end) {
   return lane0 + (uint32_t)(row * step) < end ? lane0 + (uint32_t)(row * step) : end;
 }

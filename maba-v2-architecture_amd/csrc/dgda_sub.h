@@ -256,18 +256,18 @@ __device__ __forceinline__ int sub_run(const SubArgs& a, SubSmem<PRO, DK>& sm, i
   Row<!G16, NKT> pg[4], pb[4];
   Row<!G16, NVT> pw[4];
   Row<false, 4> tq[7], tk[7], tv[7], xg[3][4];   // fused prologue: rows 4g-3 .. 4g+3, and the gate rows
-  // rows past the end re-read the last one, rows before the first (replaced by the history) the first
+  // rows past the end re-read the last one, as do rows before the first (replaced by the history)
   auto prefetch = [&](int cc) {
     const int t0 = cc * SC;
     if constexpr (PRO) {
-      const int d = min(t0, 3), last = a.L - 1 - (t0 - d);   // rows are counted from token t0 - d
+      const int d = min(t0, 3);   // rows are counted from token t0 - d
       auto rows = [&](int s, auto& x, int m0, auto n_c) {
         const char* p = base(a.px[s], a.pxs0[s], 0, a.pxs1[s], 2, t0 - d);
         const int S = 2 * a.pxs1[s], chb = 2 * (hi * 64 + kch);
-        const int lane0 = 4 * g * S + chb, end = last * S + chb;
+        const uint32_t lane0 = 4u * g * S + chb, end = row_end(a.L - 1 - (t0 - d), SC - 1 + d, S, chb);
 #pragma unroll
         for (int m = 0; m < decltype(n_c)::value; ++m)
-          x[m] = load_row<false, 4>(p + (uint32_t)max(min(lane0 + (m + m0 + d) * S, end), chb));
+          x[m] = load_row<false, 4>(p + row_offset(lane0, m + m0 + d, S, end));
       };
       using std::integral_constant;
       if (!MAP) rows(0, tq, -3, integral_constant<int, 7>{});

@@ -194,7 +194,7 @@ extern "C" int maba_hip_dgda_layer_prefill(const maba_tensor* const* xs, const m
         ((uintptr_t)t->data & 7) || t->stride[0] % 4 || t->stride[1] % 4 || !fits32s(t))
       return fail(MABA_ERR_UNSUPPORTED, "dgda_layer_prefill: projections must be bf16 [B,L,C], unit channel "
                   "stride, 8-byte aligned rows");
-    // the kernels address a sequence's rows with 32-bit offsets
+    // the kernels address the 19 rows under a sub-chunk's conv taps with 32-bit byte offsets
     if ((L + SC) * t->stride[1] + C > INT32_MAX)
       return fail(MABA_ERR_UNSUPPORTED, "dgda_layer_prefill: L * row stride must stay below 2^31 elements");
   }

@@ -144,3 +144,17 @@ def test_rows_beyond_32_bits(dev):
     o, S = _call(inp, best)
     o2, S2 = _call(far, best)
     assert torch.equal(o, o2) and torch.equal(S, S2)
+
+
+def test_layer_rows_beyond_32_bits(dev):
+    """600 tokens of projections 4 MiB apart: their bytes leave 31 bits, their elements do not."""
+    from maba_sparse.kernels import hip_backend as hb
+    g = torch.Generator().manual_seed(6)
+    x = torch.randn(1, 600, 6 * 64, generator=g).bfloat16().to(dev)
+    convs = [torch.randn(64, 1, 4, generator=g).bfloat16().to(dev) for _ in range(3)]
+    far = torch.empty(600, 1 << 21, dtype=torch.bfloat16, device=dev)[None, :, : 6 * 64]
+    far.copy_(x)
+    want = hb.hip_dgda_layer_prefill(x.split(64, dim=-1), convs)
+    got = hb.hip_dgda_layer_prefill(far.split(64, dim=-1), convs)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    assert all(torch.equal(a, b) for a, b in zip(got[2], want[2]))

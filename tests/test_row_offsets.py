@@ -39,3 +39,25 @@ def test_op_rows(rows, L, stride, es):
             for g in range(4):
                 for i in range(4):
                     assert rows(left, SC - 1, step, first, 4 * g, i) == min(4 * g + i, left) * step + first
+
+
+@pytest.mark.parametrize("L,stride", [(400_000, 3840), (559_000, 3840), (600, 1 << 21), (300_000, 640), (16, (1 << 31) // 33),
+                                      (5, (1 << 31) // 22), (1, (1 << 31) // 18), (1, 3840)])
+def test_layer_rows(rows, L, stride):
+    """The fused layer's seven rows per lane, three of them taps, up to its limit on L * stride."""
+    C = 640
+    stride = stride // 4 * 4
+    assert (L + SC) * stride + C <= 2 ** 31 - 1
+    step, first = 2 * stride, 2 * (C - 4)
+    n = -(-L // SC)
+    for sc in {0, n - 1, n // 2, min(1, n - 1)}:
+        d = min(sc * SC, 3)
+        left = L - 1 - (sc * SC - d)
+        for g in range(4):
+            for m in range(7):
+                r = 4 * g + m - 3 + d
+                got = rows(left, SC - 1 + d, step, first, 4 * g, r - 4 * g)
+                if r < 0:   # replaced by the history: some row of the sequence
+                    assert got % step == first and got // step <= left
+                else:
+                    assert got == min(r, left) * step + first

@@ -69,7 +69,8 @@ def assert_close(actual, expected, rtol, atol, what=""):
     a = actual.detach().double().cpu().numpy() if isinstance(actual, torch.Tensor) else np.asarray(actual, np.float64)
     e = np.asarray(expected, np.float64)
     assert a.shape == e.shape, f"{what}: shape {a.shape} vs {e.shape}"
-    bad = np.abs(a - e) > atol + rtol * np.abs(e)
+    # a NaN (or an infinity) where the other side has none is outside every tolerance
+    bad = ~((np.isfinite(e) & (np.abs(a - e) <= atol + rtol * np.abs(e))) | (a == e) | (np.isnan(a) & np.isnan(e)))
     if bad.any():
         i = np.unravel_index(np.argmax(np.abs(a - e) - rtol * np.abs(e)), a.shape)
         raise AssertionError(

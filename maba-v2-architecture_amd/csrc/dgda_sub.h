@@ -907,7 +907,7 @@ __global__ __launch_bounds__(64, 1) void dgda_sub_scan_kernel(SubArgs a) {
   __shared__ uint8_t alive[SUB_MAX_SEG];
   int any = 0;
   for (int k = threadIdx.x; k < kend; k += blockDim.x) {
-    alive[k] = k >= 1 && (zc[2 * k] < 0 || zc[2 * k + 1] < 0);
+    alive[k] = k < 1 ? 0 : (zc[2 * k] < 0 ? 1 : 0) | (zc[2 * k + 1] < 0 ? 2 : 0);   // M's column halves
     any |= alive[k];
   }
   if (!__syncthreads_or(any)) return;
@@ -934,7 +934,20 @@ __global__ __launch_bounds__(64, 1) void dgda_sub_scan_kernel(SubArgs a) {
   for (int d = 0; d < DEPTH; ++d) load(buf[d], 1 + d);
   // The step is straight-line code (a vanished slot's products are dropped and its N stored
   // back), so that the wait for one slot's loads is not a wait for the later slots'.
-  auto step = [&](Slot& b, int k, bool alive) {
+  auto step = [&](Slot& b, int k, int alive) {
+    if constexpr (DK == 128) {
+      // one half of M's columns vanished: its wave stored nothing there
+      if (alive == 1 || alive == 2) {
+        const bool drop = alive == (g < 2 ? 2 : 1);   // lane groups 0, 1 hold columns 0 .. 63
+#pragma unroll
+        for (int kt = 0; kt < NKT; ++kt)
+#pragma unroll
+          for (int p = 0; p < NP; ++p) {
+            b.mh[kt][p] = drop ? i16x8{} : b.mh[kt][p];
+            b.ml[kt][p] = drop ? i16x8{} : b.ml[kt][p];
+          }
+      }
+    }
     i16x8 sh[NP], sl[NP];
 #pragma unroll
     for (int p = 0; p < NP; ++p) {

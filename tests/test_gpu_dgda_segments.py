@@ -131,6 +131,20 @@ def test_layer_strong_decay_gates(dev):
     assert_close(S, eS, 2e-3, 2e-3, "state")
 
 
+@pytest.mark.parametrize("fast", [0, 64])
+@pytest.mark.parametrize("per_token", [-3.0, -200.0])
+def test_transition_that_vanishes_by_half(dev, fast, per_token):
+    """d_k = 128: the transition's columns of one half of the channels vanish, the other half's do
+    not.  Two waves form a map, and the one whose columns vanish stores nothing."""
+    inp = dgda_inputs(1, 2, 1300, dk=128, dv=64, seed=11, decay="slow", gates="channel", device=dev, with_state=True)
+    inp["log_alpha"][..., fast: fast + 64] = per_token
+    eo, eS = odgda.dgda_prefill_seq(**oracle_dgda_args(inp))
+    for nbytes in _sizes(inp):
+        o, S = _call(inp, nbytes, s0=inp["initial_state"])
+        assert_close(o, eo, 2e-3, 2e-3, f"out {nbytes}")
+        assert_close(S, eS, 2e-3, 2e-3, f"state {nbytes}")
+
+
 def test_rows_beyond_32_bits(dev):
     """600 tokens 4 MiB apart: the sequence's bytes leave 32 bits, a sub-chunk's do not."""
     inp = dgda_inputs(1, 2, 600, seed=4, decay="slow", gates="channel", qkv_dtype=torch.float32, device=dev)

@@ -30,7 +30,10 @@
 //  * the running reference m of a query moves only when a score passes it by 2^8 (the sums
 //    hold that easily in fp32); only then do lanes exchange maxima and the sums rescale;
 //  * a key's weight is folded into the exponent as its log2, so an unlisted block is a bias of
-//    -inf and a block listed once costs nothing;
+//    -inf and a block listed once costs nothing.  Where that score is infinite or NaN the sum is
+//    NaN; the tile's largest score is therefore taken with the maximum that carries NaN, and only
+//    a tile that has one masks its rows with selects (no cost per score: v_maximum3_f32, two
+//    scores each, 2.67 -> 2.60 ms at the first size below against fmaxf);
 //  * the probabilities' sum is a product with a row of ones, on the matrix unit;
 //  * which union entries a query lists is a row of bits in LDS, one word per 32 entries, in
 //    place of comparing the entry with all of the query's slots (which remains for unions
@@ -342,31 +345,40 @@ __global__ __launch_bounds__(256, NP == 4 ? 2 : 3) void maba_sa_prefill_kernel(P
       sc[rb] = acc;
     }
     // lane (query c16, g) holds the scores of keys 16 rb + 4 g + i; x: relative to the reference
+    auto drop = [&]() {   // the rows without weight, one by one
+      uint32_t vm = vmask;
+      asm volatile("" : "+v"(vm));   // the bit tests stay in the callers' branches
+#pragma unroll
+      for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[rb][i] = ((vm >> (4 * rb + i)) & 1u) ? x[rb][i] : -INFINITY;
+    };
     auto relative = [&]() {
       const float bias = lw == -INFINITY ? -INFINITY : st.m == -INFINITY ? lw : lw - st.m;
 #pragma unroll
       for (int rb = 0; rb < 4; ++rb)
 #pragma unroll
         for (int i = 0; i < 4; ++i) x[rb][i] = fmaf(sc[rb][i], sl2, bias);
-      if (part) {
-        uint32_t vm = vmask;
-        asm volatile("" : "+v"(vm));   // the bit tests stay in this branch
-#pragma unroll
-        for (int rb = 0; rb < 4; ++rb)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) x[rb][i] = ((vm >> (4 * rb + i)) & 1u) ? x[rb][i] : -INFINITY;
-      }
+      if (part) drop();
     };
-    auto largest = [&]() {
+    auto largest = [&](auto max2) {
       float mx = -INFINITY;
 #pragma unroll
-      for (int rb = 0; rb < 4; ++rb) mx = fmaxf(fmaxf(mx, fmaxf(x[rb][0], x[rb][1])), fmaxf(x[rb][2], x[rb][3]));
+      for (int rb = 0; rb < 4; ++rb)
+        mx = max2(max2(max2(max2(mx, x[rb][0]), x[rb][1]), x[rb][2]), x[rb][3]);
       return mx;
     };
     relative();
-    const float mx = largest();
-    if (__ballot(mx > PF_SLACK || (st.m == -INFINITY && lw != -INFINITY)) != 0ull) {
-      // some query's reference moves: to the largest score so far, in all of its lanes
+    float mx = largest([](float p, float q) { return __builtin_elementwise_maximum(p, q); });   // NaN if any x is
+    if (__ballot(!(mx <= PF_SLACK) || (st.m == -INFINITY && lw != -INFINITY)) != 0ull) {
+      // Some query's reference moves: to the largest score so far, in all of its lanes.  Or a score
+      // is NaN: of a query that weights the row, whose result it is, or an infinity (or NaN) that the
+      // bias of -inf did not take away from the other queries, which the rows' masks then do.
+      const bool nan = __ballot(mx != mx) != 0ull;
+      if (nan) {
+        drop();
+        mx = largest([](float p, float q) { return fmaxf(p, q); });   // a NaN moves no reference
+      }
       const float base = st.m == -INFINITY ? 0.f : st.m;
       float top = lw == -INFINITY ? -INFINITY : mx - lw + base;
       top = group_max(top);
@@ -377,6 +389,7 @@ __global__ __launch_bounds__(256, NP == 4 ? 2 : 3) void maba_sa_prefill_kernel(P
 #pragma unroll
       for (int dt = 0; dt < NDT; ++dt) st.z[dt] *= corr;
       relative();
+      if (nan) drop();
     }
     i16x4 ph[4], pl[4];
 #pragma unroll

@@ -53,6 +53,28 @@ def test_references_that_move(dev, scale, dup):
     _check(dev, case, scale, f"scale {scale}")
 
 
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("channels", [1, 64])
+@pytest.mark.parametrize("scale", [0.125, -0.125])
+@pytest.mark.parametrize("dup", [False, True])
+def test_non_finite_key_stays_with_its_block(dev, bad, channels, scale, dup):
+    """A key whose scores are infinite (either sign) or NaN changes nothing for the queries that do
+    not list its block."""
+    case = list(_case(1, 2, 150, 1000, 64, 4, 8, dup=dup))
+    if not dup:
+        case[6] = _distinct(1, 150, 16, 4, 5)
+    q, k, v, kh, vh, early, idx, gate = case
+    others = (idx[0] != 5).all(dim=-1).nonzero()[:, 0]   # block 5 is outside every query's window too
+    assert 50 < others.numel() < 150
+    exp = osa.maba_sa_prefill_heads(*(to_np(t) if t is not None else None for t in (q, k, v, kh, vh, early)), idx.numpy(),
+                                    to_np(gate), window=128, n_sink=4, scale=scale)
+    case[1] = k.clone()
+    case[1][:, :, 5 * 64 + 7, :channels] = bad
+    d = lambda t: None if t is None else t.to(dev)  # noqa: E731
+    out = _hip().hip_maba_sa_prefill(*(d(t) for t in case), scale=scale, out_dtype=torch.float32)
+    assert_close(out[:, :, others.to(dev)], exp[:, :, others.numpy()], 2e-3, 2e-3, f"{bad} {channels}")
+
+
 def test_far_rows(dev):
     """Key rows 2^23 elements apart."""
     q, k, v, kh, vh, early, idx, gate = _case(1, 1, 70, 70, 64, 2, 9)

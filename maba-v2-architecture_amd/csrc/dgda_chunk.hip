@@ -14,7 +14,7 @@
 //
 // Sequence parallelism (only B*H = 40 recurrences at the BASELINE shape, but
 // 256 CUs): the (b,h)-major sequence of all B*H*nchunks chunks is cut into slots
-// of U chunks, U = max(CPS_FINE, ceil(total / (2 * CUs))), so that the output pass runs
+// of U chunks, at least ceil(total / (2 * CUs)) (see fine_slot), so that the output pass runs
 // exactly one wave of workgroups (two per CU) of equal length.  A segment is the
 // part of one (b,h) sequence inside one slot; each (b,h) has up to nseg_max.
 //   pass 1 (dgda_chunk_kernel<AGG>) runs every segment but the first of each (b,h)
@@ -40,6 +40,8 @@
 // A operand is read from LDS at the matching two column groups.  Raw bf16 inputs
 // are exact MFMA operands; fp32 operands (S, u, L, A, T) are split into bf16
 // hi + lo parts (two or three MFMAs) so products carry ~16 mantissa bits.
+#include <algorithm>
+
 #include "dgda_common.h"
 
 namespace maba {
@@ -65,10 +67,10 @@ constexpr float ZC_CONTRACT = 1.99f;
 // the true initial state and every segment with zc[s] >= 0 from a zero start,
 // writing all their outputs and their final states N_s (the true final state for
 // segment 0); N_s is then exact wherever s = 0 or zc[s] >= 0.  OUT_FIX (one
-// workgroup per segment s >= 1) re-runs the first zc[s] chunks of those segments
-// from the true start state, and every segment whose M never vanished in full; it
-// forms its start state itself from the last exact N_j and the maps (M, N) of the
-// segments between.
+// workgroup per slot, which ends at once where the slot starts a sequence) re-runs the
+// first zc[s] chunks of the segments s >= 1 from the true start state, and every segment
+// whose M never vanished in full; it forms its start state itself from the last exact
+// N_j and the maps (M, N) of the segments between.
 // With fast decay zc[s] is 1 or 2, so the aggregate and fix-up passes shrink to a
 // chunk or two per segment.  With one segment per (b,h) only OUT_ZERO runs.
 constexpr int OUT_ZERO = 1, OUT_FIX = 2;
@@ -765,18 +767,34 @@ static size_t chunk_geom_bytes(const SlotGeom& gm, int64_t BH) {
   return (size_t)(nseg * 64 * 128) * sizeof(float) + (size_t)nseg * sizeof(int);
 }
 
-// Slots of CPS chunks at least, or of CPS_FINE where the workspace holds that many segments: a
-// workgroup takes about 4.6 us per chunk however few there are, so slots of 16 chunks leave an
-// idle chip waiting for them (CPS 16 -> 4, us, decay that vanishes / that remembers: B=1 H=10
-// T=2048 85 -> 38 / 211 -> 79; B=2 T=5000 92 -> 51 / 218 -> 156; B=2 T=10007 93 -> 66 /
-// 228 -> 198; B=4 T=8192 105 -> 80 / 330 -> 240; no change at T=32768).  2 measured as 4 where
-// maps vanish and slower with many surviving ones (B=1 T=5000 161 against 100), 8 slower.
+// Chunks per slot with the preferred workspace.  A workgroup takes about 4.6 us per chunk however
+// few there are, so slots of 16 chunks leave an idle chip waiting for them: CPS_FINE, or what
+// fills two workgroups per CU.  But where maps survive, a segment's fix-up workgroup applies those
+// before it one after the other (2.4 us each, more with two workgroups per CU), so a sequence is
+// cut less where that walk gets long: beyond WALK segments to one workgroup per CU (where slots of
+// CPS would be), and never into more than WALK_MAX while CPS does not cut it so either.
+// H heads, T tokens, us with slots of CPS / of CPS_FINE without these bounds / of this rule, decay
+// that remembers (and that vanishes):
+//   H=10 T=2048 207 / 77 / 77 (85 / 35 / 35)       H=16 T=8192 225 / 203 / 141 (86 / 46 / 53)
+//   H=8 T=16384 239 / 321 / 171 (86 / 47 / 53)     H=8 T=32768 270 / 390 / 270 (87 / 67 / 87)
+//   H=4 T=32768 269 / 561 / 231 (86 / 47 / 53)     H=1 T=131072 450 / 1511 / 448 (86 / 48 / 86)
+// CPS_FINE of 2 measured as 4 where maps vanish and slower with many surviving ones (H=10 T=5000
+// 161 against 100), 8 slower.
+constexpr int WALK = 24, WALK_MAX = 64;
+static int64_t fine_slot(int64_t BH, int64_t nch) {
+  const int64_t cus = device_cu_count();
+  int64_t U = std::max<int64_t>(CPS_FINE, ceil_div(BH * nch, 2 * cus));
+  if (U >= CPS || ceil_div(nch, U) <= WALK) return U;
+  if (ceil_div(BH * nch, cus) <= CPS) U = std::max(U, ceil_div(BH * nch, cus));
+  return std::max(U, std::min<int64_t>(CPS, ceil_div(nch, WALK_MAX)));
+}
+
 // A sequence that CPS leaves whole is cut where that costs nothing even if every map survives
 // and each segment runs twice: from 15 chunks (B=4 T=1000 75 -> 38 / 75 -> 71, but 11 chunks
 // 53 -> 39 / 53 -> 68), and while each slot has a CU (B=8 T=1000, 320 slots: 75 -> 46 / 75 -> 104).
 static SlotGeom chunk_geom(int64_t BH, int64_t L, size_t ws_bytes) {
   const int64_t nch = ceil_div(L, CH) > 0 ? ceil_div(L, CH) : 1;
-  const SlotGeom coarse = slot_geom(BH, nch, CPS), fine = slot_geom(BH, nch, CPS_FINE);
+  const SlotGeom coarse = slot_geom(BH, nch, CPS), fine = slot_geom(BH, nch, fine_slot(BH, nch));
   const bool pays = coarse.nseg_max > 1 ||
                     (nch > SHORT_CHUNKS && ceil_div(BH * nch, fine.U) <= device_cu_count());
   return pays && chunk_geom_bytes(fine, BH) <= ws_bytes ? fine : coarse;

@@ -52,7 +52,7 @@ def test_segments_follow_the_workspace(dev, dk, dv, decay):
 
 
 @pytest.mark.parametrize("B,H,L", [(1, 1, 14 * 64), (1, 2, 14 * 64 + 1), (2, 3, 16 * 64), (3, 1, 16 * 64 + 1), (1, 3, 2100),
-                                   (65, 1, 1000)])
+                                   (65, 1, 1000), (1, 1, 300 * 64), (1, 10, 7000)])
 @pytest.mark.parametrize("decay", ["baseline", "slow"])
 def test_chunk_segments_follow_the_workspace(dev, B, H, L, decay):
     """Per-token gates: slots of four chunks with the preferred workspace, of sixteen with any

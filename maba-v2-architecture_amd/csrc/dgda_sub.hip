@@ -4,6 +4,7 @@
 #include "dgda_sub.h"
 
 #include <algorithm>
+#include <cmath>
 
 namespace maba {
 
@@ -62,6 +63,14 @@ constexpr int64_t SUB_MIN_LEN = 5;
 // (B=4 H=10 T=32768 per-channel bf16: 436 us against 470), and twice as many segments cost
 // their re-runs (the fused layer at B=1 T=32768, 10 sub-chunks each: 493 us against 412).
 constexpr int64_t SUB_LEN_2 = 32;
+// Segments per sequence at most, in units of the square root of its sub-chunks.  Where transitions
+// survive the scan takes a step per segment (0.7 us at d_k = 64, 9 at 128), and every sub-chunk is
+// run twice, so few heads over a long sequence are not cut until every SIMD has a wave.  One head,
+// without / with this bound / at 3, us, decay that remembers (and that vanishes): d_k = 64 T=131072
+// 943 / 584 / 465 (86 / 95 / 136), T=32768 398 / 284 / 235 (56 / 57 / 78); d_k = 128 T=65536 1953 /
+// 1513 / 1015 (160 / 146 / 172); the fused layer T=65536 771 / 451 / 418 (770 / 147 / 202: without
+// it segments end before their transitions vanish).
+constexpr double SUB_SEG_ROOT = 6;
 
 static int64_t sub_chunks(int64_t L) { return ceil_div(L, SC); }
 static size_t sub_slot_bytes(int64_t dk, int64_t dv) { return (size_t)(dk * (dv + dk)) * sizeof(float) + 2 * sizeof(int); }
@@ -71,10 +80,10 @@ struct SubCut { int nseg, seglen, cols; };
 
 // As many segments as fill one wave per SIMD, or two (see SUB_LEN_2; always at d_k = 32, whose
 // waves hold a quarter of the state, never at d_k = 128, whose state leaves registers for one),
-// and no more than the workspace holds.  Where that leaves half the SIMDs without work a wave
-// takes 32 columns instead of 64 (narrow; not in the fused layer, whose staging is most of a
-// sub-chunk): the key side is done twice, but a sub-chunk takes a wave less time (B=2 H=10
-// bf16: T=160 54 -> 37 us, T=1000 57 -> 48 us).
+// no more than SUB_SEG_ROOT lets a scan walk, and no more than the workspace holds.  Where that
+// leaves half the SIMDs without work a wave takes 32 columns instead of 64 (narrow; not in the fused
+// layer, whose staging is most of a sub-chunk): the key side is done twice, but a sub-chunk takes a
+// wave less time (B=2 H=10 bf16: T=160 54 -> 37 us, T=1000 57 -> 48 us).
 static SubCut sub_cut(int64_t BH, int64_t L, int64_t dk, int64_t dv, size_t ws_bytes, bool narrow) {
   const int64_t nch = sub_chunks(L);
   const int64_t simds = 4 * (int64_t)device_cu_count();
@@ -82,6 +91,8 @@ static SubCut sub_cut(int64_t BH, int64_t L, int64_t dk, int64_t dv, size_t ws_b
   const bool two = dk == 32 || (dk == 64 && nch * waves >= SUB_LEN_2 * 2 * simds);
   int64_t n = (two ? 2 : 1) * simds / waves;
   if (n > ceil_div(nch, SUB_MIN_LEN)) n = ceil_div(nch, SUB_MIN_LEN);
+  const int64_t most = (int64_t)(SUB_SEG_ROOT * std::sqrt((double)nch));
+  if (n > most) n = most;
   const int64_t fit = (int64_t)(ws_bytes / ((size_t)(BH > 0 ? BH : 1) * sub_slot_bytes(dk, dv)));
   if (n > fit) n = fit;
   if (n > SUB_MAX_SEG) n = SUB_MAX_SEG;

@@ -39,3 +39,11 @@ def test_chunk_cut_is_bounded(BH):
 def test_chunk_cut_where_walks_are_short():
     """Two heads' short prompts are still cut into slots of four chunks."""
     assert _chunk_segments(20, 2048) == 9 and _chunk_segments(40, 1500) == 7
+
+
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("BH", [1, 2, 4, 10, 40, 160])
+def test_sub_chunk_cut_is_bounded(BH, d):
+    for T in (100, 1000, 4096, 10007, 32768, 131072, 1 << 20, 1 << 24):
+        n = _nbytes(1, BH, T, d, "channel", "preferred") / (BH * (d * 2 * d * 4 + 8))
+        assert n <= 6 * (-(-T // 16)) ** 0.5, f"{T} tokens"

@@ -255,27 +255,30 @@ __device__ __forceinline__ int sub_run(const SubArgs& a, SubSmem<PRO, DK>& sm, i
   Row<F32IN, NVT> pv[4];
   Row<!G16, NKT> pg[4], pb[4];
   Row<!G16, NVT> pw[4];
-  Row<false, 4> tq[7], tk[7], tv[7], xg[3][4];   // fused prologue: rows 4g-3 .. 4g+3, and the gate rows
+  // fused prologue: rows 4g-3 .. 4g+3 of q, k, v, and the gates' rows (key side, value side)
+  Row<false, 4> tq[7], tk[7], xg[2][4];
+  Row<false, NVT> tv[7], xw[4];
   // rows past the end re-read the last one, as do rows before the first (replaced by the history)
   auto prefetch = [&](int cc) {
     const int t0 = cc * SC;
     if constexpr (PRO) {
       const int d = min(t0, 3);   // rows are counted from token t0 - d
-      auto rows = [&](int s, auto& x, int m0, auto n_c) {
+      auto rows = [&](int s, auto& x, int ch, int m0, auto n_c) {
+        constexpr int N = sizeof(x[0]) / 2;
         const char* p = base(a.px[s], a.pxs0[s], 0, a.pxs1[s], 2, t0 - d);
-        const int S = 2 * a.pxs1[s], chb = 2 * (hi * 64 + kch);
+        const int S = 2 * a.pxs1[s], chb = 2 * (hi * 64 + ch);
         const uint32_t lane0 = 4u * g * S + chb, end = row_end(a.L - 1 - (t0 - d), SC - 1 + d, S, chb);
 #pragma unroll
         for (int m = 0; m < decltype(n_c)::value; ++m)
-          x[m] = load_row<false, 4>(p + row_offset(lane0, m + m0 + d, S, end));
+          x[m] = load_row<false, N>(p + row_offset(lane0, m + m0 + d, S, end));
       };
       using std::integral_constant;
-      if (!MAP) rows(0, tq, -3, integral_constant<int, 7>{});
-      rows(1, tk, -3, integral_constant<int, 7>{});
-      if (!MAP) rows(2, tv, -3, integral_constant<int, 7>{});
-      rows(3, xg[0], 0, integral_constant<int, 4>{});
-      rows(4, xg[1], 0, integral_constant<int, 4>{});
-      if (!MAP) rows(5, xg[2], 0, integral_constant<int, 4>{});
+      if (!MAP) rows(0, tq, kch, -3, integral_constant<int, 7>{});
+      rows(1, tk, kch, -3, integral_constant<int, 7>{});
+      if (!MAP) rows(2, tv, col, -3, integral_constant<int, 7>{});
+      rows(3, xg[0], kch, 0, integral_constant<int, 4>{});
+      rows(4, xg[1], kch, 0, integral_constant<int, 4>{});
+      if (!MAP) rows(5, xw, col, 0, integral_constant<int, 4>{});
     } else {
       const char* bk = base(a.k, a.ks0, a.ks1, a.ks2, ES, t0);
       const char* bv = base(a.vp, a.vs0, a.vs1, a.vs2, ES, t0);
@@ -302,27 +305,29 @@ __device__ __forceinline__ int sub_run(const SubArgs& a, SubSmem<PRO, DK>& sm, i
     }
   };
   // fused prologue: taps before token 0 come from the history, or are zero
-  auto hist_rows = [&](int s, Row<false, 4> (&t)[7]) {
+  auto hist_rows = [&](int s, auto& t, int ch) {
+    constexpr int N = sizeof(t[0]) / 2;
     if (g != 0) return;
 #pragma unroll
     for (int m = 0; m < 3; ++m) {
-      uint32_t h[4] = {0, 0, 0, 0};
+      uint32_t h[N] = {};
       if (a.ph[s]) {
-        const uint16_t* hp = a.ph[s] + (int64_t)bi * a.phs0[s] + (int64_t)(hi * 64 + kch) * a.phs1[s] + (int64_t)m * a.phs2[s];
+        const uint16_t* hp = a.ph[s] + (int64_t)bi * a.phs0[s] + (int64_t)(hi * 64 + ch) * a.phs1[s] + (int64_t)m * a.phs2[s];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) h[e] = hp[(int64_t)e * a.phs1[s]];
+        for (int e = 0; e < N; ++e) h[e] = hp[(int64_t)e * a.phs1[s]];
       }
-      t[m].w[0] = h[0] | (h[1] << 16);
-      t[m].w[1] = h[2] | (h[3] << 16);
+#pragma unroll
+      for (int e = 0; e < N; e += 2) t[m].w[e / 2] = h[e] | (h[e + 1] << 16);
     }
   };
-  // fused prologue: SiLU(depthwise conv) of the lane's four tokens and channels
-  auto conv = [&](int s, const Row<false, 4> (&t)[7], float (&y)[4][4]) {
-    f32x4 w[4];
+  // fused prologue: SiLU(depthwise conv) of the lane's four tokens and N channels from ch on
+  auto conv = [&](int s, const auto& t, int ch, auto& y) {
+    constexpr int N = sizeof(y[0]) / sizeof(float);
+    fvec<N> w[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) w[j] = *(const f32x4*)&sm.cw[s][j][PRO ? kch : 0];
+    for (int j = 0; j < 4; ++j) w[j] = *(const fvec<N>*)&sm.cw[s][j][PRO ? ch : 0];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
+    for (int e = 0; e < N; ++e) {
       float x[7];
 #pragma unroll
       for (int m = 0; m < 7; ++m) x[m] = row_at<false>(t[m], e);
@@ -380,11 +385,11 @@ __device__ __forceinline__ int sub_run(const SubArgs& a, SubSmem<PRO, DK>& sm, i
     f32x4 ve[NCT];                         // w*v, then the solve's right-hand side
     if constexpr (PRO) {
       if (cc == 0) {
-        if (!MAP) hist_rows(0, tq);
-        hist_rows(1, tk);
-        if (!MAP) hist_rows(2, tv);
+        if (!MAP) hist_rows(0, tq, kch);
+        hist_rows(1, tk, kch);
+        if (!MAP) hist_rows(2, tv, col);
       }
-      conv(1, tk, kk);
+      conv(1, tk, kch, kk);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const float ss = row16_sum(kk[i][0] * kk[i][0] + kk[i][1] * kk[i][1] + kk[i][2] * kk[i][2] + kk[i][3] * kk[i][3]);
@@ -398,13 +403,13 @@ __device__ __forceinline__ int sub_run(const SubArgs& a, SubSmem<PRO, DK>& sm, i
         }
       }
       if (!MAP) {
-        float vv[4][4];
-        conv(2, tv, vv);
+        float vv[4][NVT];
+        conv(2, tv, col, vv);
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
-          for (int j = 0; j < NVT; ++j) ve[j][i] = pro_sigmoid(row_at<false>(xg[2][i], j)) * vv[i][j];
-        conv(0, tq, qq);
+          for (int j = 0; j < NVT; ++j) ve[j][i] = pro_sigmoid(row_at<false>(xw[i], j)) * vv[i][j];
+        conv(0, tq, kch, qq);
       }
     } else {
       auto convert = [&](auto f16_c) {
@@ -750,7 +755,7 @@ __device__ __forceinline__ void sub_new_history(const SubArgs& a, int lane, int 
 // lane and runs one.
 template <bool F32IN, bool G16, bool GCH, bool PRO, int DK, int DV>
 __global__ __launch_bounds__(64, DK == 128 ? 1 : 2) void dgda_sub_kernel(SubArgs a) {
-  static_assert(!PRO || (DK == 64 && DV == 64), "the fused prologue takes 64-channel heads");
+  static_assert(!PRO || DK == 64, "the fused prologue takes 64-channel heads");
   static_assert((DK == 32 || DK == 64 || DK == 128) && (DV == 32 || DV == 64), "head sizes");
   constexpr int NKT = DK / 16, NVT = DV / 16;
   constexpr int MC = DK < 64 ? DK : 64, NMT = MC / 16, NCG = DK / MC;   // transition columns per wave, waves per map

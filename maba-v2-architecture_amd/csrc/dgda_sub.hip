@@ -81,9 +81,9 @@ struct SubCut { int nseg, seglen, cols; };
 // As many segments as fill one wave per SIMD, or two (see SUB_LEN_2; always at d_k = 32, whose
 // waves hold a quarter of the state, never at d_k = 128, whose state leaves registers for one),
 // no more than SUB_SEG_ROOT lets a scan walk, and no more than the workspace holds.  Where that
-// leaves half the SIMDs without work a wave takes 32 columns instead of 64 (narrow; not in the fused
-// layer, whose staging is most of a sub-chunk): the key side is done twice, but a sub-chunk takes a
-// wave less time (B=2 H=10 bf16: T=160 54 -> 37 us, T=1000 57 -> 48 us).
+// leaves half the SIMDs without work a wave takes 32 columns instead of 64 (narrow): the key side is
+// done twice, but a sub-chunk takes a wave less time (B=2 H=10 bf16: T=160 54 -> 37 us, T=1000 57 ->
+// 48 us; the fused layer at H=10, T=100 52 -> 45 us, T=160 68 -> 59, T=1000 87 -> 77).
 static SubCut sub_cut(int64_t BH, int64_t L, int64_t dk, int64_t dv, size_t ws_bytes, bool narrow) {
   const int64_t nch = sub_chunks(L);
   const int64_t simds = 4 * (int64_t)device_cu_count();
@@ -131,6 +131,26 @@ static int sub_place(SubArgs& a, int64_t BH, int64_t L, int64_t dk, int64_t dv, 
   a.agg = (float*)ws;
   a.zc = (int*)(a.agg + BH * a.nseg * dk * (dv + dk));
   return c.cols;
+}
+
+// No byte of the new history belongs to the old one.
+static bool histories_apart(const maba_tensor* const* hist, maba_tensor* const* new_hist) {
+  auto range = [](const maba_tensor* t, uintptr_t& lo, uintptr_t& hi) {
+    lo = hi = (uintptr_t)t->data;
+    for (int d = 0; d < 3; ++d) {
+      const int64_t span = (t->shape[d] - 1) * t->stride[d] * (t->dtype == MABA_F32 ? 4 : 2);
+      (span < 0 ? lo : hi) += span;
+    }
+    hi += 4;
+  };
+  for (int s = 0; s < 3; ++s)
+    for (int n = 0; n < 3; ++n) {
+      uintptr_t l0, h0, l1, h1;
+      range(hist[s], l0, h0);
+      range(new_hist[n], l1, h1);
+      if (l0 < h1 && l1 < h0) return false;
+    }
+  return true;
 }
 
 // One vector store per lane and token: aligned rows.
@@ -257,8 +277,10 @@ extern "C" int maba_hip_dgda_layer_prefill(const maba_tensor* const* xs, const m
   a.sf = mview4(final_state);
   a.H = (int)H; a.L = (int)L; a.BH = (int)BH;
   a.use_log = 1; a.has_s0 = initial_state != nullptr;
-  sub_place(a, BH, L, 64, 64, workspace, workspace_bytes, false);
-  // the new history is written by the last launch, after the first one has read the old: it
-  // may overwrite it in place
-  return run_sub_passes<true, 64, 64>(a, false, false, true, (hipStream_t)stream);
+  // the new history is written by the last launch, after the first one has read the old: it may
+  // overwrite it in place; where one launch is all, by the one wave per head that read it
+  const int cols = sub_place(a, BH, L, 64, 64, workspace, workspace_bytes,
+                             !hist || sub_cut(BH, L, 64, 64, workspace_bytes, true).nseg > 1 || histories_apart(hist, new_hist));
+  return cols == 32 ? run_sub_passes<true, 64, 32>(a, false, false, true, (hipStream_t)stream)
+                    : run_sub_passes<true, 64, 64>(a, false, false, true, (hipStream_t)stream);
 }

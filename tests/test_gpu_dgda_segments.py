@@ -172,3 +172,21 @@ def test_layer_rows_beyond_32_bits(dev):
     got = hb.hip_dgda_layer_prefill(far.split(64, dim=-1), convs)
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
     assert all(torch.equal(a, b) for a, b in zip(got[2], want[2]))
+
+
+@pytest.mark.parametrize("L", [1, 15, 100, 300])
+def test_layer_columns_per_wave(dev, L):
+    """Few heads take 32 value columns per wave, many 64: the same heads give the same bits."""
+    from maba_sparse.kernels import hip_backend as hb
+    g = torch.Generator().manual_seed(L)
+    rn = lambda *s: torch.randn(*s, generator=g).bfloat16().to(dev)  # noqa: E731
+    x, convs, hist = rn(1, L, 6 * 128), [rn(128, 1, 4) for _ in range(3)], [rn(1, 128, 3) for _ in range(3)]
+    many = 600   # 1,200 heads: more waves than SIMDs, one segment
+    args = lambda n: (x.expand(n, -1, -1).contiguous().split(128, dim=-1), convs, [h.expand(n, -1, -1).contiguous() for h in hist])  # noqa: E731
+    one, all_ = hb.hip_dgda_layer_prefill(*args(1)), hb.hip_dgda_layer_prefill(*args(many))
+    for a, b in zip((one[0], one[1], *one[2]), (all_[0], all_[1], *all_[2])):
+        if L <= 100:   # one segment either way
+            assert torch.equal(b, a.expand_as(b))
+        else:
+            assert_close(b[0], to_np(a[0]), 1e-2, 1e-2, "cut differs")
+            assert torch.equal(b, b[:1].expand_as(b))

@@ -71,6 +71,13 @@ constexpr int64_t SUB_LEN_2 = 32;
 // 1513 / 1015 (160 / 146 / 172); the fused layer T=65536 771 / 451 / 418 (770 / 147 / 202: without
 // it segments end before their transitions vanish).
 constexpr double SUB_SEG_ROOT = 6;
+// A short sequence of many heads stays whole where cutting it does not pay if its transitions
+// survive: every sub-chunk is run twice, on SIMDs that segments and transitions share, and joining
+// them takes as long as SUB_ENDS sub-chunks.  B H = 160, T=200, cut into three / whole, us, decay that
+// remembers (and that vanishes): 67 / 50 (53 / 50); BH = 320, T=320 110 / 76 (73 / 76), T=500 154 /
+// 117 (90 / 117).  Beyond SUB_SHORT sub-chunks the segments of vanishing transitions gain more than that.
+constexpr int64_t SUB_SHORT = 64;
+constexpr int SUB_ENDS = 8;
 
 static int64_t sub_chunks(int64_t L) { return ceil_div(L, SC); }
 static size_t sub_slot_bytes(int64_t dk, int64_t dv) { return (size_t)(dk * (dv + dk)) * sizeof(float) + 2 * sizeof(int); }
@@ -98,11 +105,20 @@ static SubCut sub_cut(int64_t BH, int64_t L, int64_t dk, int64_t dv, size_t ws_b
   if (n > SUB_MAX_SEG) n = SUB_MAX_SEG;
   // two short segments take no less time one after the other (the second's re-run) than one
   if (n < 2 || (n == 2 && nch < 4 * SUB_MIN_LEN)) n = 1;
-  const int64_t len = nch > 0 ? ceil_div(nch, n) : 0;
-  SubCut c;
-  c.seglen = (int)len;
-  c.nseg = len > 0 ? (int)ceil_div(nch, len) : 1;
-  c.cols = dv == 32 || (narrow && 2 * waves * c.nseg <= simds) ? 32 : 64;
+  auto cut = [&](int64_t n) {
+    const int64_t len = nch > 0 ? ceil_div(nch, n) : 0;
+    SubCut c;
+    c.seglen = (int)len;
+    c.nseg = len > 0 ? (int)ceil_div(nch, len) : 1;
+    c.cols = dv == 32 || (narrow && 2 * waves * c.nseg <= simds) ? 32 : 64;
+    return c;
+  };
+  const SubCut c = cut(n);
+  if (dk == 64 && c.nseg > 1 && nch <= SUB_SHORT) {
+    const int64_t main = waves * (c.cols < dv ? 64 / c.cols : 1) * c.nseg + BH * (c.nseg - 1);   // the first launch's waves
+    const double share = std::max(1.0, (double)main / simds);
+    if (2 * main > simds && 2 * c.seglen * share + SUB_ENDS > nch) return cut(1);
+  }
   return c;
 }
 

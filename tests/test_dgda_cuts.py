@@ -47,3 +47,11 @@ def test_sub_chunk_cut_is_bounded(BH, d):
     for T in (100, 1000, 4096, 10007, 32768, 131072, 1 << 20, 1 << 24):
         n = _nbytes(1, BH, T, d, "channel", "preferred") / (BH * (d * 2 * d * 4 + 8))
         assert n <= 6 * (-(-T // 16)) ** 0.5, f"{T} tokens"
+
+
+@pytest.mark.parametrize("BH,T,segments", [(160, 200, 1), (160, 240, 1), (320, 200, 1), (320, 500, 1), (320, 1000, 1),
+                                           (160, 320, 4), (10, 200, 3), (40, 320, 4), (320, 1100, 3), (160, 1000, 6)])
+def test_sub_chunk_short_sequences(BH, T, segments):
+    """Many heads' short sequences stay whole, few heads' and long ones are cut."""
+    n = _nbytes(1, BH, T, 64, "channel", "preferred") / (BH * (64 * 128 * 4 + 8))
+    assert max(1, n) == segments

@@ -203,6 +203,12 @@ __device__ __forceinline__ void split2(float x0, float x1, uint32_t& h, uint32_t
   h = cvt_pk_bf16(x0, x1);
   l = cvt_pk_bf16(bf16_rem<0>(h, x0), bf16_rem<1>(h, x1));
 }
+// The same of a pair that stays in use: bf16_rem's dot product overwrites its operand, so it would
+// cost a copy, and wait states on either side.
+__device__ __forceinline__ void split2_kept(float x0, float x1, uint32_t& h, uint32_t& l) {
+  h = cvt_pk_bf16(x0, x1);
+  l = cvt_pk_bf16(x0 - __uint_as_float(h << 16), x1 - __uint_as_float(h & 0xffff0000u));
+}
 __device__ __forceinline__ i16x8 pack8(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
   typedef uint32_t u4 __attribute__((ext_vector_type(4)));
   const u4 v = {a, b, c, d};
@@ -251,6 +257,25 @@ __device__ __forceinline__ int sub_run(const SubArgs& a, SubSmem<PRO, DK>& sm, i
   auto base = [&](const void* p, int s0, int s1, int s2, int es, int t0) {
     return (const char*)p + ((int64_t)bi * s0 + (int64_t)hi * s1 + (int64_t)t0 * s2) * es;
   };
+  // Output waves of the fused layer and of 32 columns keep pointers to the rows to load next (a
+  // twentieth of a sub-chunk's instructions otherwise); elsewhere their registers cost more (64
+  // columns at 160 heads T=1000 135 us without, 137 with).
+  constexpr bool HOIST = !MAP && DK == 64 && (PRO || DV == 32);
+  const char* src[6] = {};
+  if constexpr (HOIST) {
+    const int t0 = c_begin * SC;
+    if constexpr (PRO) {
+#pragma unroll
+      for (int s = 0; s < 6; ++s) src[s] = base(a.px[s], a.pxs0[s], 0, a.pxs1[s], 2, max(t0 - 3, 0));
+    } else {
+      src[0] = base(a.q, a.qs0, a.qs1, a.qs2, ES, t0);
+      src[1] = base(a.k, a.ks0, a.ks1, a.ks2, ES, t0);
+      src[2] = base(a.vp, a.vs0, a.vs1, a.vs2, ES, t0);
+      src[3] = base(a.gp, a.gs0, a.gs1, a.gs2, EG, t0);
+      src[4] = base(a.bp, a.bs0, a.bs1, a.bs2, EG, t0);
+      src[5] = base(a.wp, a.ws0, a.ws1, a.ws2, EG, t0);
+    }
+  }
   Row<F32IN, NKT> pq[4], pk[4];
   Row<F32IN, NVT> pv[4];
   Row<!G16, NKT> pg[4], pb[4];
@@ -265,12 +290,13 @@ __device__ __forceinline__ int sub_run(const SubArgs& a, SubSmem<PRO, DK>& sm, i
       const int d = min(t0, 3);   // rows are counted from token t0 - d
       auto rows = [&](int s, auto& x, int ch, int m0, auto n_c) {
         constexpr int N = sizeof(x[0]) / 2;
-        const char* p = base(a.px[s], a.pxs0[s], 0, a.pxs1[s], 2, t0 - d);
+        const char* p = !HOIST ? base(a.px[s], a.pxs0[s], 0, a.pxs1[s], 2, t0 - d) : src[s];
         const int S = 2 * a.pxs1[s], chb = 2 * (hi * 64 + ch);
         const uint32_t lane0 = 4u * g * S + chb, end = row_end(a.L - 1 - (t0 - d), SC - 1 + d, S, chb);
 #pragma unroll
         for (int m = 0; m < decltype(n_c)::value; ++m)
           x[m] = load_row<false, N>(p + row_offset(lane0, m + m0 + d, S, end));
+        if (HOIST) src[s] += (int64_t)(cc + 1 < c_end ? SC - 3 + d : 0) * S;
       };
       using std::integral_constant;
       if (!MAP) rows(0, tq, kch, -3, integral_constant<int, 7>{});
@@ -280,27 +306,25 @@ __device__ __forceinline__ int sub_run(const SubArgs& a, SubSmem<PRO, DK>& sm, i
       rows(4, xg[1], kch, 0, integral_constant<int, 4>{});
       if (!MAP) rows(5, xw, col, 0, integral_constant<int, 4>{});
     } else {
-      const char* bk = base(a.k, a.ks0, a.ks1, a.ks2, ES, t0);
-      const char* bv = base(a.vp, a.vs0, a.vs1, a.vs2, ES, t0);
-      const char* bg = base(a.gp, a.gs0, a.gs1, a.gs2, EG, t0);
-      const char* bb = base(a.bp, a.bs0, a.bs1, a.bs2, EG, t0);
-      const char* bw = base(a.wp, a.ws0, a.ws1, a.ws2, EG, t0);
-      auto rows = [&](const char* p, int S, int chb, auto& x, auto load) {
+      auto rows = [&](int s, const void* b, int s0, int s1, int s2, int es, int chb, auto& x, auto load) {
+        const int S = s2 * es;
+        const char* p = !HOIST ? base(b, s0, s1, s2, es, t0) : src[s];
         const uint32_t lane0 = 4 * g * S + chb, end = row_end(a.L - 1 - t0, SC - 1, S, chb);
 #pragma unroll
         for (int i = 0; i < 4; ++i) x[i] = load(p + row_offset(lane0, i, S, end));
+        if (HOIST) src[s] += cc + 1 < c_end ? SC * S : 0;
       };
       auto lk = [](const char* p) { return load_row<F32IN, NKT>(p); };
       auto lv = [](const char* p) { return load_row<F32IN, NVT>(p); };
       // a gate's rows at channel stride 1, or its element at stride 0 (then chb is zero)
       const int ck = kch * EG, cv = col * EG;
-      rows(bk, a.ks2 * ES, kch * ES, pk, lk);
-      rows(bg, a.gs2 * EG, GCH ? ck : ck * a.gs3, pg, [&](const char* p) { return load_gate<G16, GCH, NKT>(p, a.gs3); });
-      rows(bb, a.bs2 * EG, GCH ? ck : ck * a.bs3, pb, [&](const char* p) { return load_gate<G16, GCH, NKT>(p, a.bs3); });
+      rows(1, a.k, a.ks0, a.ks1, a.ks2, ES, kch * ES, pk, lk);
+      rows(3, a.gp, a.gs0, a.gs1, a.gs2, EG, GCH ? ck : ck * a.gs3, pg, [&](const char* p) { return load_gate<G16, GCH, NKT>(p, a.gs3); });
+      rows(4, a.bp, a.bs0, a.bs1, a.bs2, EG, GCH ? ck : ck * a.bs3, pb, [&](const char* p) { return load_gate<G16, GCH, NKT>(p, a.bs3); });
       if (!MAP) {
-        rows(base(a.q, a.qs0, a.qs1, a.qs2, ES, t0), a.qs2 * ES, kch * ES, pq, lk);
-        rows(bv, a.vs2 * ES, col * ES, pv, lv);
-        rows(bw, a.ws2 * EG, GCH ? cv : cv * a.ws3, pw, [&](const char* p) { return load_gate<G16, GCH, NVT>(p, a.ws3); });
+        rows(0, a.q, a.qs0, a.qs1, a.qs2, ES, kch * ES, pq, lk);
+        rows(2, a.vp, a.vs0, a.vs1, a.vs2, ES, col * ES, pv, lv);
+        rows(5, a.wp, a.ws0, a.ws1, a.ws2, EG, GCH ? cv : cv * a.ws3, pw, [&](const char* p) { return load_gate<G16, GCH, NVT>(p, a.ws3); });
       }
     }
   };
@@ -431,11 +455,18 @@ __device__ __forceinline__ int sub_run(const SubArgs& a, SubSmem<PRO, DK>& sm, i
       };
       if (!F32IN && a.f16) convert(std::true_type{});   // one branch, not one per element
       else convert(std::false_type{});
+      if (a.use_log) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < NKT; ++j)
-          la[i][j] = a.use_log ? la[i][j] * LOG2E : __builtin_amdgcn_logf(fmaxf(la[i][j], 1e-20f));
+          for (int j = 0; j < NKT; ++j) la[i][j] *= LOG2E;
+      } else {
+        asm volatile("");   // keeps this a branch
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int j = 0; j < NKT; ++j) la[i][j] = __builtin_amdgcn_logf(fmaxf(la[i][j], 1e-20f));
+      }
     }
     if (MAP) {
 #pragma unroll
@@ -539,14 +570,15 @@ __device__ __forceinline__ int sub_run(const SubArgs& a, SubSmem<PRO, DK>& sm, i
       // ---- row operands to LDS; the update's A operand kf stays in registers
       i16x8 kf[NKT];
       {
+        uint32_t kh_[4][NKT / 2], kl_[4][NKT / 2];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int tk_ = 4 * g + i;
-          uint32_t bh_[NKT / 2], bl_[NKT / 2], qh_[NKT / 2], ql_[NKT / 2], kh_[NKT / 2], kl_[NKT / 2];
+          uint32_t bh_[NKT / 2], bl_[NKT / 2], qh_[NKT / 2], ql_[NKT / 2];
 #pragma unroll
           for (int j = 0; j < NKT; j += 2) {
             split2(-(be[i][j] * kk[i][j]) * e[i][j], -(be[i][j + 1] * kk[i][j + 1]) * e[i][j + 1], bh_[j / 2], bl_[j / 2]);
-            split2(kx[i][j], kx[i][j + 1], kh_[j / 2], kl_[j / 2]);
+            split2(kx[i][j], kx[i][j + 1], kh_[i][j / 2], kl_[i][j / 2]);
             if (!MAP) split2(qq[i][j] * e[i][j], qq[i][j + 1] * e[i][j + 1], qh_[j / 2], ql_[j / 2]);
           }
           auto put = [&](short* dst, const uint32_t (&v)[NKT / 2]) {
@@ -557,8 +589,8 @@ __device__ __forceinline__ int sub_run(const SubArgs& a, SubSmem<PRO, DK>& sm, i
           };
           put(sm.r.BKh, bh_);
           put(sm.r.BKl, bl_);
-          put(sm.r.KIh, kh_);
-          put(sm.r.KIl, kl_);
+          put(sm.r.KIh, kh_[i]);
+          put(sm.r.KIl, kl_[i]);
           if (!MAP) {
             put(sm.r.QEh, qh_);
             put(sm.r.QEl, ql_);
@@ -566,10 +598,10 @@ __device__ __forceinline__ int sub_run(const SubArgs& a, SubSmem<PRO, DK>& sm, i
         }
 #pragma unroll
         for (int j = 0; j < NKT; ++j) {
-          uint32_t h0, h1, l0, l1;
-          split2(kx[0][j], kx[1][j], h0, l0);
-          split2(kx[2][j], kx[3][j], h1, l1);
-          kf[j] = pack8(h0, h1, l0, l1);   // [hi | lo] of tokens 4g .. 4g+3, channel kch + j
+          // [hi | lo] of tokens 4g .. 4g+3, channel kch + j, from the pairs of channels
+          const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;
+          auto two = [&](const uint32_t (&v)[4][NKT / 2], int i) { return __builtin_amdgcn_perm(v[i + 1][j / 2], v[i][j / 2], sel); };
+          kf[j] = pack8(two(kh_, 0), two(kh_, 2), two(kl_, 0), two(kl_, 2));
         }
         if (g == 3) {
 #pragma unroll
@@ -629,7 +661,7 @@ __device__ __forceinline__ int sub_run(const SubArgs& a, SubSmem<PRO, DK>& sm, i
 #pragma unroll
           for (int e = 0; e < 8; e += 2) {
             const int l0 = 8 * p + e, l1 = l0 + 1;
-            split2(Sr[l0 % NKT][t][l0 / NKT], Sr[l1 % NKT][t][l1 / NKT], h[e / 2], l[e / 2]);
+            split2_kept(Sr[l0 % NKT][t][l0 / NKT], Sr[l1 % NKT][t][l1 / NKT], h[e / 2], l[e / 2]);
           }
           const i16x8 sh = pack8(h[0], h[1], h[2], h[3]), sl = pack8(l[0], l[1], l[2], l[3]);
           ve[t] = mma32(ve[t], bh8[p], sh);

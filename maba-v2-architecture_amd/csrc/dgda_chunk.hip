@@ -781,8 +781,7 @@ static size_t chunk_geom_bytes(const SlotGeom& gm, int64_t BH) {
 // CPS_FINE of 2 measured as 4 where maps vanish and slower with many surviving ones (H=10 T=5000
 // 161 against 100), 8 slower.
 constexpr int WALK = 24, WALK_MAX = 64;
-static int64_t fine_slot(int64_t BH, int64_t nch) {
-  const int64_t cus = device_cu_count();
+static int64_t fine_slot(int64_t BH, int64_t nch, int64_t cus) {
   int64_t U = std::max<int64_t>(CPS_FINE, ceil_div(BH * nch, 2 * cus));
   if (U >= CPS || ceil_div(nch, U) <= WALK) return U;
   if (ceil_div(BH * nch, cus) <= CPS) U = std::max(U, ceil_div(BH * nch, cus));
@@ -794,9 +793,9 @@ static int64_t fine_slot(int64_t BH, int64_t nch) {
 // 53 -> 39 / 53 -> 68), and while each slot has a CU (B=8 T=1000, 320 slots: 75 -> 46 / 75 -> 104).
 static SlotGeom chunk_geom(int64_t BH, int64_t L, size_t ws_bytes) {
   const int64_t nch = ceil_div(L, CH) > 0 ? ceil_div(L, CH) : 1;
-  const SlotGeom coarse = slot_geom(BH, nch, CPS), fine = slot_geom(BH, nch, fine_slot(BH, nch));
-  const bool pays = coarse.nseg_max > 1 ||
-                    (nch > SHORT_CHUNKS && ceil_div(BH * nch, fine.U) <= device_cu_count());
+  const int64_t cus = device_cu_count();
+  const SlotGeom coarse = slot_geom(BH, nch, CPS, cus), fine = slot_geom(BH, nch, fine_slot(BH, nch, cus), cus);
+  const bool pays = coarse.nseg_max > 1 || (nch > SHORT_CHUNKS && ceil_div(BH * nch, fine.U) <= cus);
   return pays && chunk_geom_bytes(fine, BH) <= ws_bytes ? fine : coarse;
 }
 
@@ -833,8 +832,6 @@ int launch_dgda_chunk(const maba_tensor* q, const maba_tensor* k, const maba_ten
   a.U = gm.U;
   a.nseg_max = gm.nseg_max;
   a.use_log = use_log; a.has_s0 = s0 != nullptr;
-  const size_t need = dgda_chunk_workspace(BH, L);
-  if (ws_bytes < need) return fail(MABA_ERR_WORKSPACE, "dgda_prefill: workspace too small");
   const int64_t nsegs = BH * a.nseg_max;
   a.agg = (float*)ws;
   a.zc = (int*)(a.agg + nsegs * 64 * 128);

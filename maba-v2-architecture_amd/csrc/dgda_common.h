@@ -185,8 +185,8 @@ __device__ __forceinline__ int seg_count_of(int nchunks, int64_t U, int bh) {
 // workgroups per CU, at least min_u chunks per slot.
 struct SlotGeom { int64_t U; int nseg_max; };
 
-inline SlotGeom slot_geom(int64_t BH, int64_t nch, int64_t min_u) {
-  const int64_t slots = 2 * (int64_t)device_cu_count();
+inline SlotGeom slot_geom(int64_t BH, int64_t nch, int64_t min_u, int64_t cus) {
+  const int64_t slots = 2 * cus;
   int64_t U = (BH * nch + slots - 1) / slots;
   if (U < min_u) U = min_u;
   SlotGeom gm;

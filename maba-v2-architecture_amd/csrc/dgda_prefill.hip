@@ -132,28 +132,29 @@ int launch_dgda_sub(const maba_tensor* q, const maba_tensor* k, const maba_tenso
 
 using namespace maba;
 
+// The call picks its path from every operand (k, w and out included), which the queries do not see.
+// Each path's least size depends only on the shapes, so the larger of those of the paths that q, v
+// and the gates admit is returned: the call's choice always fits.
+static size_t prefill_workspace(const maba_tensor* q, const maba_tensor* v, const maba_tensor* gate, const maba_tensor* b,
+                                bool preferred) {
+  if (!q || q->ndim != 4 || !v || v->ndim != 4 || !gate || !b) return 0;
+  const int64_t BH = q->shape[0] * q->shape[1], L = q->shape[2], dk = q->shape[3], dv = v->shape[3];
+  const bool chunk = dgda_chunk_supported(q, q, v, gate, b), sub = dgda_sub_supported(q, q, v, gate, b, nullptr, nullptr);
+  size_t n = 0;
+  if (chunk) n = preferred ? std::max(dgda_chunk_workspace(BH, L), dgda_chunk_workspace_preferred(BH, L)) : dgda_chunk_workspace(BH, L);
+  if (sub) n = std::max(n, dgda_sub_workspace(BH, L, dk, dv));
+  if (sub && !chunk && preferred) n = std::max(n, dgda_sub_workspace_preferred(BH, L, dk, dv));
+  return n;
+}
+
 extern "C" size_t maba_hip_dgda_prefill_workspace_size(const maba_tensor* q, const maba_tensor* v,
                                                       const maba_tensor* gate, const maba_tensor* b) {
-  if (!q || q->ndim != 4 || !v || v->ndim != 4 || !gate || !b) return 0;
-  // The call picks its path from every operand (k, w and out included), which this query
-  // does not see.  Both workspace sizes depend only on the shapes, so the larger of those
-  // of the paths that q, v and the gates admit is returned: the call's choice always fits.
-  const int64_t BH = q->shape[0] * q->shape[1], L = q->shape[2];
-  size_t n = 0;
-  if (dgda_chunk_supported(q, q, v, gate, b)) n = dgda_chunk_workspace(BH, L);
-  if (dgda_sub_supported(q, q, v, gate, b, nullptr, nullptr))
-    n = std::max(n, dgda_sub_workspace(BH, L, q->shape[3], v->shape[3]));
-  return n;
+  return prefill_workspace(q, v, gate, b, false);
 }
 
 extern "C" size_t maba_hip_dgda_prefill_workspace_preferred(const maba_tensor* q, const maba_tensor* v,
                                                            const maba_tensor* gate, const maba_tensor* b) {
-  size_t n = maba_hip_dgda_prefill_workspace_size(q, v, gate, b);
-  if (n && dgda_chunk_supported(q, q, v, gate, b))
-    n = std::max(n, dgda_chunk_workspace_preferred(q->shape[0] * q->shape[1], q->shape[2]));
-  else if (n && dgda_sub_supported(q, q, v, gate, b, nullptr, nullptr))
-    n = std::max(n, dgda_sub_workspace_preferred(q->shape[0] * q->shape[1], q->shape[2], q->shape[3], v->shape[3]));
-  return n;
+  return prefill_workspace(q, v, gate, b, true);
 }
 
 extern "C" int maba_hip_dgda_prefill(const maba_tensor* q, const maba_tensor* k, const maba_tensor* v,

@@ -124,7 +124,7 @@ static SubCut sub_cut(int64_t BH, int64_t L, int64_t dk, int64_t dv, size_t ws_b
 
 // The size the query promises to be enough; what fits in it, sub_cut works out.
 size_t dgda_sub_workspace(int64_t BH, int64_t L, int64_t dk, int64_t dv) {
-  const SlotGeom gm = slot_geom(BH, sub_chunks(L) > 0 ? sub_chunks(L) : 1, 64);
+  const SlotGeom gm = slot_geom(BH, sub_chunks(L) > 0 ? sub_chunks(L) : 1, 64, device_cu_count());
   if (gm.nseg_max <= 1) return 16;
   const int64_t dvc = dv == 128 ? 64 : dv;
   return (size_t)(BH * gm.nseg_max * dk * (dvc + dk)) * sizeof(float) + (size_t)(BH * gm.nseg_max) * sizeof(int);
@@ -199,7 +199,6 @@ int launch_dgda_sub(const maba_tensor* q, const maba_tensor* k, const maba_tenso
   a.H = (int)H; a.L = (int)L; a.BH = (int)BH;
   a.use_log = use_log; a.has_s0 = s0 != nullptr;
   a.f16 = q->dtype == MABA_F16;
-  if (ws_bytes < dgda_sub_workspace(BH, L, dk, dv)) return fail(MABA_ERR_WORKSPACE, "dgda_prefill: workspace too small");
   const int cols = sub_place(a, BH, L, dk, dv, ws, ws_bytes, true);
   const bool f32in = q->dtype == MABA_F32, g16 = gate->dtype != MABA_F32;
   const bool gch = a.gs3 == 1 && a.bs3 == 1 && a.ws3 == 1;

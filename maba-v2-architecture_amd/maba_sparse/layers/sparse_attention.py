@@ -34,8 +34,10 @@ from maba_sparse.layers._wcache import WeightCacheMixin, cached
 from maba_sparse.layers.indexer import DGIndexer, _Growing
 
 # Fused prefill: the head-space kernel is taken while 16 consecutive queries list fewer than
-# this many distinct blocks, in units of top_k (the measured crossover with the latent kernel)
+# this many distinct blocks, in units of top_k (where it meets the latent kernel, see _prefill_form):
+# for heads of together at most five times d_c and at most 32 blocks per query, and otherwise
 PREFILL_UNION_LIMIT = 6.9
+PREFILL_UNION_LIMIT_WIDE = 5.25
 
 
 class LatentCache:
@@ -124,7 +126,8 @@ class MabaSparseAttention(WeightCacheMixin, nn.Module):
         # fused bf16 prefill: "auto" picks the latent or the head-space kernel from the
         # selections' sharing (see _prefill_form); the union limit is in units of top_k
         self.prefill_form = "auto"
-        self.prefill_union_limit = PREFILL_UNION_LIMIT
+        self.prefill_union_limit = (PREFILL_UNION_LIMIT if H * dh <= 5 * self.d_c and self.top_k <= 32
+                                    else PREFILL_UNION_LIMIT_WIDE)
         self._install_weight_cache_hooks()
 
     def reset_cache(self) -> None:
@@ -294,10 +297,13 @@ class MabaSparseAttention(WeightCacheMixin, nn.Module):
         as at decode); the head-space kernel gives each run of 64 queries the union of their
         blocks, staged once per tile and computed by each 16-query wave that lists it (16
         queries share every key tile, per head).  Its cost grows with the union of 16
-        consecutive queries' blocks, the latent kernel's does not: measured at 10 heads of 64,
-        d_c 128, top-32 (heads / latent, ms): random queries at 32k tokens, 5.1 K distinct blocks
-        per 16 queries, 2.83 / 4.05; at 64k, 6.5 K, 7.63 / 8.52; at 128k, 7.6 K, 21.2 / 18.8, and
-        with queries partly alike, 4.9 K, 11.0 / 18.8, so the two are equal near 7 K.  Neighbouring
+        consecutive queries' blocks and with the heads' channels, the latent kernel's with d_c
+        alone.  Measured (heads / latent, ms; union in units of top_k), 10 heads of 64, d_c 128,
+        top-32: 32k tokens, union 5.1, 2.80 / 4.42; 64k, 6.5, 7.95 / 9.20; 128k, 6.9, 17.9 / 20.2,
+        7.4, 19.9 / 20.2, 7.6, 21.2 / 18.8; 256k, 7.4, 42.5 / 47.7; top-16, 128k, 7.0, 9.4 / 16.3.
+        16 heads of 32, 128k, 6.7, 21.5 / 21.8.  The latent kernel wins earlier where the heads are
+        wider against d_c or a query lists more blocks: 16 heads of 64, 64k, 5.8, 10.4 / 10.2; heads of
+        128, 5.35, 11.7 / 9.4; d_c 64, 5.8, 6.6 / 4.9; top-64, 128k, 6.1, 29.8 / 28.1.  Neighbouring
         queries of a trained or randomly initialised model select nearly the same blocks (about 3 K).
         The union is counted on the GPU from ``idx``
         (``hip_prefill_union``; elsewhere one segmented sort); ``self.prefill_form`` may force either."""

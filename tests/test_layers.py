@@ -216,3 +216,15 @@ def test_prefill_form_follows_selection_sharing():
     assert layer._prefill_form(shared[:, :1]) == "heads"                 # one row for all queries
     layer.prefill_form = "latent"
     assert layer._prefill_form(shared) == "latent"
+
+
+@pytest.mark.parametrize("H,dh,dc,K,limit", [(10, 64, 128, 32, 6.9), (16, 32, 128, 8, 6.9), (5, 128, 128, 32, 6.9),
+                                             (10, 128, 128, 32, 5.25), (16, 64, 128, 32, 5.25), (10, 64, 64, 32, 5.25),
+                                             (10, 64, 128, 64, 5.25)])
+def test_sa_prefill_form_limit(monkeypatch, H, dh, dc, K, limit):
+    """The fused prefill's choice: where the two kernels were measured to meet, by heads, d_c and top_k."""
+    sa = MabaSparseAttention(dim=64, n_heads=H, d_head=dh, d_c=dc, top_k=K)
+    for ratio, form in ((limit - 0.1, "heads"), (limit + 0.1, "latent")):
+        n = int(ratio * K)                  # distinct blocks of the only 16 queries
+        idx = (torch.arange(16 * K) % n).view(1, 16, K)
+        assert sa._prefill_form(idx) == form, ratio

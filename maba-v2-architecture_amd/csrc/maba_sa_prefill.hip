@@ -59,6 +59,16 @@ constexpr int PF_LIST = 64 * PF_MAXK;   // the union of a workgroup's 64 queries
 constexpr int PF_QWORDS = 16;        // words of a query's row of union bits (512 entries)
 constexpr float PF_SLACK = 8.f;      // a score may pass the running reference by 2^8
 
+// The workgroup's union of blocks; behind a list of at most 32 PF_QWORDS of them, the rows of bits.
+union PfList {
+  uint16_t block[PF_LIST];
+  struct {
+    uint16_t list[32 * PF_QWORDS];
+    uint32_t qbits[64][PF_QWORDS];   // per query, the list entries it lists
+  } behind;
+};
+static_assert(sizeof(PfList) == PF_LIST * 2, "the rows of bits fit behind the list");
+
 typedef __attribute__((ext_vector_type(8))) short pf16x8;
 typedef __attribute__((ext_vector_type(4))) short pf16x4;
 
@@ -118,7 +128,8 @@ __global__ __launch_bounds__(256, NP == 4 ? 2 : 3) void maba_sa_prefill_kernel(P
   __shared__ __attribute__((aligned(16))) short s_k[2][TE];
   __shared__ __attribute__((aligned(16))) short s_v[2][TE];
   __shared__ uint32_t s_bits[PF_WORDS];
-  __shared__ uint16_t s_list[PF_LIST];
+  __shared__ PfList s_union;
+  uint16_t* s_list = s_union.block;
   __shared__ uint32_t s_need[4][PF_LIST / 32];    // per wave: the list entries its queries list
   // Set-up only, in value buffer 1 (first written by the first tile's prefetch, after the
   // set-up's last barrier): the list position of each bitmap word's first block, the list length.
@@ -127,8 +138,7 @@ __global__ __launch_bounds__(256, NP == 4 ? 2 : 3) void maba_sa_prefill_kernel(P
   int* s_count = s_nlist + 1;   // some query lists a block twice: slots are counted
   static_assert((PF_WORDS + 2) * 4 <= TE * 2, "set-up tables fit one value buffer");
   // per query, the list entries it lists, behind the entries of a list that short
-  uint32_t (*s_qbits)[PF_QWORDS] = (uint32_t (*)[PF_QWORDS])(s_list + 32 * PF_QWORDS);
-  static_assert(64 * PF_QWORDS * 4 + 32 * PF_QWORDS * 2 <= PF_LIST * 2, "the rows of bits fit behind the list");
+  uint32_t (*s_qbits)[PF_QWORDS] = s_union.behind.qbits;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int g = lane >> 4, c16 = lane & 15;
   const int64_t b = blockIdx.z;

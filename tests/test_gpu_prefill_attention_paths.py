@@ -1,6 +1,7 @@
 """Branches of the head-space MABA-SA prefill that only some selections or shapes take, against
 the float64 oracle (rtol = atol = 2e-3, as test_gpu_prefill_attention.py): distinct blocks read
 from bits, a union too long for them, references that move far, rows whose offsets need 64 bits."""
+import numpy as np
 import pytest
 import torch
 
@@ -102,3 +103,40 @@ def test_prefill_union_counts(dev, B, Lq, K, nb):
     d = idx.to(dev)
     assert sum(hb.hip_prefill_union(d).tolist()) == want
     assert sum(hb.hip_prefill_union(d.permute(2, 0, 1).contiguous().permute(1, 2, 0)).tolist()) == want
+
+
+@pytest.mark.parametrize("form", ["heads", "latent"])
+@pytest.mark.parametrize("T", [40, 777])
+def test_layer_output_in_64_bits(dev, form, T):
+    """The bf16 layer's output through either kernel, from its input to after ``o_proj``, against the
+    whole in 64 bits (given the selections, which depend on rounding).  The 2-norm of the difference:
+    seven bf16 roundings in a row (q; the latent rows; keys or absorbed queries; values; means; the
+    heads' output; the layer's) of 2^-9 / sqrt(3) each and their effect on the scores; 4e-3 expected,
+    1.5e-2 allowed."""
+    from maba_sparse.layers import MabaSparseAttention
+    torch.manual_seed(3)
+    H, dh, D = 5, 64, 320
+    layer = MabaSparseAttention(dim=D, n_heads=H, d_head=dh, d_c=128, d_idx=32, top_k=6).to(dev, torch.bfloat16).eval()
+    layer.prefill_form = form
+    seen = {}
+    fused = layer._fused_prefill
+    layer._fused_prefill = lambda x, q, c, idx: (seen.update(idx=idx), fused(x, q, c, idx))[1]
+    x = torch.randn(2, T, D, device=dev).bfloat16()
+    with torch.no_grad():
+        y, _ = layer(x)
+    lin = lambda t, m: t @ to_np(m.weight).T + (0 if m.bias is None else to_np(m.bias))  # noqa: E731
+    heads = lambda t: t.reshape(2, -1, H, dh).transpose(0, 2, 1, 3)  # noqa: E731
+    xd = to_np(x)
+    c = lin(xd, layer.kv_down_proj)
+    nc = T // 64
+    means = c[:, : nc * 64].reshape(2, nc, 64, 128).mean(axis=2)
+    n_early = min(T, 63)
+    early = c[:, :n_early].cumsum(axis=1) / np.arange(1, n_early + 1)[:, None]
+    kh, vh = (heads(lin(means, m)) if nc else None for m in (layer.k_up_proj, layer.v_up_proj))
+    o = osa.maba_sa_prefill_heads(heads(lin(xd, layer.q_proj)), heads(lin(c, layer.k_up_proj)), heads(lin(c, layer.v_up_proj)),
+                                  kh, vh, heads(lin(early, layer.v_up_proj)), seen["idx"].cpu().numpy(),
+                                  lin(xd, layer.stream_gate), scale=dh ** -0.5)
+    want = lin(o.transpose(0, 2, 1, 3).reshape(2, T, H * dh), layer.o_proj)
+    err = np.linalg.norm(to_np(y) - want) / np.linalg.norm(want)
+    assert err < 1.5e-2, err
+    print(f"{form} {T}: {err:.2e}")

@@ -71,13 +71,16 @@ constexpr int64_t SUB_LEN_2 = 32;
 // 1513 / 1015 (160 / 146 / 172); the fused layer T=65536 771 / 451 / 418 (770 / 147 / 202: without
 // it segments end before their transitions vanish).
 constexpr double SUB_SEG_ROOT = 6;
-// A short sequence of many heads stays whole where cutting it does not pay if its transitions
-// survive: every sub-chunk is run twice, on SIMDs that segments and transitions share, and joining
-// them takes as long as SUB_ENDS sub-chunks.  B H = 160, T=200, cut into three / whole, us, decay that
-// remembers (and that vanishes): 67 / 50 (53 / 50); BH = 320, T=320 110 / 76 (73 / 76), T=500 154 /
-// 117 (90 / 117).  Beyond SUB_SHORT sub-chunks the segments of vanishing transitions gain more than that.
+// A short sequence stays whole where cutting it does not pay if its transitions survive: every
+// sub-chunk is run twice, on SIMDs that segments and transitions share once these are more than
+// half as many as the SIMDs (below that segments always paid), and joining them takes as long as
+// SUB_ENDS sub-chunks.  B H = 160, T=200, cut into three / whole, us, decay that remembers (and that
+// vanishes): 67 / 50 (53 / 50); BH = 320, T=320 110 / 76 (73 / 76), T=500 154 / 117 (90 / 117); d_k =
+// 128, d_v = 64, BH = 160, T=170 101 / 61 (fp32).  At d_k = 32 a sub-chunk takes 2.2 us and the three
+// launches of a cut call 34 us of the host's time: T=170 35 / 30.  d_k = d_v = 128 always gained.
+// Beyond SUB_SHORT sub-chunks the segments of vanishing transitions gain more than that.
 constexpr int64_t SUB_SHORT = 64;
-constexpr int SUB_ENDS = 8;
+constexpr int SUB_ENDS = 8, SUB_ENDS_32 = 5;
 
 static int64_t sub_chunks(int64_t L) { return ceil_div(L, SC); }
 static size_t sub_slot_bytes(int64_t dk, int64_t dv) { return (size_t)(dk * (dv + dk)) * sizeof(float) + 2 * sizeof(int); }
@@ -114,10 +117,11 @@ static SubCut sub_cut(int64_t BH, int64_t L, int64_t dk, int64_t dv, size_t ws_b
     return c;
   };
   const SubCut c = cut(n);
-  if (dk == 64 && c.nseg > 1 && nch <= SUB_SHORT) {
-    const int64_t main = waves * (c.cols < dv ? 64 / c.cols : 1) * c.nseg + BH * (c.nseg - 1);   // the first launch's waves
-    const double share = std::max(1.0, (double)main / simds);
-    if (2 * main > simds && 2 * c.seglen * share + SUB_ENDS > nch) return cut(1);
+  if (c.nseg > 1 && nch <= SUB_SHORT && (dk < 128 || dv < 128)) {
+    // the first launch's waves: 32 or 64 output columns each, 64 columns of a transition
+    const int64_t main = waves * (c.cols < dv ? 64 / c.cols : 1) * c.nseg + BH * (c.nseg - 1) * (dk == 128 ? 2 : 1);
+    const double share = std::max(1.0, (double)main / (dk == 32 ? 2 * simds : simds));
+    if ((dk == 32 || 2 * main > simds) && 2 * c.seglen * share + (dk == 32 ? SUB_ENDS_32 : SUB_ENDS) > nch) return cut(1);
   }
   return c;
 }

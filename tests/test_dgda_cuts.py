@@ -12,11 +12,11 @@ pytestmark = pytest.mark.skipif(not os.path.exists(N.LIB_PATH), reason="libmaba_
 CUS = 256
 
 
-def _nbytes(B, H, T, d, gates, which):
-    q = _t([B, H, T, d])
+def _nbytes(B, H, T, d, gates, which, dv=None):
+    q, v = _t([B, H, T, d]), _t([B, H, T, dv or d])
     token = [H * T, T, 1, 0]
     gate = lambda: _t([B, H, T, d], N.MABA_F32, token if gates == "token" else None)  # noqa: E731
-    return getattr(N.load(), f"maba_hip_dgda_prefill_workspace_{which}")(q, q, gate(), gate())
+    return getattr(N.load(), f"maba_hip_dgda_prefill_workspace_{which}")(q, v, gate(), gate())
 
 
 def _chunk_segments(BH, T, which="preferred"):
@@ -49,9 +49,12 @@ def test_sub_chunk_cut_is_bounded(BH, d):
         assert n <= 6 * (-(-T // 16)) ** 0.5, f"{T} tokens"
 
 
-@pytest.mark.parametrize("BH,T,segments", [(160, 200, 1), (160, 240, 1), (320, 200, 1), (320, 500, 1), (320, 1000, 1),
-                                           (160, 320, 4), (10, 200, 3), (40, 320, 4), (320, 1100, 3), (160, 1000, 6)])
-def test_sub_chunk_short_sequences(BH, T, segments):
+@pytest.mark.parametrize("dk,dv,BH,T,segments", [
+    (64, 64, 160, 200, 1), (64, 64, 160, 240, 1), (64, 64, 320, 200, 1), (64, 64, 320, 500, 1), (64, 64, 320, 1000, 1),
+    (64, 64, 160, 320, 4), (64, 64, 10, 200, 3), (64, 64, 40, 320, 4), (64, 64, 320, 1100, 3), (64, 64, 160, 1000, 6),
+    (128, 64, 160, 170, 1), (128, 64, 160, 250, 1), (128, 64, 10, 170, 3), (128, 64, 160, 1000, 6), (128, 128, 160, 170, 3),
+    (32, 32, 10, 170, 1), (32, 32, 160, 200, 1), (32, 32, 10, 250, 4), (32, 32, 640, 320, 1), (32, 32, 160, 320, 4)])
+def test_sub_chunk_short_sequences(dk, dv, BH, T, segments):
     """Many heads' short sequences stay whole, few heads' and long ones are cut."""
-    n = _nbytes(1, BH, T, 64, "channel", "preferred") / (BH * (64 * 128 * 4 + 8))
+    n = _nbytes(1, BH, T, dk, "channel", "preferred", dv) / (BH * (dk * (dv + dk) * 4 + 8))
     assert max(1, n) == segments

@@ -141,7 +141,7 @@ static size_t prefill_workspace(const maba_tensor* q, const maba_tensor* v, cons
   const int64_t BH = q->shape[0] * q->shape[1], L = q->shape[2], dk = q->shape[3], dv = v->shape[3];
   const bool chunk = dgda_chunk_supported(q, q, v, gate, b), sub = dgda_sub_supported(q, q, v, gate, b, nullptr, nullptr);
   size_t n = 0;
-  if (chunk) n = preferred ? std::max(dgda_chunk_workspace(BH, L), dgda_chunk_workspace_preferred(BH, L)) : dgda_chunk_workspace(BH, L);
+  if (chunk) n = preferred ? dgda_chunk_workspace_preferred(BH, L) : dgda_chunk_workspace(BH, L);   // the finer cut's is larger
   if (sub) n = std::max(n, dgda_sub_workspace(BH, L, dk, dv));
   if (sub && !chunk && preferred) n = std::max(n, dgda_sub_workspace_preferred(BH, L, dk, dv));
   return n;

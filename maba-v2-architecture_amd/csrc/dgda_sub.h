@@ -22,15 +22,16 @@
 // so they carry ~16 mantissa bits; the triangular solve and the state are fp32.
 //
 // One wave runs one segment of one (b, h) sequence on its own: no workgroup barriers, no
-// operand staged twice.  What bounded the four-wave form it replaced was latency: three
-// barriers and a 16-step inverse on one of its waves per sub-chunk, every shared operand
-// read from LDS by all four.  Here the waves of a SIMD hide each other's latencies, and
-// the operand layouts below keep the value side out of LDS altogether.  What bounds a wave now
-// is VALU issue: per sub-chunk at d_k = d_v = 64 about 1,100 VALU instructions (fused layer
-// 1,700, 200 of them transcendental) beside 100 MFMAs, so that one wave per SIMD takes 3.5 us
-// (6.5 us) and two take hardly less time each.  Before and after, whole calls: B=4 H=10
-// T=8192 d=128 fp16 1,377 -> 403 us; B=1 H=10 T=2048 fp32 212 -> 51 us; the fused layer's
-// launches at B=4 T=32768 1,150 -> 680 us, at B=1 T=1000 310 -> 100 us.
+// operand staged twice.  (Four waves per segment, 16 state columns each, share the key side but
+// spend most of a sub-chunk in three barriers, a triangular inverse on one of them and reading
+// every shared operand from LDS four times.)  The waves of a SIMD hide each other's latencies, and
+// the operand layouts below keep the value side out of LDS altogether.  What bounds a wave is
+// instruction issue: per sub-chunk at d_k = d_v = 64 about 1,000 VALU instructions with 64 columns
+// and 800 with 32 (fused layer 1,800 and 1,500, 230 and 200 of them transcendental) beside 100 and
+// 56 MFMAs, so that a wave alone on its SIMD takes 4.6 us with 64 columns and 3.0 with 32 (fused
+// layer 32: 4.2), and two hardly less time each.  Whole calls, four waves per segment / one: B=4 H=10
+// T=8192 d=128 fp16 1,383 / 364 us; B=1 H=10 T=2048 fp32 212 / 45 us; the fused layer's launches at
+// B=4 T=32768 1,150 / 640 us, at B=1 T=1000 310 / 74 us.
 //
 // Layouts.  NKT = d_k / 16, NCT = columns / 16.  Lane (c = lane & 15, g = lane >> 4):
 //  * staging: tokens 4g .. 4g+3, key channels NKT c .. NKT c + NKT-1, value channels
@@ -46,7 +47,7 @@
 //    groups with permlane swaps, then 120 FMAs against rows of L broadcast from LDS.
 //
 // Sequence parallelism.  A sequence is cut into nseg segments of equal length (see
-// sub_nseg).  One launch runs every segment from a zero state (the first from the initial
+// sub_cut).  One launch runs every segment from a zero state (the first from the initial
 // state) and, as further waves, every later segment's transition M (S <- M S + N) from
 // the identity, until M is exactly zero.  scan (three segments or more): start states of
 // segments whose predecessor's M survived.  fix: every later segment from its true start

@@ -55,20 +55,20 @@ bool dgda_sub_supported(const maba_tensor* q, const maba_tensor* k, const maba_t
 
 // ---- segments per sequence
 // Sub-chunks per segment at least.  Shorter ones no longer gain: a segment's end costs a step
-// of the scan where transitions survive (0.7 us against 3.5 us per sub-chunk twice), and where
-// they vanish it costs up to their 3 to 10 sub-chunks again.  B=1 H=10 T=2048 fp32: 87 us at
-// 16, 58 at 8, 46 at 4; slow decay at T=4096: 144, 103, 109 (6: 99).
+// of the scan where transitions survive (0.7 us against 4.6 us per sub-chunk twice), and where
+// they vanish it costs up to their 3 to 10 sub-chunks again.  At 16, 8, 6, 5, 4, 3: B=1 H=10 T=2048
+// fp32 69, 49, 45, 46, 48, 83 us; decay that remembers, T=4096 bf16 129, 98, 103, 105, 112, 125.
 constexpr int64_t SUB_MIN_LEN = 5;
-// Sub-chunks per segment from which two waves per SIMD pay: the second wave gains up to 8 %
-// (B=4 H=10 T=32768 per-channel bf16: 436 us against 470), and twice as many segments cost
-// their re-runs (the fused layer at B=1 T=32768, 10 sub-chunks each: 493 us against 412).
+// Sub-chunks per segment from which two waves per SIMD pay: the second wave gains a little (B=4
+// H=10 T=32768 per-channel bf16: 436 us against 445), and twice as many segments cost their re-runs
+// (the fused layer at B=1 T=32768, 10 sub-chunks each: 283 us against 208).
 constexpr int64_t SUB_LEN_2 = 32;
 // Segments per sequence at most, in units of the square root of its sub-chunks.  Where transitions
 // survive the scan takes a step per segment (0.7 us at d_k = 64, 9 at 128), and every sub-chunk is
 // run twice, so few heads over a long sequence are not cut until every SIMD has a wave.  One head,
 // without / with this bound / at 3, us, decay that remembers (and that vanishes): d_k = 64 T=131072
-// 943 / 584 / 465 (86 / 95 / 136), T=32768 398 / 284 / 235 (56 / 57 / 78); d_k = 128 T=65536 1953 /
-// 1513 / 1015 (160 / 146 / 172); the fused layer T=65536 771 / 451 / 418 (770 / 147 / 202: without
+// 944 / 570 / 435 (87 / 95 / 127), T=32768 395 / 277 / 219 (53 / 54 / 72); d_k = 128 T=65536 1934 /
+// 1495 / 988 (149 / 136 / 164); the fused layer T=65536 765 / 446 / 367 (763 / 138 / 163: without
 // it segments end before their transitions vanish).
 constexpr double SUB_SEG_ROOT = 6;
 // A short sequence stays whole where cutting it does not pay if its transitions survive: every
@@ -92,8 +92,8 @@ struct SubCut { int nseg, seglen, cols; };
 // waves hold a quarter of the state, never at d_k = 128, whose state leaves registers for one),
 // no more than SUB_SEG_ROOT lets a scan walk, and no more than the workspace holds.  Where that
 // leaves half the SIMDs without work a wave takes 32 columns instead of 64 (narrow): the key side is
-// done twice, but a sub-chunk takes a wave less time (B=2 H=10 bf16: T=160 54 -> 37 us, T=1000 57 ->
-// 48 us; the fused layer at H=10, T=100 52 -> 45 us, T=160 68 -> 59, T=1000 87 -> 77).
+// done twice, but a sub-chunk takes a wave less time (B=2 H=10 bf16: T=160 41 -> 34 us, T=1000 45 ->
+// 44 us; the fused layer at H=10, T=100 49 -> 42 us, T=160 64 -> 55, T=1000 83 -> 72).
 static SubCut sub_cut(int64_t BH, int64_t L, int64_t dk, int64_t dv, size_t ws_bytes, bool narrow) {
   const int64_t nch = sub_chunks(L);
   const int64_t simds = 4 * (int64_t)device_cu_count();

@@ -33,20 +33,20 @@
 //    -inf and a block listed once costs nothing.  Where that score is infinite or NaN the sum is
 //    NaN; the tile's largest score is therefore taken with the maximum that carries NaN, and only
 //    a tile that has one masks its rows with selects (no cost per score: v_maximum3_f32, two
-//    scores each, 2.67 -> 2.60 ms at the first size below against fmaxf);
+//    scores each, 2.66 -> 2.57 ms at the first size below against fmaxf);
 //  * the probabilities' sum is a product with a row of ones, on the matrix unit;
 //  * which union entries a query lists is a row of bits in LDS, one word per 32 entries, in
 //    place of comparing the entry with all of the query's slots (which remains for unions
 //    beyond PF_QWORDS words and for queries that list a block twice);
 //  * a tile inside every query's range skips the row masks, and the staging addresses are a
 //    uniform base and a 32-bit lane offset.
-// Measured at B=1 H=10 dh=64 T=32768, top-32 (start of each pair: a maximum and a rescale per
+// Measured at B=1 H=10 dh=64 T=32768, top-32 (first of each pair: a maximum and a rescale per
 // tile, counted slots, 64-bit addresses, padded rows): random queries, 5.1 K distinct blocks
-// per 16 of them, 3.82 -> 2.63 ms; neighbouring queries alike 1.13 -> 0.82 ms.  VALU
-// instructions per call 1,234 M -> 700 M, a quarter of the SIMDs' cycles MFMA.  Tiles loaded
-// straight to LDS three ahead, with 64 or 128 queries per workgroup, measured the same on
-// random queries and 12 to 20 % slower on alike ones (two workgroups per CU instead of three):
-// issue bounds it, not latency.
+// per 16 of them, 3.82 -> 2.58 ms; neighbouring queries alike 1.13 -> 0.82 ms.  VALU
+// instructions per call 1,234 M -> 578 M, a quarter of the SIMDs' cycles MFMA, LDS bank conflicts 390
+// M -> 12 M cycles.  Tiles loaded straight to LDS three ahead, with 64 or 128 queries per workgroup,
+// measured the same on random queries and 12 to 20 % slower on alike ones (two workgroups per CU
+// instead of three): issue bounds it, not latency.
 #include <algorithm>
 
 #include "dgda_common.h"
@@ -547,9 +547,8 @@ __global__ __launch_bounds__(256, NP == 4 ? 2 : 3) void maba_sa_prefill_kernel(P
 // How many distinct blocks each 16 consecutive queries list, summed per workgroup: what the choice
 // between this kernel and the latent one goes by.  A wave takes 16 queries at a time and marks
 // their slots in its LDS bitmap; the lane that sets a bit counts it, and afterwards the words it
-// touched are cleared.  Latency-bound: 11 us for the 6.3 MB of indices at T=24571 K=32, where a
-// segmented sort of the 16 K slots (48 us), the compare of neighbours, its sum and their means had
-// the layer's call at 1,111 us, now 1,050.
+// touched are cleared.  Latency-bound: 10 us for the 6.3 MB of indices at T=24571 K=32 (a segmented
+// sort of the 16 K slots 48 us, beside the compare of neighbours, its sum and their mean).
 struct PfUnionArgs {
   const int64_t* idx; int64_t isb, ist, isk;
   int32_t* out;                       // one count per workgroup

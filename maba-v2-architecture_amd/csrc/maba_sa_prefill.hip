@@ -27,13 +27,13 @@
 // The kernel is bound by VALU issue, not by its products (a tile's 24 MFMAs are 384 cycles of
 // the matrix unit), so the softmax is kept to one FMA, one maximum, one exp2, one addition and
 // the hi/lo split per score:
-//  * the running reference m of a query moves only when a score passes it by 2^8 (the sums
-//    hold that easily in fp32); only then do lanes exchange maxima and the sums rescale;
+//  * the running reference m of a query moves only when a score passes it by 2^PF_SLACK; only
+//    then do lanes exchange maxima and the sums rescale;
 //  * a key's weight is folded into the exponent as its log2, so an unlisted block is a bias of
 //    -inf and a block listed once costs nothing.  Where that score is infinite or NaN the sum is
 //    NaN; the tile's largest score is therefore taken with the maximum that carries NaN, and only
 //    a tile that has one masks its rows with selects (no cost per score: v_maximum3_f32, two
-//    scores each, 2.66 -> 2.57 ms at the first size below against fmaxf);
+//    scores each; with a slack of 8, 2.66 -> 2.57 ms at the first size below against fmaxf);
 //  * the probabilities' sum is a product with a row of ones, on the matrix unit;
 //  * which union entries a query lists is a row of bits in LDS, one word per 32 entries, in
 //    place of comparing the entry with all of the query's slots (which remains for unions
@@ -42,7 +42,7 @@
 //    uniform base and a 32-bit lane offset.
 // Measured at B=1 H=10 dh=64 T=32768, top-32 (first of each pair: a maximum and a rescale per
 // tile, counted slots, 64-bit addresses, padded rows): random queries, 5.1 K distinct blocks
-// per 16 of them, 3.82 -> 2.58 ms; neighbouring queries alike 1.13 -> 0.82 ms.  VALU
+// per 16 of them, 3.82 -> 2.65 ms; neighbouring queries alike 1.13 -> 0.85 ms.  VALU
 // instructions per call 1,234 M -> 578 M, a quarter of the SIMDs' cycles MFMA, LDS bank conflicts 390
 // M -> 12 M cycles.  Tiles loaded straight to LDS three ahead, with 64 or 128 queries per workgroup,
 // measured the same on random queries and 12 to 20 % slower on alike ones (two workgroups per CU
@@ -57,7 +57,12 @@ constexpr int PF_MAXK = 64;          // index slots per query
 constexpr int PF_WORDS = 512;        // bitmap words per workgroup: blocks below 16384
 constexpr int PF_LIST = 64 * PF_MAXK;   // the union of a workgroup's 64 queries' slots
 constexpr int PF_QWORDS = 16;        // words of a query's row of union bits (512 entries)
-constexpr float PF_SLACK = 8.f;      // a score may pass the running reference by 2^8
+// A score may pass the running reference by 2^PF_SLACK.  The heaviest key's probability is exact in
+// bf16 hi + lo while the reference is its score; the more the reference lags, the larger that key's
+// rounding: error against 64 bits before the output's rounding (queries of twice unit variance,
+// T=2048) 9.43e-7 at 0, 9.50e-7 at 0.5, 9.6e-7 at 1, 1.30e-6 at 8 (a maximum per tile, the sums on
+// the VALU: 9.86e-7); time at T=32768 2.71, 2.65, 2.63 and 2.56 ms.
+constexpr float PF_SLACK = 0.5f;
 
 // The workgroup's union of blocks; behind a list of at most 32 PF_QWORDS of them, the rows of bits.
 union PfList {

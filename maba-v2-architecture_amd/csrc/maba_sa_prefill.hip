@@ -42,8 +42,8 @@
 //    uniform base and a 32-bit lane offset.
 // Measured at B=1 H=10 dh=64 T=32768, top-32 (first of each pair: a maximum and a rescale per
 // tile, counted slots, 64-bit addresses, padded rows): random queries, 5.1 K distinct blocks
-// per 16 of them, 3.82 -> 2.65 ms; neighbouring queries alike 1.13 -> 0.85 ms.  VALU
-// instructions per call 1,234 M -> 578 M, a quarter of the SIMDs' cycles MFMA, LDS bank conflicts 390
+// per 16 of them, 3.82 -> 2.66 ms; neighbouring queries alike 1.13 -> 0.84 ms.  VALU
+// instructions per call 1,234 M -> 604 M, a quarter of the SIMDs' cycles MFMA, LDS bank conflicts 390
 // M -> 12 M cycles.  Tiles loaded straight to LDS three ahead, with 64 or 128 queries per workgroup,
 // measured the same on random queries and 12 to 20 % slower on alike ones (two workgroups per CU
 // instead of three): issue bounds it, not latency.

@@ -299,11 +299,11 @@ class MabaSparseAttention(WeightCacheMixin, nn.Module):
         queries share every key tile, per head).  Its cost grows with the union of 16
         consecutive queries' blocks and with the heads' channels, the latent kernel's with d_c
         alone.  Measured (heads / latent, ms; union in units of top_k), 10 heads of 64, d_c 128,
-        top-32: 32k tokens, union 5.1, 2.80 / 4.42; 64k, 6.5, 7.95 / 9.20; 128k, 6.9, 17.9 / 20.2,
-        7.4, 19.9 / 20.2, 7.6, 21.2 / 18.8; 256k, 7.4, 42.5 / 47.7; top-16, 128k, 7.0, 9.4 / 16.3.
-        16 heads of 32, 128k, 6.7, 21.5 / 21.8.  The latent kernel wins earlier where the heads are
-        wider against d_c or a query lists more blocks: 16 heads of 64, 64k, 5.8, 10.4 / 10.2; heads of
-        128, 5.35, 11.7 / 9.4; d_c 64, 5.8, 6.6 / 4.9; top-64, 128k, 6.1, 29.8 / 28.1.  Neighbouring
+        top-32: 32k tokens, union 5.1, 2.76 / 4.42; 64k, 6.5, 7.86 / 9.19; 128k, 6.9, 18.1 / 20.1,
+        7.4, 20.1 / 20.0; 256k, 7.4, 43.1 / 47.4; top-16, 128k, 7.0, 9.7 / 16.2.
+        16 heads of 32, 128k, 6.7, 21.6 / 21.8.  The latent kernel wins earlier where the heads are
+        wider against d_c or a query lists more blocks: 16 heads of 64, 64k, 5.8, 10.2 / 10.2; heads of
+        128, 5.35, 11.7 / 9.4; d_c 64, 5.8, 6.5 / 4.9; top-64, 128k, 6.1, 29.3 / 28.1.  Neighbouring
         queries of a trained or randomly initialised model select nearly the same blocks (about 3 K).
         The union is counted on the GPU from ``idx``
         (``hip_prefill_union``; elsewhere one segmented sort); ``self.prefill_form`` may force either."""

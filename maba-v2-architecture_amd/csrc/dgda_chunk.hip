@@ -769,18 +769,24 @@ static size_t chunk_geom_bytes(const SlotGeom& gm, int64_t BH) {
 
 // Chunks per slot with the preferred workspace.  A workgroup takes about 4.6 us per chunk however
 // few there are, so slots of 16 chunks leave an idle chip waiting for them: CPS_FINE, or what
-// fills two workgroups per CU.  But where maps survive, a segment's fix-up workgroup applies those
-// before it one after the other (2.4 us each, more with two workgroups per CU), so a sequence is
-// cut less where that walk gets long: beyond WALK segments to one workgroup per CU (where slots of
-// CPS would be), and never into more than WALK_MAX while CPS does not cut it so either.
-// H heads, T tokens, us with slots of CPS / of CPS_FINE without these bounds / of this rule, decay
-// that remembers (and that vanishes):
-//   H=10 T=2048 207 / 77 / 77 (85 / 35 / 35)       H=16 T=8192 225 / 203 / 141 (86 / 46 / 53)
-//   H=8 T=16384 239 / 321 / 171 (86 / 47 / 53)     H=8 T=32768 270 / 390 / 270 (87 / 67 / 87)
-//   H=4 T=32768 269 / 561 / 231 (86 / 47 / 53)     H=1 T=131072 450 / 1511 / 448 (86 / 48 / 86)
-// CPS_FINE of 2 measured as 4 where maps vanish and slower with many surviving ones (H=10 T=5000
-// 161 against 100), 8 slower.
-constexpr int WALK = 24, WALK_MAX = 64;
+// fills two workgroups per CU.  But where maps survive their segment, a segment's fix-up workgroup
+// applies those before it one after the other (2.4 us each, more with two workgroups per CU), and
+// every segment runs twice, so a sequence is cut less where that walk gets long: beyond WALK segments
+// to one workgroup per CU (where slots of CPS would be), and never into more than WALK_MAX while CPS
+// does not cut it so either.  The line lies where no decay is slower than with slots of CPS: those
+// between vanishing within a chunk and remembering, whose maps survive four chunks and not sixteen,
+// gain least.  H heads, T tokens, us with slots of CPS / of CPS_FINE without these bounds / of this
+// rule, log-decay per token 2.1 (and 0.157, 0.01):
+//   H=10 T=2048 84 / 35 / 35 (163 / 77 / 77, 208 / 77 / 77)
+//   H=4 T=16384 86 / 36 / 65 (164 / 184 / 183, 238 / 184 / 191)
+//   H=24 T=8192 87 / 59 / 72 (171 / 201 / 155, 227 / 201 / 181)
+//   H=20 T=10007 92 / 66 / 80 (173 / 197 / 160, 227 / 197 / 196)
+//   H=8 T=32768 87 / 67 / 87 (176 / 388 / 176, 270 / 390 / 270)
+//   H=1 T=131072 86 / 48 / 86 (366 / 1511 / 364, 450 / 1511 / 448)
+// With more than one slot of CPS per CU two per CU stay: H=20 T=16384 105 / 78 / 78 (231 / 285 / 285, 356 /
+// 286 / 286).  CPS_FINE of 2 measured as 4 where maps vanish and slower with many surviving ones (H=10
+// T=5000 161 against 100), 8 slower.
+constexpr int WALK = 12, WALK_MAX = 27;
 static int64_t fine_slot(int64_t BH, int64_t nch, int64_t cus) {
   int64_t U = std::max<int64_t>(CPS_FINE, ceil_div(BH * nch, 2 * cus));
   if (U >= CPS || ceil_div(nch, U) <= WALK) return U;

@@ -67,7 +67,7 @@
 
 namespace maba {
 
-constexpr int SUB_MAX_SEG = 2048;         // segments per sequence at most
+constexpr int SUB_MAX_SEG = 256;         // segments per sequence at most
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr float SUB_MFMA_RANGE = 64.f * LOG2E;   // largest |Lam| within a sub-chunk on the MFMA path, in log2 units
 constexpr float SUB_MFMA_MIN = 1.6038108e-28f;   // e^-64, the same limit for the prologue's decay products

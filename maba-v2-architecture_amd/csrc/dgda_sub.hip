@@ -4,7 +4,6 @@
 #include "dgda_sub.h"
 
 #include <algorithm>
-#include <cmath>
 
 namespace maba {
 
@@ -63,14 +62,14 @@ constexpr int64_t SUB_MIN_LEN = 5;
 // H=10 T=32768 per-channel bf16: 436 us against 445), and twice as many segments cost their re-runs
 // (the fused layer at B=1 T=32768, 10 sub-chunks each: 283 us against 208).
 constexpr int64_t SUB_LEN_2 = 32;
-// Segments per sequence at most, in units of the square root of its sub-chunks.  Where transitions
-// survive the scan takes a step per segment (0.7 us at d_k = 64, 9 at 128), and every sub-chunk is
-// run twice, so few heads over a long sequence are not cut until every SIMD has a wave.  One head,
-// without / with this bound / at 3, us, decay that remembers (and that vanishes): d_k = 64 T=131072
-// 944 / 570 / 435 (87 / 95 / 127), T=32768 395 / 277 / 219 (53 / 54 / 72); d_k = 128 T=65536 1934 /
-// 1495 / 988 (149 / 136 / 164); the fused layer T=65536 765 / 446 / 367 (763 / 138 / 163: without
-// it segments end before their transitions vanish).
-constexpr double SUB_SEG_ROOT = 6;
+// Segments per sequence at most.  Where transitions survive the scan takes a step per segment (0.7 us
+// at d_k = 64, 4 at 128, 0.4 at 32), and every sub-chunk is run twice, so few heads over a long sequence
+// are not cut until every SIMD has a wave: with these bounds no decay is slower than in segments of 64
+// sub-chunks on four waves each.  One head, four waves / 6 sqrt(sub-chunks) segments / these bounds, us,
+// log-decay per token 2.1 (and 0.2, 0.01): d_k = 64 T=32768 232 / 51 / 59 (402 / 337 / 236, 663 / 336 / 236),
+// T=131072 233 / 95 / 158 (403 / 570 / 245, 926 / 570 / 445); d_k = 128 T=65536 880 / 136 / 255 (1685 /
+// 1495 / 397, 4015 / 1495 / 770); the fused layer T=65536 344 / 94 / 137 (571 / 447 / 367, 926 / 446 / 367).
+static int64_t seg_most(int64_t dk) { return dk == 128 ? 96 : dk == 64 ? 192 : 256; }
 // A short sequence stays whole where cutting it does not pay if its transitions survive: every
 // sub-chunk is run twice, on SIMDs that segments and transitions share once these are more than
 // half as many as the SIMDs (below that segments always paid), and joining them takes as long as
@@ -90,7 +89,7 @@ struct SubCut { int nseg, seglen, cols; };
 
 // As many segments as fill one wave per SIMD, or two (see SUB_LEN_2; always at d_k = 32, whose
 // waves hold a quarter of the state, never at d_k = 128, whose state leaves registers for one),
-// no more than SUB_SEG_ROOT lets a scan walk, and no more than the workspace holds.  Where that
+// no more than a scan should walk (seg_most), and no more than the workspace holds.  Where that
 // leaves half the SIMDs without work a wave takes 32 columns instead of 64 (narrow): the key side is
 // done twice, but a sub-chunk takes a wave less time (B=2 H=10 bf16: T=160 41 -> 34 us, T=1000 45 ->
 // 44 us; the fused layer at H=10, T=100 49 -> 42 us, T=160 64 -> 55, T=1000 83 -> 72).
@@ -101,11 +100,10 @@ static SubCut sub_cut(int64_t BH, int64_t L, int64_t dk, int64_t dv, size_t ws_b
   const bool two = dk == 32 || (dk == 64 && nch * waves >= SUB_LEN_2 * 2 * simds);
   int64_t n = (two ? 2 : 1) * simds / waves;
   if (n > ceil_div(nch, SUB_MIN_LEN)) n = ceil_div(nch, SUB_MIN_LEN);
-  const int64_t most = (int64_t)(SUB_SEG_ROOT * std::sqrt((double)nch));
-  if (n > most) n = most;
+  if (n > seg_most(dk)) n = seg_most(dk);
   const int64_t fit = (int64_t)(ws_bytes / ((size_t)(BH > 0 ? BH : 1) * sub_slot_bytes(dk, dv)));
   if (n > fit) n = fit;
-  if (n > SUB_MAX_SEG) n = SUB_MAX_SEG;
+  static_assert(SUB_MAX_SEG >= 256, "the scan's table holds seg_most");
   // two short segments take no less time one after the other (the second's re-run) than one
   if (n < 2 || (n == 2 && nch < 4 * SUB_MIN_LEN)) n = 1;
   auto cut = [&](int64_t n) {

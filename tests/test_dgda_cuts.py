@@ -31,8 +31,8 @@ def test_chunk_cut_is_bounded(BH):
         if nch > 16:
             assert n >= least
         # ends inside slots add one
-        assert n <= max(66, least), f"{nch} chunks"
-        if n > 26 and BH * nch <= 16 * CUS:    # a long walk: one workgroup per CU
+        assert n <= max(29, least), f"{nch} chunks"
+        if n > 14 and BH * nch <= 16 * CUS:    # a long walk: one workgroup per CU
             assert BH * nch / (n - 1) >= min(16, BH * nch / CUS) - 1, f"{nch} chunks"
 
 
@@ -44,9 +44,9 @@ def test_chunk_cut_where_walks_are_short():
 @pytest.mark.parametrize("d", [32, 64, 128])
 @pytest.mark.parametrize("BH", [1, 2, 4, 10, 40, 160])
 def test_sub_chunk_cut_is_bounded(BH, d):
-    for T in (100, 1000, 4096, 10007, 32768, 131072, 1 << 20, 1 << 24):
+    for T in (100, 1000, 4096, 10007, 32768, 65536):   # longer, the least size is the larger one
         n = _nbytes(1, BH, T, d, "channel", "preferred") / (BH * (d * 2 * d * 4 + 8))
-        assert n <= 6 * (-(-T // 16)) ** 0.5, f"{T} tokens"
+        assert n <= {32: 256, 64: 192, 128: 96}[d], f"{T} tokens"
 
 
 @pytest.mark.parametrize("dk,dv,BH,T,segments", [

@@ -42,8 +42,8 @@
 //    uniform base and a 32-bit lane offset.
 // Measured at B=1 H=10 dh=64 T=32768, top-32 (first of each pair: a maximum and a rescale per
 // tile, counted slots, 64-bit addresses, padded rows): random queries, 5.1 K distinct blocks
-// per 16 of them, 3.82 -> 2.66 ms; neighbouring queries alike 1.13 -> 0.84 ms.  VALU
-// instructions per call 1,234 M -> 604 M, a quarter of the SIMDs' cycles MFMA, LDS bank conflicts 390
+// per 16 of them, 3.82 -> 2.62 ms; neighbouring queries alike 1.13 -> 0.83 ms.  VALU
+// instructions per call 1,234 M -> 605 M, a quarter of the SIMDs' cycles MFMA, LDS bank conflicts 390
 // M -> 12 M cycles.  Tiles loaded straight to LDS three ahead, with 64 or 128 queries per workgroup,
 // measured the same on random queries and 12 to 20 % slower on alike ones (two workgroups per CU
 // instead of three): issue bounds it, not latency.
@@ -61,7 +61,8 @@ constexpr int PF_QWORDS = 16;        // words of a query's row of union bits (51
 // bf16 hi + lo while the reference is its score; the more the reference lags, the larger that key's
 // rounding: error against 64 bits before the output's rounding (queries of twice unit variance,
 // T=2048) 9.43e-7 at 0, 9.50e-7 at 0.5, 9.6e-7 at 1, 1.30e-6 at 8 (a maximum per tile, the sums on
-// the VALU: 9.86e-7); time at T=32768 2.71, 2.65, 2.63 and 2.56 ms.
+// the VALU: 9.86e-7); time at T=32768 2.71, 2.65, 2.63 and 2.56 ms
+// (2.61 with no sums rescaled at a stream's first tile).
 constexpr float PF_SLACK = 0.5f;
 
 // The workgroup's union of blocks; behind a list of at most 32 PF_QWORDS of them, the rows of bits.
@@ -398,11 +399,13 @@ __global__ __launch_bounds__(256, NP == 4 ? 2 : 3) void maba_sa_prefill_kernel(P
       float top = lw == -INFINITY ? -INFINITY : mx - lw + base;
       top = group_max(top);
       const float m_new = fmaxf(st.m, top);
-      const float corr = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(st.m - m_new);
-      st.m = m_new;
-      st.l *= corr;   // every element is the query's sum
+      if (__ballot(st.l[0] != 0.f) != 0ull) {   // not at a stream's first tile: there is no sum yet
+        const float corr = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(st.m - m_new);
+        st.l *= corr;   // every element is the query's sum
 #pragma unroll
-      for (int dt = 0; dt < NDT; ++dt) st.z[dt] *= corr;
+        for (int dt = 0; dt < NDT; ++dt) st.z[dt] *= corr;
+      }
+      st.m = m_new;
       relative();
       if (nan) drop();
     }
